@@ -193,7 +193,7 @@ _NP_DTYPE = {F32: np.float32, F16: np.float16, BF16: np.uint16, U32: np.uint32, 
 class DeviceBuffer:
     """A hipMalloc'ed buffer with a shape and an rmlx dtype tag (bf16 travels as uint16 bits)."""
 
-    _view = None  # see address()
+    _view = None  # see view()
 
     def __init__(self, shape, dtype):
         self.shape = tuple(int(s) for s in shape)
@@ -219,13 +219,16 @@ class DeviceBuffer:
         check(lib().rmlx_hip_memcpy_d2h(out.ctypes.data, self.ptr, self.nbytes, None))
         return out
 
-    def address(self):
-        """Address of this buffer's rmlx_array view (what `array()` builds), kept while pointer, shape and type stay the same."""
+    def view(self):
+        """This buffer's rmlx_array (what `array()` builds) with its `address`, kept while pointer, shape and type stay the same.  A
+        call holds the object until it returns: another thread may build and keep a new one meanwhile."""
         key = (self.ptr, self.shape, self.dtype)
-        if self._view is None or self._view[0] != key:
+        kept = self._view
+        if kept is None or kept[0] != key:
             a = self.array()
-            self._view = (key, a, ctypes.addressof(a))
-        return self._view[2]
+            a.address = ctypes.addressof(a)
+            kept = self._view = (key, a)
+        return kept[1]
 
     def array(self, shape=None, offset_elems=0):
         """The rmlx_array view handed to the C ABI."""
