@@ -362,7 +362,8 @@ __global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (M
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   static_assert(KP == 1 || R == 1, "split rows: one row per wave group");
-  // (the last block of an N that is no multiple of the block starts earlier and computes some rows once more, to the same bits)
+  // (the last block of an N that is no multiple of the block starts earlier and computes some rows once more; it stores only its
+  // own, from blk0 on, because the output may be the epilogue's operand)
   const uint32_t blk0 = blockIdx.x * (kWaves * R / KP), last0 = p.N - kWaves * R / KP;
   const uint32_t row0 = (blk0 < last0 ? blk0 : last0) + (wave / KP) * R;
   const uint32_t kp = wave % KP;
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (M
   load_activations<BITS, MR, NORM>(img, p.x, p.M, mrow0, p.norm_w, p.inv_rms, tid, xv);
   // ... the epilogue operand of the output this lane will write (lane r * MR + m) ...
   const uint32_t out_m = mrow0 + lane % MR, out_n = row0 + lane / MR;
-  const bool writes = lane < R * MR && out_m < p.M;
+  const bool writes = lane < R * MR && out_m < p.M && out_n >= blk0;
   float epi_val = 0.f;
   if (p.epi_kind != EPI_NONE && writes) {
     const uint64_t oi = (uint64_t)out_m * p.N + out_n;
@@ -514,8 +515,9 @@ __global__ __launch_bounds__(kThreads, 1) void qmv_m1_loop_kernel(M1Params p) {
   // next block's weights are already in flight while the current block is multiplied.
   const uint32_t nblk = (p.N + kWaves * R - 1) / (kWaves * R);
   const uint32_t my_blocks = blockIdx.x < nblk ? (nblk - 1 - blockIdx.x) / gridDim.x + 1 : 0u;
+  auto block_start = [&](uint32_t i) { return (blockIdx.x + i * gridDim.x) * (kWaves * R); };
   auto block_row0 = [&](uint32_t i) {  // (the last block of an N that is no multiple of the block: as above)
-    const uint32_t blk0 = (blockIdx.x + i * gridDim.x) * (kWaves * R), last0 = p.N - kWaves * R;
+    const uint32_t blk0 = block_start(i), last0 = p.N - kWaves * R;
     return (blk0 < last0 ? blk0 : last0) + wave * R;
   };
 
@@ -604,11 +606,12 @@ __global__ __launch_bounds__(kThreads, 1) void qmv_m1_loop_kernel(M1Params p) {
           const float t2 = wave_sum(racc[r][m]);
           mine = lane == r * MR + m ? t2 : mine;
         }
-      if (writes) {  // residual add / SwiGLU gate in f32, one rounding (quantized.rs:3206-3246)
+      const uint32_t out_n = block_row0(pr_blk) + lane / MR;
+      if (writes && out_n >= block_start(pr_blk)) {  // residual add / SwiGLU gate in f32, one rounding (quantized.rs:3206-3246)
         if (p.epi_kind == EPI_RESIDUAL) mine += epi_val;
         else if (p.epi_kind == EPI_SWIGLU) mine = epi_val / (1.0f + __expf(-epi_val)) * mine;
         if (GATHER && gather_zeros) mine = 0.f;
-        p.out[(uint64_t)out_m * p.N + block_row0(pr_blk) + lane / MR] = __float2half(mine);
+        p.out[(uint64_t)out_m * p.N + out_n] = __float2half(mine);
       }
       pr_c0 = 0;
       ++pr_blk;

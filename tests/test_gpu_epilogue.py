@@ -1,0 +1,42 @@
+"""Fused epilogues (residual add, SwiGLU gate) on the GPU: outputs written over the operand."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tests.helpers import make_weight, make_x
+
+pytestmark = pytest.mark.gpu
+
+
+def _calls(rt):
+    return {"residual": rt.lib().rmlx_hip_qmm_add_residual, "swiglu": rt.lib().rmlx_hip_qmm_swiglu}
+
+
+def _in_place_equals_apart(rt, m, n, k, bits, gs=64, repeats=3):
+    """out == operand gives the bits of an output of its own."""
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(m + n + k + bits + gs)
+    qw = ops.QuantizedWeight.from_numpy(*make_weight(rng, n, k, bits, gs), gs, bits)
+    x = DeviceBuffer.from_numpy(make_x(rng, m, k))
+    e = rng.standard_normal((m, n)).astype(np.float16)
+    xa = x.array()
+    for name, fn in _calls(rt).items():
+        ed, apart = DeviceBuffer.from_numpy(e), DeviceBuffer((m, n), rt.F16)
+        ea = ed.array()
+        rt.check(fn(qw.handle, ctypes.byref(xa), ctypes.byref(ea), apart.ptr, apart.nbytes, None))
+        want = apart.numpy()
+        for _ in range(repeats):
+            own = DeviceBuffer.from_numpy(e)
+            oa = own.array()
+            rt.check(fn(qw.handle, ctypes.byref(xa), ctypes.byref(oa), own.ptr, own.nbytes, None))
+            assert np.array_equal(own.numpy().view(np.uint16), want.view(np.uint16)), f"{name} M={m} N={n} K={k} bits={bits} gs={gs}"
+
+
+@pytest.mark.parametrize("m,n,k,bits", [(1, 12296, 4096, 4), (1, 33001, 4096, 4), (1, 33001, 1024, 8), (2, 12289, 512, 4), (1, 4104, 12288, 4),
+                                        (1, 1023, 12288, 4), (1, 515, 16384, 8), (1, 9, 512, 4), (1, 112257, 1408, 4)])
+def test_in_place_over_an_overlapping_last_block(hip, m, n, k, bits):
+    """Single-row kernel, a number of weight rows that is no multiple of a block (of one and two rows per wave, of rows split over
+    waves, of workgroups that walk several blocks): the rows that two blocks compute are stored by one of them."""
+    _in_place_equals_apart(hip, m, n, k, bits)
