@@ -179,7 +179,7 @@ int32_t rmlx_hip_qmm_select(const rmlx_qweight* qw, const rmlx_array* x, int32_t
  * `qmm_swiglu_into_cb` :8345-8452): out = x @ dequant(W)^T + residual, resp.
  * out = silu(gate_result) * (x @ dequant(W)^T).  residual / gate_result: [M, out_features],
  * Float16 or Float32 (the reference's are Float32), same validation message as the reference
- * ("... shape must be [M, N]"); out is f16.  Evaluated in f32 on the accumulator with one rounding
+ * ("... shape must be [M, N]"); out is f16 and may be an f16 operand itself (the same address; no other overlap).  Evaluated in f32 on the accumulator with one rounding
  * in the GEMM kernel; after the GEMV / portable kernels as a separate elementwise pass.  Unlike the
  * reference (Q4, M > 32 only) every shape the batched entry point takes is accepted. */
 int32_t rmlx_hip_qmm_add_residual(const rmlx_qweight* qw, const rmlx_array* x, const rmlx_array* residual,

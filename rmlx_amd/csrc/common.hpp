@@ -233,8 +233,8 @@ struct QmmArgs {
   bool workspace_has_partials = false;  // LDS-staged GEMM: the workspace was sized with N, so a launch of few tiles may split K
 };
 enum { EPI_NONE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2 };
-// out[i] = out[i] + e[i]  /  silu(e[i]) * out[i], in place on f16 out (kernels without a fused epilogue)
-int32_t launch_epilogue(__half* out, int kind, const void* e, int32_t e_dtype, size_t n, hipStream_t s);
+// out[i] = src[i] + e[i]  /  silu(e[i]) * src[i], f16 src (kernels without a fused epilogue; out may be src or the f16 operand e)
+int32_t launch_epilogue(__half* out, const __half* src, int kind, const void* e, int32_t e_dtype, size_t n, hipStream_t s);
 size_t qmm_workspace_bytes(uint32_t M, uint32_t K, uint32_t N = 0);
 // split-K partial sums of the register-weights GEMM (0 when the launch is not split); pass the buffer in QmmArgs::workspace
 size_t qmm_rw_workspace_bytes(uint32_t M, uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);

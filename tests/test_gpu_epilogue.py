@@ -40,3 +40,11 @@ def test_in_place_over_an_overlapping_last_block(hip, m, n, k, bits):
     """Single-row kernel, a number of weight rows that is no multiple of a block (of one and two rows per wave, of rows split over
     waves, of workgroups that walk several blocks): the rows that two blocks compute are stored by one of them."""
     _in_place_equals_apart(hip, m, n, k, bits)
+
+
+@pytest.mark.parametrize("m,n,k,bits,gs", [(5, 4096, 4096, 4, 64), (12, 512, 1024, 8, 64), (3, 24576, 1024, 4, 32), (3, 5, 64, 4, 64), (3, 8, 32, 4, 32),
+                                           (130, 192, 320, 4, 64), (130, 512, 1024, 4, 64), (600, 4096, 4096, 4, 64),
+                                           (130, 4096, 8192, 4, 64), (600, 2051, 1088, 4, 64), (33, 130, 4160, 8, 64)])
+def test_in_place_on_every_kernel(hip, m, n, k, bits, gs):
+    """Streaming GEMVs, portable and LDS-staged kernels (the epilogue in a pass of its own) and the GEMMs that fuse it."""
+    _in_place_equals_apart(hip, m, n, k, bits, gs, repeats=1)
