@@ -322,24 +322,21 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
   if (!DUAL && (p.partial != nullptr || p.out_f32)) {
     if (kg != 0) return;
     float* o = p.partial != nullptr ? p.partial + (uint64_t)t_.split * p.M * p.N : static_cast<float*>(p.out);
-    const uint64_t o0 = (uint64_t)row_lo * p.N + n0;
-    const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(o + o0, 0, 0x7FFFFFFF, 0x00020000);
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
       const uint32_t m = i * 32 + r;
+      if (m >= rows) continue;
+      float* const om = o + (uint64_t)(row_lo + m) * p.N + n0;
 #pragma unroll
       for (int eg = 0; eg < 4; ++eg) {
         const uint32_t c = wv * 32 + 8 * eg + 4 * hh;
-        u4 v;
+        f4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = t_.zeros ? 0u : __float_as_uint(acc[i][eg * 4 + e]);
-        const uint32_t at0 = m < rows ? (m * p.N + c) * 4 : kOutside;
-        if (cols == BNO) {
-          __builtin_amdgcn_raw_buffer_store_b128(v, orsrc, at0, 0, 0);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) __builtin_amdgcn_raw_buffer_store_b32(v[e], orsrc, c + e < cols ? at0 + 4 * e : kOutside, 0, 0);
-        }
+        for (int e = 0; e < 4; ++e) v[e] = t_.zeros ? 0.f : acc[i][eg * 4 + e];
+        if (c + 4 <= cols) reinterpret_cast<f4_any*>(om + c)->v = v;
+        else
+          for (uint32_t e = 0; e < 4; ++e)
+            if (c + e < cols) om[c + e] = v[e];
       }
     }
     return;

@@ -48,3 +48,21 @@ def test_in_place_over_an_overlapping_last_block(hip, m, n, k, bits):
 def test_in_place_on_every_kernel(hip, m, n, k, bits, gs):
     """Streaming GEMVs, portable and LDS-staged kernels (the epilogue in a pass of its own) and the GEMMs that fuse it."""
     _in_place_equals_apart(hip, m, n, k, bits, gs, repeats=1)
+
+
+def test_residual_over_more_than_two_gib_of_sums(hip):
+    """256 rows x 2.2 million columns: offsets within a tile's rows pass 2 GiB where the sums are f32."""
+    from oracle import model
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    from tests.helpers import assert_close
+    m, n, k = 256, 2_200_032, 64
+    rng = np.random.default_rng(5)
+    words, s, b = make_weight(rng, n, k)
+    qw = ops.QuantizedWeight.from_numpy(words, s, b, 64, 4)
+    x = make_x(rng, m, k)
+    cols = np.unique(np.concatenate([np.arange(0, 300), rng.integers(0, n, 300), np.arange(n - 300, n)]))
+    e = np.zeros((m, n), np.float16)
+    e[:, cols] = rng.standard_normal((m, len(cols))).astype(np.float16)
+    out = ops.qmm_add_residual(DeviceBuffer.from_numpy(x), qw, DeviceBuffer.from_numpy(e)).numpy()[:, cols]
+    assert_close(out, model.qmm(x.astype(np.float64), words[cols], s[cols], b[cols], 64, 4) + e[:, cols].astype(np.float64), "residual")
