@@ -288,7 +288,7 @@ int32_t launch_qmm_rw_grouped(const GroupedQmmArgs& a, hipStream_t s);
 struct TilePlan { uint32_t wn, mi, kw, splits; };
 bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, double* us);  // us: estimated time of the launch
-size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N, int epi_kind);
+size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N);
 int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s);
 // The same over a table of row tiles of 256 rows of one expert (x_rows: rows of x; out f16 or f32, a pair f16)
 bool qmm_tile_grouped_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits, uint32_t x_rows);

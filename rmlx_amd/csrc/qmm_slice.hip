@@ -261,6 +261,7 @@ __device__ __forceinline__ void slice_body(const TileParams p, const Tile t_, ch
           for (uint32_t e = 0; e < 4; ++e)
             if (c + e < cols) q[e] = v[e];
       } else {
+        if (!DUAL && p.epi_kind != EPI_NONE && m < rows && c < cols) tile_epilogue(p, (uint64_t)(row_lo + m) * p.N + n0 + c, cols - c, v);
         const h2 lo = {(_Float16)v[0], (_Float16)v[1]}, hi = {(_Float16)v[2], (_Float16)v[3]};
         *reinterpret_cast<u2*>(outs + (m * U + ((c >> 3) ^ (m & kKey))) * 16 + (c & 4) * 2) = (u2){h2bits(lo), h2bits(hi)};
       }

@@ -373,6 +373,7 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
         f4 v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = t_.zeros ? 0.f : acc[i][eg * 4 + e];
+        if (!DUAL && p.epi_kind != EPI_NONE && m < rows && c < cols) tile_epilogue(p, (uint64_t)(row_lo + m) * p.N + n0 + c, cols - c, v);
         const h2 lo = {(_Float16)v[0], (_Float16)v[1]}, hi = {(_Float16)v[2], (_Float16)v[3]};
         *reinterpret_cast<u2*>(lds + (m * U + ((c >> 3) ^ (m & kKey))) * 16 + hh * 8) = (u2){h2bits(lo), h2bits(hi)};
       }
@@ -430,18 +431,10 @@ __global__ __launch_bounds__(256) void tile_splits_sum_kernel(TileParams p) {
     else
       for (uint32_t e = 0; e < n; ++e) v[e] += q[e];
   }
+  if (p.epi_kind != EPI_NONE) tile_epilogue(p, i, n, v);
   _Float16* out = static_cast<_Float16*>(p.out) + i;
-  h2 o[2];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    if (p.epi_kind != EPI_NONE && (uint32_t)e < n) {
-      const float g = p.epi_dtype == RMLX_DTYPE_F32 ? static_cast<const float*>(p.epi)[i + e] : (float)static_cast<const _Float16*>(p.epi)[i + e];
-      v[e] = p.epi_kind == EPI_RESIDUAL ? v[e] + g : g / (1.0f + __expf(-g)) * v[e];
-    }
-    o[e / 2][e % 2] = (_Float16)v[e];
-  }
+  const h2 o[2] = {{(_Float16)v[0], (_Float16)v[1]}, {(_Float16)v[2], (_Float16)v[3]}};
   if (n == 4) {
-    struct __attribute__((packed, aligned(2))) u2_any { u2 v; };
     reinterpret_cast<u2_any*>(out)->v = (u2){h2bits(o[0]), h2bits(o[1])};
   } else {
     for (uint32_t e = 0; e < n; ++e) out[e] = o[e / 2][e % 2];
@@ -538,8 +531,8 @@ TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, double
   return e.plan;
 }
 
-size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N, int epi_kind) {
-  return plan.splits > 1 || epi_kind != EPI_NONE ? (size_t)plan.splits * M * N * sizeof(float) : 0;
+size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N) {
+  return plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
 }
 
 int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s) {
@@ -553,7 +546,7 @@ int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s) {
   p.tiles_m = (a.M + plan.mi * 32 - 1) / (plan.mi * 32);
   p.tiles_n = (a.N + plan.wn * 32 - 1) / (plan.wn * 32);
   p.splits = plan.splits;
-  p.partial = plan.splits > 1 || a.epi_kind != EPI_NONE ? static_cast<float*>(a.workspace) : nullptr;
+  p.partial = plan.splits > 1 ? static_cast<float*>(a.workspace) : nullptr;
   p.epi_kind = a.epi_kind; p.epi = a.epi; p.epi_dtype = a.epi_dtype;
   const uint64_t wgs = (uint64_t)p.tiles_m * p.tiles_n * p.splits;
   if (wgs > 0x7FFFFFFFull) return fail(RMLX_INVALID_SHAPE, "qmm: grid too large");

@@ -66,3 +66,24 @@ def test_residual_over_more_than_two_gib_of_sums(hip):
     e[:, cols] = rng.standard_normal((m, len(cols))).astype(np.float16)
     out = ops.qmm_add_residual(DeviceBuffer.from_numpy(x), qw, DeviceBuffer.from_numpy(e)).numpy()[:, cols]
     assert_close(out, model.qmm(x.astype(np.float64), words[cols], s[cols], b[cols], 64, 4) + e[:, cols].astype(np.float64), "residual")
+
+
+@pytest.mark.parametrize("m,n,k,bits", [(2048, 4096, 4096, 4), (3001, 14336, 4096, 4), (512, 12288, 4096, 8), (128, 12288, 4096, 4)])
+def test_fused_in_the_store_of_one_launch(hip, m, n, k, bits):
+    """No block of the output's size is taken for an epilogue, and the result is the f32 sum rounded once: added to the plain
+    product's f16 in 64 bits it differs by at most both roundings (2^-11 of either value)."""
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(m + n)
+    qw = ops.QuantizedWeight.from_numpy(*make_weight(rng, n, k, bits), 64, bits)
+    x = DeviceBuffer.from_numpy(make_x(rng, m, k))
+    e = rng.standard_normal((m, n)).astype(np.float16)
+    ed, stream = DeviceBuffer.from_numpy(e), hip.Stream()
+    plain = ops.affine_quantized_matmul_batched(x, qw, stream=stream)
+    stream.sync()
+    before = hip.scratch_allocations()
+    out = ops.qmm_add_residual(x, qw, ed, stream=stream)
+    stream.sync()
+    assert hip.scratch_allocations() == before
+    p, got = plain.numpy().astype(np.float64), out.numpy().astype(np.float64)
+    assert np.all(np.abs(got - (p + e)) <= 2.0 ** -11 * (np.abs(p) + np.abs(got)) * 1.01 + 1e-7)
