@@ -170,8 +170,7 @@ int32_t rmlx_hip_affine_quantized_matmul_batched(const rmlx_qweight* qw, const r
  * tiles (what kernel 2 resolves to when those tiles make at most one round over the chip and the register-weights GEMM
  * would need more than one round of its 32 x 64 tiles; K <= 4096), 11 = the MFMA GEMM with 32 x 64 tiles and K split four
  * ways inside the workgroup (4-bit weights at group size 64, N % 64 == 0, K % 2048 == 0), 12 = the large-tile MFMA GEMM
- * (tiles of up to 256 x 256; 4- / 8-bit weights, every group size, any N and K; selector 9
- * resolves to it where the automatic choice does). */
+ * (tiles of up to 256 x 256; 4- / 8-bit weights, every group size, any N and K). */
 int32_t rmlx_hip_qmm_select(const rmlx_qweight* qw, const rmlx_array* x, int32_t kernel,
                             void* out_f16_dev, size_t out_bytes, rmlx_stream stream);
 
