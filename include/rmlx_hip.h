@@ -170,7 +170,12 @@ int32_t rmlx_hip_affine_quantized_matmul_batched(const rmlx_qweight* qw, const r
  * tiles (what kernel 2 resolves to when those tiles make at most one round over the chip and the register-weights GEMM
  * would need more than one round of its 32 x 64 tiles; K <= 4096), 11 = the MFMA GEMM with 32 x 64 tiles and K split four
  * ways inside the workgroup (4-bit weights at group size 64, N % 64 == 0, K % 2048 == 0), 12 = the large-tile MFMA GEMM
- * (tiles of up to 256 x 256; 4- / 8-bit weights, every group size, any N and K). */
+ * (tiles of up to 256 x 256; 4- / 8-bit weights, every group size, any N and K), 13 = the same with exact weights, in two products,
+ * 14 = the multi-row streaming GEMV over 4-bit matrices that kernel 6 does not take (any N, any K of whole groups of 64 or 128).
+ * Precision: kernels 1, 3, 6, 13 and 14 multiply with scale * q + bias as it is (integer dot products scaled in f32, f32 weights, or two f16
+ * parts of 21 bits together); the GEMMs 2, 5 and 7 to 12 round every weight to f16, which adds 1.8e-4 of the result to the 2.1e-4 of
+ * rounding it.  The automatic choice rounds weights only where it has always run such a GEMM: 4- / 8-bit matrices in multiples of 64, at
+ * row counts beyond the GEMVs'. */
 int32_t rmlx_hip_qmm_select(const rmlx_qweight* qw, const rmlx_array* x, int32_t kernel,
                             void* out_f16_dev, size_t out_bytes, rmlx_stream stream);
 

@@ -149,6 +149,9 @@ struct QmvArgs {
 };
 int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s);
 bool qmv_q4_supported(uint32_t N, uint32_t K, uint32_t group_size);
+// The same over any N and any K of whole groups (64 or 128): plain matrices, f16 output
+bool qmv_q4_ragged_supported(uint32_t N, uint32_t K, uint32_t group_size);
+int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s);
 // Gate / up projection of single rows through chosen experts (qmv_m1.hip): position a = activation row a / top_k (x, no
 // row map) through expert idx[a] (idx == null: pick a % top_k of the ranking the kernel makes itself, see route_logits) of the two stacked matrices of `a` (w0 / w1, expert strides), out[a, :] = silu(gate) * up
 // in f16 [assignments, N]; 4- or 8-bit weights, the shapes of the single-row GEMV.  chunk_tab / M / mr of `a` are not used.
@@ -230,6 +233,7 @@ struct QmmArgs {
   int32_t epi_dtype;
   const void* w_packed = nullptr;  // K-split GEMMs: the weights in their tile-contiguous order (gemm_layout_bytes), or null
   uint32_t group_size = 64;        // LDS-staged GEMM (the other GEMMs take it as a launch argument)
+  int exact = 0;                   // tile GEMMs: weights in two products (tile.hpp) instead of rounded to f16
   bool workspace_has_partials = false;  // LDS-staged GEMM: the workspace was sized with N, so a launch of few tiles may split K
 };
 enum { EPI_NONE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2 };
@@ -276,6 +280,7 @@ struct GroupedQmmArgs {
   const uint32_t* row_map;   // nullable: source row of position p is row_map[p]
   void* out;                 // f16 [positions, N] (f32 when out_f32; not for a pair)
   int out_f32;
+  int exact;                 // tile GEMMs: see QmmArgs
   const uint32_t* tile_tab; const uint32_t* n_tiles_dev;
   uint32_t max_tiles;        // row tiles the grid covers (>= *n_tiles_dev)
   uint32_t tile_rows;        // rows per tile the table was built for: 32 or kGroupedTileRows
@@ -287,10 +292,10 @@ int32_t launch_qmm_rw_grouped(const GroupedQmmArgs& a, hipStream_t s);
 // (kw >= 4: qmm_slice.hip, mi 1 or 2), K cut into `splits` ranges (f32 partial sums in QmmArgs::workspace, added up by a second kernel).
 struct TilePlan { uint32_t wn, mi, kw, splits; };
 bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
-TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, double* us);  // us: estimated time of the launch
+TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us);  // us: estimated time of the launch
 size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N);
 int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s);
-// The same over a table of row tiles of 256 rows of one expert (x_rows: rows of x; out f16 or f32, a pair f16)
+// The same over a table of row tiles of 32, 64, 128 or 256 rows of one expert (x_rows: rows of x; out f16 or f32, a pair f16)
 bool qmm_tile_grouped_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits, uint32_t x_rows);
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
 // The same over row tiles of at most 32 rows, for few rows per expert (qmm_slice.hip)

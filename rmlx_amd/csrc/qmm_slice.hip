@@ -33,7 +33,7 @@ constexpr uint32_t slice_lds_all(int bits, int mi, int wn, int kg, int ks, int S
   return loop > sums ? loop : sums;
 }
 
-template <int BITS, int MI, int WN, int KG, int KS, int S, bool DUAL>
+template <int BITS, int MI, int WN, int KG, int KS, int S, bool DUAL, bool EXACT>
 __device__ __forceinline__ void slice_body(const TileParams p, const Tile t_, char* const lds) {
   constexpr int kWaves = WN * KG, BM = 32 * MI, BN = 64 * WN, BNO = DUAL ? BN / 2 : BN, KB = 16 * KS * KG;
   constexpr uint32_t kRound = kWaves * 1024, kUnitBytes = WN * 2048;
@@ -181,11 +181,16 @@ __device__ __forceinline__ void slice_body(const TileParams p, const Tile t_, ch
       for (int ni = 0; ni < 2; ++ni) {
         const _Float16 sv = __builtin_bit_cast(_Float16, (uint16_t)o.s[ni]), bv = __builtin_bit_cast(_Float16, (uint16_t)o.b[ni]);
         const h2 s2 = {sv, sv}, b2 = {bv, bv};
-        h8 w;
-        if constexpr (BITS == 4) w = weights_q4(o.w[ni][j], s2, b2);
-        else w = weights_q8(o.w[ni][2 * j], o.w[ni][2 * j + 1], s2, b2);
+        Weights w;
+        if constexpr (EXACT && BITS == 4) w = split_q4(o.w[ni][j], (float)sv, (float)bv);
+        else if constexpr (EXACT) w = split_q8(o.w[ni][2 * j], o.w[ni][2 * j + 1], (float)sv, (float)bv);
+        else if constexpr (BITS == 4) w.hi = weights_q4(o.w[ni][j], s2, b2);
+        else w.hi = weights_q8(o.w[ni][2 * j], o.w[ni][2 * j + 1], s2, b2);
 #pragma unroll
-        for (int i = 0; i < MI; ++i) acc[i][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w, o.a[i][j], acc[i][ni], 0, 0, 0);
+        for (int i = 0; i < MI; ++i) acc[i][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w.hi, o.a[i][j], acc[i][ni], 0, 0, 0);
+        if constexpr (EXACT)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) acc[i][ni] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w.lo, o.a[i][j], acc[i][ni], 0, 0, 0);
       }
   };
 
@@ -303,20 +308,21 @@ __device__ __forceinline__ void slice_body(const TileParams p, const Tile t_, ch
   }
 }
 
-template <int BITS, int MIMAX, int WN, int KG, int KS, int S, int WPE, bool DUAL>
+template <int BITS, int MIMAX, int WN, int KG, int KS, int S, int WPE, bool DUAL, bool EXACT>
 __global__ __launch_bounds__(WN * KG * 64, WPE) void qmm_slice_kernel(TileParams p) {
   __shared__ __align__(1024) char lds[slice_lds_all(BITS, MIMAX, WN, KG, KS, S)];
   Tile t;
   if (!tile_of(p, MIMAX * 32, &t)) return;
-  if (MIMAX == 2 && t.rows > 32) slice_body<BITS, MIMAX, WN, KG, KS, S, DUAL>(p, t, lds);
-  else slice_body<BITS, 1, WN, KG, KS, S, DUAL>(p, t, lds);
+  if (MIMAX == 2 && t.rows > 32) slice_body<BITS, MIMAX, WN, KG, KS, S, DUAL, EXACT>(p, t, lds);
+  else slice_body<BITS, 1, WN, KG, KS, S, DUAL, EXACT>(p, t, lds);
 }
 
 template <int BITS, int MI, int WN, int KG, int KS, int S, bool DUAL>
 void launch_one(const TileParams& p, dim3 grid, hipStream_t s) {
   // (two workgroups per CU where their LDS allows it)
   constexpr int kWpe = slice_lds_all(BITS, MI, WN, KG, KS, S) <= 80 * 1024 ? WN * KG / 2 : WN * KG / 4;
-  hipLaunchKernelGGL((qmm_slice_kernel<BITS, MI, WN, KG, KS, S, kWpe, DUAL>), grid, dim3(WN * KG * 64), 0, s, p);
+  if (p.exact) hipLaunchKernelGGL((qmm_slice_kernel<BITS, MI, WN, KG, KS, S, kWpe, DUAL, true>), grid, dim3(WN * KG * 64), 0, s, p);
+  else hipLaunchKernelGGL((qmm_slice_kernel<BITS, MI, WN, KG, KS, S, kWpe, DUAL, false>), grid, dim3(WN * KG * 64), 0, s, p);
 }
 
 template <int BITS>
@@ -342,7 +348,7 @@ int32_t launch_qmm_slice_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipSt
   TileParams p{};
   p.w = a.w; p.s = a.s; p.b = a.b; p.w1 = a.w1; p.s1 = a.s1; p.b1 = a.b1;
   p.x = a.x; p.out = a.out; p.N = a.N; p.K = a.K; p.group_size = a.group_size;
-  p.out_f32 = a.out_f32;
+  p.out_f32 = a.out_f32; p.exact = a.exact;
   p.tile_tab = a.tile_tab; p.n_tiles = a.n_tiles_dev; p.row_map = a.row_map; p.x_rows = x_rows;
   p.estride_w = a.expert_stride_w; p.estride_s = a.expert_stride_s;
   p.splits = 1;

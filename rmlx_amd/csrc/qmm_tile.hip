@@ -49,7 +49,7 @@ constexpr uint32_t kernel_lds() {
   return most;
 }
 
-template <int BITS, int WN, int MI, int KW, bool DUAL>
+template <int BITS, int WN, int MI, int KW, bool DUAL, bool EXACT>
 __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, char* lds) {
   constexpr int BM = MI * 32, BN = WN * 32, BNO = DUAL ? BN / 2 : BN, S = kStages, R = (S + 1) / 2;
   constexpr int kThreads = WN * KW * 64, kPieces = (BM / 8 + WN - 1) / WN * WN;
@@ -167,9 +167,13 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
     b2 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(braw, braw, 0x01000100u));
   };
   auto word = [](const u4& v, int c) -> uint32_t { return c == 0 ? v.x : (c == 1 ? v.y : (c == 2 ? v.z : v.w)); };
-  auto operand = [&](int k) -> h8 {
-    if constexpr (BITS == 4) return weights_q4(word(wq[0], k), s2, b2);
-    else return weights_q8(word(wq[(k >> 1) % WV], 2 * (k & 1)), word(wq[(k >> 1) % WV], 2 * (k & 1) + 1), s2, b2);
+  auto operand = [&](int k) -> Weights {
+    Weights w;
+    if constexpr (EXACT && BITS == 4) w = split_q4(word(wq[0], k), (float)s2[0], (float)b2[0]);
+    else if constexpr (EXACT) w = split_q8(word(wq[(k >> 1) % WV], 2 * (k & 1)), word(wq[(k >> 1) % WV], 2 * (k & 1) + 1), (float)s2[0], (float)b2[0]);
+    else if constexpr (BITS == 4) w.hi = weights_q4(word(wq[0], k), s2, b2);
+    else w.hi = weights_q8(word(wq[(k >> 1) % WV], 2 * (k & 1)), word(wq[(k >> 1) % WV], 2 * (k & 1) + 1), s2, b2);
+    return w;
   };
 
   f16v acc[MI];
@@ -192,7 +196,8 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
     // Few fragments: a group of matrix instructions is shorter than an LDS read.  All operands of a step are read during the step
     // before, each into the registers that its predecessor has just left; group t + S goes out during step t into step t's slots.
     wait_dma_and_barrier<(S - 2) * kStep + (R - 1) * kRound>();  // groups 0 and 1 have arrived
-    h8 bf[4][MI], wf;
+    h8 bf[4][MI];
+    Weights wf;
     load_sb(t0);
     load_wq(0, 0);
 #pragma unroll
@@ -218,9 +223,15 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
       for (int k = 0; k < 4; ++k) {
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf, bf[k][i], acc[i], 0, 0, 0);
-          bf[k][i] = read_a(nxt, i, k);
+          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf.hi, bf[k][i], acc[i], 0, 0, 0);
+          if constexpr (!EXACT) bf[k][i] = read_a(nxt, i, k);
         }
+        if constexpr (EXACT)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) {
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf.lo, bf[k][i], acc[i], 0, 0, 0);
+            bf[k][i] = read_a(nxt, i, k);
+          }
         if (k < 3) {
           wf = operand(k + 1);
           dma_group(std::integral_constant<bool, par == 1>{}, t + S, slot8 * kABytes, BITS == 8 ? slot8 : slot_r, k);
@@ -243,7 +254,8 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
   } else {
     // Group t + S - 1 goes out during step t, between its matrix instructions, into the slots that step t - 1 has left.
     wait_dma_and_barrier<(S - 2) * kStep + (R - 2) * kRound>();
-    h8 bf[MI], wf;
+    h8 bf[MI];
+    Weights wf;
     load_sb(t0);
     load_wq(0, 0);
 #pragma unroll
@@ -259,7 +271,8 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
       const uint32_t nxt = slot_nxt * kABytes;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        h8 bn[MI], wn;
+        h8 bn[MI];
+        Weights wn;
         if (k < 3) {
 #pragma unroll
           for (int i = 0; i < MI; ++i) bn[i] = read_a(stage, i, k + 1);
@@ -274,7 +287,10 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
           for (int i = 0; i < MI; ++i) bn[i] = read_a(nxt, i, 0);
         }
 #pragma unroll
-        for (int i = 0; i < MI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf, bf[i], acc[i], 0, 0, 0);
+        for (int i = 0; i < MI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf.hi, bf[i], acc[i], 0, 0, 0);
+        if constexpr (EXACT)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf.lo, bf[i], acc[i], 0, 0, 0);
         if (k == 3) {
           pick_sb();
           wn = operand(0);
@@ -396,7 +412,7 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
   }
 }
 
-template <int BITS, int WN, int MIMAX, int KW, bool DUAL>
+template <int BITS, int WN, int MIMAX, int KW, bool DUAL, bool EXACT>
 __global__ __launch_bounds__(WN * KW * 64, 2) void qmm_tile_kernel(TileParams p) {
   __shared__ __align__(1024) char lds[kernel_lds<BITS, WN, MIMAX, KW>()];
   Tile t;
@@ -404,7 +420,7 @@ __global__ __launch_bounds__(WN * KW * 64, 2) void qmm_tile_kernel(TileParams p)
   const uint32_t frags = (t.rows + 31) / 32;
   auto go = [&](auto mi) {
     constexpr int MI = decltype(mi)::value;
-    if constexpr (MI <= MIMAX) tile_body<BITS, WN, MI, KW, DUAL>(p, t, lds);
+    if constexpr (MI <= MIMAX) tile_body<BITS, WN, MI, KW, DUAL, EXACT>(p, t, lds);
   };
   using std::integral_constant;
   switch (frags) {
@@ -441,19 +457,25 @@ __global__ __launch_bounds__(256) void tile_splits_sum_kernel(TileParams p) {
   }
 }
 
+template <int BITS, bool EXACT>
+void launch_tile_as(const TileParams& p, const TilePlan& plan, dim3 grid, hipStream_t s) {
+  if (p.w1 != nullptr) {
+    if (plan.mi == 8) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 8, 8, 1, true, EXACT>), grid, dim3(512), 0, s, p);
+    else if (plan.mi == 4) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 4, 1, true, EXACT>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 2, 1, true, EXACT>), grid, dim3(256), 0, s, p);
+  }
+  else if (plan.wn == 8 && plan.mi == 8) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 8, 8, 1, false, EXACT>), grid, dim3(512), 0, s, p);
+  else if (plan.wn == 8) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 8, 4, 1, false, EXACT>), grid, dim3(512), 0, s, p);
+  else if (plan.mi == 4 && plan.kw == 1) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 4, 1, false, EXACT>), grid, dim3(256), 0, s, p);
+  else if (plan.mi == 4) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 4, 2, false, EXACT>), grid, dim3(512), 0, s, p);
+  else if (plan.kw == 1) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 2, 1, false, EXACT>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 2, 2, false, EXACT>), grid, dim3(512), 0, s, p);
+}
+
 template <int BITS>
 void launch_tile(const TileParams& p, const TilePlan& plan, dim3 grid, hipStream_t s) {
-  if (p.w1 != nullptr) {
-    if (plan.mi == 8) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 8, 8, 1, true>), grid, dim3(512), 0, s, p);
-    else if (plan.mi == 4) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 4, 1, true>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 2, 1, true>), grid, dim3(256), 0, s, p);
-  }
-  else if (plan.wn == 8 && plan.mi == 8) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 8, 8, 1, false>), grid, dim3(512), 0, s, p);
-  else if (plan.wn == 8) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 8, 4, 1, false>), grid, dim3(512), 0, s, p);
-  else if (plan.mi == 4 && plan.kw == 1) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 4, 1, false>), grid, dim3(256), 0, s, p);
-  else if (plan.mi == 4) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 4, 2, false>), grid, dim3(512), 0, s, p);
-  else if (plan.kw == 1) hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 2, 1, false>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((qmm_tile_kernel<BITS, 4, 2, 2, false>), grid, dim3(512), 0, s, p);
+  if (p.exact) launch_tile_as<BITS, true>(p, plan, grid, s);
+  else launch_tile_as<BITS, false>(p, plan, grid, s);
 }
 
 }  // namespace
@@ -468,7 +490,7 @@ bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
 // 1, 2, .. of them); fragments cost half as much on an idle chip as on a full one, where the clock falls.  A launch adds its start
 // and end, a K split the kernel that adds up the partial sums.  Fitted to about 15000 timed launches (780 shapes, every plan and
 // split): 6 % mean error, and the picks are 1.3 % slower on average than the fastest plan.
-static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, double* us) {
+static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us) {
   // (kw >= 4: waves along k, steps of `k` values)
   struct Cost { uint32_t wn, mi, kw; int per_cu; double start, step[3][2], sum, sum_per_mi; uint32_t k; };
   static const Cost costs[2][10] = {
@@ -492,6 +514,7 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
        {2, 2, 8, 1, 5.17, {{0.061, 0.452}}, 2.30, 0.00, 256},
        {4, 1, 4, 1, 4.56, {{0.032, 1.080}}, 3.39, 0.00, 256},
        {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128}}};
+  constexpr double kExactStep = 1.6;  // two products: 8 to 2000 rows 1.57 to 1.7 x, 8-bit up to 64 rows 1.35
   const double cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
   const uint32_t rounds = (K + 127) / 128;
   TilePlan best{4, 2, 1, 1};
@@ -505,11 +528,12 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
       if (splits > 1 && (rounds < 2 * splits * c.kw || (double)(tiles * splits) > 1.6 * c.per_cu * cus || (uint64_t)splits * M * N > (1u << 27))) break;
       const double load = (double)(tiles * splits) / cus, full = std::floor(load / c.per_cu), rest = load - full * c.per_cu;
       const double steps = c.k != 0 ? (stages + splits - 1) / splits : 2.0 * ((((rounds + splits - 1) / splits) + c.kw - 1) / c.kw);
-      double t = c.start + steps * full * (c.step[c.per_cu - 1][0] + c.step[c.per_cu - 1][1] * frags);
+      double t = steps * full * (c.step[c.per_cu - 1][0] + c.step[c.per_cu - 1][1] * frags);
       if (rest > 1e-9) {
         const double* s = c.step[(int)std::ceil(rest - 1e-9) - 1];
         t += steps * (s[0] + s[1] * frags * (full > 0 || load >= 1 ? 1.0 : 0.5 + 0.5 * load));
       }
+      t = c.start + (exact ? kExactStep : 1.0) * t;
       if (splits > 1) t += c.sum + c.sum_per_mi * splits * ((double)M * N / (1 << 20));
       if (t < best_us) { best_us = t; best = TilePlan{c.wn, c.mi, c.kw, splits}; }
     }
@@ -519,13 +543,14 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
 }
 
 // (about 1 us of arithmetic, asked for twice per call by launches that take 5: the last plans of a thread are kept)
-TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, double* us) {
+TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us) {
   struct Kept { uint32_t M, N, K, bits; TilePlan plan; double us; };
   thread_local Kept kept[64] = {};
-  Kept& e = kept[(M * 31 + N * 7 + K + bits) & 63];
-  if (e.M != M || e.N != N || e.K != K || e.bits != bits) {
-    e.plan = estimate_plan(M, N, K, bits, &e.us);
-    e.M = M; e.N = N; e.K = K; e.bits = bits;
+  const uint32_t kind = bits + (exact ? 1 : 0);
+  Kept& e = kept[(M * 31 + N * 7 + K + kind) & 63];
+  if (e.M != M || e.N != N || e.K != K || e.bits != kind) {
+    e.plan = estimate_plan(M, N, K, bits, exact, &e.us);
+    e.M = M; e.N = N; e.K = K; e.bits = kind;
   }
   if (us != nullptr) *us = e.us;
   return e.plan;
@@ -547,7 +572,7 @@ int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s) {
   p.tiles_n = (a.N + plan.wn * 32 - 1) / (plan.wn * 32);
   p.splits = plan.splits;
   p.partial = plan.splits > 1 ? static_cast<float*>(a.workspace) : nullptr;
-  p.epi_kind = a.epi_kind; p.epi = a.epi; p.epi_dtype = a.epi_dtype;
+  p.epi_kind = a.epi_kind; p.epi = a.epi; p.epi_dtype = a.epi_dtype; p.exact = a.exact;
   const uint64_t wgs = (uint64_t)p.tiles_m * p.tiles_n * p.splits;
   if (wgs > 0x7FFFFFFFull) return fail(RMLX_INVALID_SHAPE, "qmm: grid too large");
   if (plan.kw >= 4) launch_qmm_slice(p, a.bits, plan, dim3((unsigned)wgs), s);
@@ -570,7 +595,7 @@ int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStr
   TileParams p{};
   p.w = a.w; p.s = a.s; p.b = a.b; p.w1 = a.w1; p.s1 = a.s1; p.b1 = a.b1;
   p.x = a.x; p.out = a.out; p.N = a.N; p.K = a.K; p.group_size = a.group_size;
-  p.out_f32 = a.out_f32;
+  p.out_f32 = a.out_f32; p.exact = a.exact;
   p.tile_tab = a.tile_tab; p.n_tiles = a.n_tiles_dev; p.row_map = a.row_map; p.x_rows = x_rows;
   p.estride_w = a.expert_stride_w; p.estride_s = a.expert_stride_s;
   p.splits = 1;

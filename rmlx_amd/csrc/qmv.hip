@@ -82,10 +82,13 @@ struct KParams {
 // (for workgroups that take several tiles; a workgroup with one tile keeps the registers for a third resident
 // workgroup per CU);
 // before the tile loop (their registers are free again when the weight loads start).
-template <int MR, int TILES, bool TAB, int SPW, bool PAIR, int REUSE>
+// RAGGED: any number of weight rows (those past the last repeat it, unstored) and a K of whole groups of 64: the lanes of the last
+// slab's second half, where K ends in its middle, multiply the row's last piece with activations of zero and a scale of zero.
+template <int MR, int TILES, bool TAB, int SPW, bool PAIR, int REUSE, bool RAGGED = false>
 __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4 : 1) void qmv_q4_kernel(KParams p) {
   static_assert(!REUSE || SPW != 0, "reuse needs a uniform slab count");
   static_assert(!PAIR || TILES == 2, "paired tiles need two tile slots");
+  static_assert(!RAGGED || (!TAB && SPW == 0 && REUSE == 0 && (TILES == 1 || PAIR)), "one matrix, guarded loads");
   constexpr int kSlots = 4 * MR;                       // 16-byte activation slots per (slab, j) block ...
   constexpr int kBlk = kSlots + 1;                     // ... followed by one slot of zeros (read by the lanes whose operand rows are empty)
   constexpr int kXsWave = kSpwMax * 4 * kBlk * 16;     // bytes of activation image per wave
@@ -123,7 +126,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
   const uint32_t K = p.K, KS = p.ks, NT = kWaves / KS;
   const uint32_t kp = wave % KS, tw = wave / KS;
   // group size 128 (p.gs128): one scale per slab, applied to both halves of it
-  const uint32_t words_per_row = K >> 3, groups_per_row = p.gs128 ? K >> 7 : K >> 6, slabs_total = K >> 7;
+  const uint32_t words_per_row = K >> 3, groups_per_row = p.gs128 ? K >> 7 : K >> 6, slabs_total = RAGGED ? (K + 127) >> 7 : K >> 7;
   constexpr bool pair = PAIR;
   const uint32_t rows_per_slot = pair ? 32u : 16u;  // weight rows (of one matrix) per wave tile slot
 
@@ -152,7 +155,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
 #pragma unroll
     for (int m = 0; m < MR; ++m) {
       xv[m] = (u4){0u, 0u, 0u, 0u};
-      if ((uint32_t)m < rows && lane < my * 16)
+      if ((uint32_t)m < rows && lane < my * 16 && (!RAGGED || (uint32_t)(sl * 16 + lane) * 8 < K))
         xv[m] = *reinterpret_cast<const u4*>(p.x + (uint64_t)srcs[m] * K + (uint32_t)(sl * 16 + lane) * 8);
     }
   };
@@ -207,7 +210,8 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
     for (int t = 0; t < TILES; ++t) {
       const uint64_t e_w = TAB ? expert * p.estride_w : 0, e_s = TAB ? expert * p.estride_s : 0;
       const bool first = t == 0 || pair;                       // which matrix
-      const uint32_t wr = tile_row + n + (pair ? 16 * t : 0);  // which row of it
+      uint32_t wr = tile_row + n + (pair ? 16 * t : 0);        // which row of it
+      if (RAGGED) wr = wr < p.ld_out ? wr : p.ld_out - 1;
       wrow[t] = reinterpret_cast<const u4*>((first ? p.w0 : p.w1) + e_w + (uint64_t)wr * words_per_row) + g;
       // scales live in the lanes with even g, biases in the lanes with odd g (exchanged later)
       const __half* sb = (g & 1) ? (first ? p.b0 : p.b1) : (first ? p.s0 : p.s1);
@@ -221,6 +225,17 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
         const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + sl;
         const uint32_t h0 = my > 0 ? hp[0] : 0u, h1 = my > 1 ? hp[1] : 0u, h2 = my > 2 ? hp[2] : 0u, h3 = my > 3 ? hp[3] : 0u;
         sbv[t] = (u4){h0 | (h0 << 16), h1 | (h1 << 16), h2 | (h2 << 16), h3 | (h3 << 16)};
+        continue;
+      }
+      if constexpr (RAGGED) {  // (rows of an odd number of groups begin at any even address)
+        struct __attribute__((packed, aligned(2))) Pair { uint32_t v; };
+        const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + 2 * sl;
+#pragma unroll
+        for (int it = 0; it < kSpwMax; ++it) {
+          if (it >= my) continue;
+          const uint32_t v = 2u * (uint32_t)(sl + it) + 1 < groups_per_row ? reinterpret_cast<const Pair*>(hp + 2 * it)->v : hp[2 * it];
+          sbv[t][it] = v;
+        }
         continue;
       }
       const uint32_t* sp = reinterpret_cast<const uint32_t*>(sbrow[t]) + sl;
@@ -237,7 +252,11 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
     for (int it = 0; it < kSpwMax; ++it) {
       if (it < my) {
 #pragma unroll
-        for (int t = 0; t < TILES; ++t) wreg[t][it] = *(wrow[t] + (sl + it) * 4);
+        for (int t = 0; t < TILES; ++t) {
+          uint32_t piece = (sl + it) * 4;
+          if (RAGGED) piece = piece + g < words_per_row / 4 ? piece : words_per_row / 4 - 1 - g;  // (at least two pieces in the slab)
+          wreg[t][it] = *(wrow[t] + (int32_t)piece);
+        }
       }
     }
   };
@@ -372,11 +391,12 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
         }
         v[t] = acc;
       }
-      const uint64_t obase = (uint64_t)(row0 + m) * p.ld_out + (wg_tile * NT + otw) * rows_per_slot + nn;
+      const uint32_t col = (wg_tile * NT + otw) * rows_per_slot + nn;
+      const uint64_t obase = (uint64_t)(row0 + m) * p.ld_out + col;
       if (TILES == 2 && !pair) v[0] = silu_f(v[0]) * v[TILES - 1];
 #pragma unroll
       for (int t = 0; t < TILES; ++t) {
-        if (t == 0 || pair) {
+        if ((t == 0 || pair) && (!RAGGED || col + 16 * t < p.ld_out)) {
           const float r = write_zeros ? 0.f : v[t];
           if (p.out_f32) reinterpret_cast<float*>(p.out)[obase + 16 * t] = r;
           else reinterpret_cast<__half*>(p.out)[obase + 16 * t] = __float2half(r);
@@ -550,6 +570,36 @@ int32_t launch_build_gather_chunks(const uint32_t* indices, uint32_t batch, uint
 // K in whole slabs of 128: a wave takes up to four slabs per pass, the last part of a pass may be shorter or empty.
 bool qmv_q4_supported(uint32_t N, uint32_t K, uint32_t group_size) {
   return (group_size == 64 || group_size == 128) && N % 16 == 0 && K % 128 == 0 && N > 0 && K > 0;
+}
+
+bool qmv_q4_ragged_supported(uint32_t N, uint32_t K, uint32_t group_size) {
+  return (group_size == 64 || group_size == 128) && N > 0 && K > 0 && K % group_size == 0;
+}
+
+// Rows of x over a matrix off the multiples above: one tile of 16 or, where those fill the chip, 32 weight rows per wave.
+int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s) {
+  if (!qmv_q4_ragged_supported(a.N, a.K, a.group_size) || a.dual || a.chunk_tab != nullptr || a.out_f32 || a.ld_out != a.N)
+    return fail(RMLX_INVALID_SHAPE, "qmv_q4 (ragged): unsupported shape N=%u K=%u group_size=%u", a.N, a.K, a.group_size);
+  if (a.M == 0) return RMLX_OK;
+  KParams p{};
+  p.w0 = a.w0; p.s0 = a.s0; p.b0 = a.b0;
+  p.w1 = a.w0; p.s1 = a.s0; p.b1 = a.b0;
+  p.x = a.x; p.out = a.out;
+  p.K = a.K; p.ld_out = a.ld_out; p.M = a.M;
+  p.gs128 = a.group_size == 128 ? 1u : 0u;
+  p.x_bf16 = a.x_bf16 ? 1u : 0u;
+  p.tpw = 1;
+  p.ks = 1;
+  while (p.ks < 8 && p.ks * kSpwMax * 128 < a.K) p.ks *= 2;
+  const uint32_t chunks = (a.M + 7) / 8, rows = 16 * (8 / p.ks);
+  const bool pair = a.M > 4 && (uint64_t)((a.N + 2 * rows - 1) / (2 * rows)) * chunks >= (uint32_t)ctx().num_cus;
+  if (chunks > 65535) return fail(RMLX_INVALID_SHAPE, "qmv_q4 (ragged): too many rows (M=%u)", a.M);
+  const dim3 grid((a.N + (pair ? 2 * rows : rows) - 1) / (pair ? 2 * rows : rows), chunks);
+  if (pair) hipLaunchKernelGGL((qmv_q4_kernel<8, 2, false, 0, true, 0, true>), grid, dim3(kThreads), 0, s, p);
+  else if (a.M > 4) hipLaunchKernelGGL((qmv_q4_kernel<8, 1, false, 0, false, 0, true>), grid, dim3(kThreads), 0, s, p);
+  else hipLaunchKernelGGL((qmv_q4_kernel<4, 1, false, 0, false, 0, true>), grid, dim3(kThreads), 0, s, p);
+  RMLX_HIP_CHECK(hipGetLastError());
+  return RMLX_OK;
 }
 
 int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s) {

@@ -10,7 +10,7 @@ struct TileParams {
   const __half* x; void* out;
   float* partial;                   // not null: f32 partial sums [splits, M, N]
   uint32_t M, N, K, group_size, tiles_m, tiles_n, splits;
-  int32_t out_f32, epi_kind, epi_dtype;
+  int32_t exact, out_f32, epi_kind, epi_dtype;
   const void* epi;
   // grouped: (expert, first row, rows) per row tile, their number, optional gather of the activation rows, strides per expert
   const uint32_t* tile_tab; const uint32_t* n_tiles; const uint32_t* row_map;
@@ -113,6 +113,44 @@ __device__ __forceinline__ void tile_epilogue(const TileParams& p, uint64_t o, u
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = p.epi_kind == EPI_RESIDUAL ? v[e] + g[e] : g[e] / (1.0f + __expf(-g[e])) * v[e];
+}
+
+// The operand of a k step: weights rounded to f16 (lo unused), or, EXACT, w = scale * q + bias rounded once to f32 and cut into hi + lo
+// of 11 bits each, multiplied one after the other (hi towards zero, so that both have one sign; 21 to 22 bits of the weight are kept, of
+// weights below 2^-4 the bits down to 2^-24).  Costs 16 vector instructions a word and a product per fragment on top:
+// 64 rows, 33001 x 2880 50.5 against 35.9 us, 2000 x 20001 x 4096 567 against 341 us; error against 64 bits 2.07e-4 of the result, that of
+// rounding it, against 2.75e-4 (E = 16, top-2 experts: 2.2e-4 against 4.4e-4).
+struct Weights { h8 hi, lo; };
+__device__ __forceinline__ void split_pair(float w0, float w1, h2* hi, h2* lo) {
+  const h2 h = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(w0, w1));
+  *hi = h;
+  *lo = (h2){(_Float16)__builtin_fmaf((float)h[0], -1.0f, w0), (_Float16)__builtin_fmaf((float)h[1], -1.0f, w1)};
+}
+__device__ __forceinline__ Weights split_q4(uint32_t w, float s, float b) {
+  const uint32_t even = w & 0x0F0F0F0Fu, odd = (w >> 4) & 0x0F0F0F0Fu;
+  const uint32_t v[2] = {__builtin_amdgcn_perm(odd, even, 0x05010400u), __builtin_amdgcn_perm(odd, even, 0x07030602u)};
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  Weights o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f2 q = i % 2 == 0 ? __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v[i / 2], 512.0f, false) : __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v[i / 2], 512.0f, true);
+    h2 hi, lo;
+    split_pair(__builtin_fmaf(q.x, s, b), __builtin_fmaf(q.y, s, b), &hi, &lo);
+    o.hi[2 * i] = hi[0]; o.hi[2 * i + 1] = hi[1]; o.lo[2 * i] = lo[0]; o.lo[2 * i + 1] = lo[1];
+  }
+  return o;
+}
+__device__ __forceinline__ Weights split_q8(uint32_t w0, uint32_t w1, float s, float b) {
+  Weights o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w = i < 2 ? w0 : w1;
+    const float q0 = (float)((w >> (i % 2 * 16)) & 0xFFu), q1 = (float)((w >> (i % 2 * 16 + 8)) & 0xFFu);
+    h2 hi, lo;
+    split_pair(__builtin_fmaf(q0, s, b), __builtin_fmaf(q1, s, b), &hi, &lo);
+    o.hi[2 * i] = hi[0]; o.hi[2 * i + 1] = hi[1]; o.lo[2 * i] = lo[0]; o.lo[2 * i + 1] = lo[1];
+  }
+  return o;
 }
 
 struct Tile { uint32_t mt, nt, split, expert, row_lo, rows; bool zeros; };
