@@ -295,8 +295,9 @@ bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
 TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us);  // us: estimated time of the launch
 size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N);
 int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s);
-// The same over a table of row tiles of 32, 64, 128 or 256 rows of one expert (x_rows: rows of x; out f16 or f32, a pair f16)
-bool qmm_tile_grouped_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits, uint32_t x_rows);
+// The same over a table of row tiles of 32, 64, 128 or 256 rows of one expert (x_rows: rows of x; out f16 or f32, a pair f16).  A row map
+// reaches the rows of an x of at most 2 GiB.
+bool qmm_tile_maps_rows(uint32_t x_rows, uint32_t K);
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
 // The same over row tiles of at most 32 rows, for few rows per expert (qmm_slice.hip)
 int32_t launch_qmm_slice_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
@@ -311,6 +312,7 @@ int32_t launch_topk_route(const float* logits, const float* bias, uint32_t T, ui
 // Stable counting sort; also emits the chunk table used by the GEMV family
 // (chunk_tab: 3 u32 per chunk; n_chunks: 1 u32).  chunk_tab / n_chunks may be null.
 // sorted_tok (nullable): token of each sorted position, sorted[p] / top_k.
+constexpr int kMaxSortedExperts = 1024;
 int32_t launch_moe_sort(const uint32_t* idx, uint32_t n_assign, uint32_t E, uint32_t top_k, uint32_t* sorted,
                         uint32_t* sorted_tok, uint32_t* inv, uint32_t* counts, uint32_t* offsets,
                         uint32_t* chunk_tab, uint32_t* n_chunks, uint32_t chunk_rows, hipStream_t s,

@@ -12,7 +12,7 @@
 namespace rmlx {
 namespace {
 
-constexpr int kMaxExperts = 1024;  // LDS histogram capacity of the sort kernel
+constexpr int kMaxExperts = kMaxSortedExperts;  // LDS histogram capacity of the sort kernel
 
 // ---- routing: one wave per token (route.hpp) --------------------------------------------------
 // (`lds_idx`: optional copy of the picks in workgroup memory, for a sort fused behind the routing)

@@ -52,8 +52,8 @@ __device__ __forceinline__ void slice_body(const TileParams p, const Tile t_, ch
   // Chunks of a row lie xor-ed with its number, so that operand reads spread over the banks; the xor is made on the address that a
   // lane loads from.  Rows past the tile's last repeat it; k past the row is loaded as zeros.
   auto at = [](const void* q, uint64_t o) { return static_cast<const void*>(static_cast<const char*>(q) + o); };
-  const bool grouped = p.tile_tab != nullptr;
-  const u4 xr = grouped ? rsrc(p.x, (uint64_t)p.x_rows * K * 2) : rsrc(at(p.x, (uint64_t)row_lo * K * 2), (uint64_t)rows * K * 2);
+  const bool mapped = p.row_map != nullptr;  // (of a grouped launch: rows from anywhere in x, which is at most 2 GiB then)
+  const u4 xr = mapped ? rsrc(p.x, (uint64_t)p.x_rows * K * 2) : rsrc(at(p.x, (uint64_t)row_lo * K * 2), (uint64_t)rows * K * 2);
   constexpr uint32_t kAPiece = 64 / CA, kWPiece = 64 / CW;    // rows of a 1 KB load
   static_assert(kWaves * kAPiece % 16 == 0 && kWaves * kWPiece % 16 == 0, "one xor for all loads of a lane");
   const uint32_t a_row = wave * kAPiece + lane / CA, ca16 = ((lane % CA) ^ (a_row & 15)) * 16;
@@ -62,7 +62,7 @@ __device__ __forceinline__ void slice_body(const TileParams p, const Tile t_, ch
   for (int q = 0; q < NA; ++q) {
     uint32_t m = q * kWaves * kAPiece + a_row;
     m = m < rows ? m : rows - 1;
-    if (grouped) m = p.row_map != nullptr ? p.row_map[row_lo + m] : row_lo + m;
+    if (mapped) m = p.row_map[row_lo + m];
     aoff[q] = m * K * 2 + ca16;
   }
   // LDS row li of the weights: column wn 64 + ni 32 + r of the tile; of a pair: column wn 32 + r of the gate (ni = 0) or up matrix
@@ -342,8 +342,8 @@ void launch_qmm_slice(const TileParams& p, uint32_t bits, const TilePlan& plan, 
 }
 
 int32_t launch_qmm_slice_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s) {
-  if (!qmm_tile_grouped_supported(a.N, a.K, a.group_size, a.bits, x_rows))
-    return fail(RMLX_INVALID_SHAPE, "grouped qmm: unsupported shape N=%u K=%u bits=%u group_size=%u", a.N, a.K, a.bits, a.group_size);
+  if (!qmm_tile_supported(a.N, a.K, a.group_size, a.bits) || (a.row_map != nullptr && !qmm_tile_maps_rows(x_rows, a.K)))
+    return fail(RMLX_INVALID_SHAPE, "grouped qmm: unsupported shape N=%u K=%u bits=%u group_size=%u, %u rows", a.N, a.K, a.bits, a.group_size, x_rows);
   if (a.max_tiles == 0) return RMLX_OK;
   TileParams p{};
   p.w = a.w; p.s = a.s; p.b = a.b; p.w1 = a.w1; p.s1 = a.s1; p.b1 = a.b1;

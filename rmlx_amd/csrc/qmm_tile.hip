@@ -76,14 +76,14 @@ __device__ __forceinline__ void tile_body(const TileParams p, const Tile t_, cha
   // activations: a piece = 8 rows of 128 bytes; the 16-byte chunk is xor-ed with the row so that the operand reads spread over
   // the banks.  Rows past the tile's last repeat it.
   const uint32_t ca = (lane & 7) ^ ((((wv & 1) * 8 + (lane >> 3)) >> 1) & 7);
-  const bool grouped = p.tile_tab != nullptr;
-  const u4 xr = grouped ? rsrc(p.x, (uint64_t)p.x_rows * K * 2) : rsrc(at(p.x, (uint64_t)row_lo * K * 2), (uint64_t)rows * K * 2);
+  const bool mapped = p.row_map != nullptr;  // (of a grouped launch: rows from anywhere in x, which is at most 2 GiB then)
+  const u4 xr = mapped ? rsrc(p.x, (uint64_t)p.x_rows * K * 2) : rsrc(at(p.x, (uint64_t)row_lo * K * 2), (uint64_t)rows * K * 2);
   uint32_t aoff[NA];
 #pragma unroll
   for (int q = 0; q < NA; ++q) {
     uint32_t m = (q * WN + wv) * 8 + (lane >> 3);
     m = m < rows ? m : rows - 1;
-    if (grouped) m = p.row_map != nullptr ? p.row_map[row_lo + m] : row_lo + m;
+    if (mapped) m = p.row_map[row_lo + m];
     aoff[q] = m * K * 2;
   }
   // weights: a piece = 16 rows of 64 bytes.  A pair's tile holds BN / 2 gate rows, then the same rows of the up matrix.
@@ -588,8 +588,8 @@ int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s) {
 }
 
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s) {
-  if (!qmm_tile_grouped_supported(a.N, a.K, a.group_size, a.bits, x_rows))
-    return fail(RMLX_INVALID_SHAPE, "grouped qmm: unsupported shape N=%u K=%u bits=%u group_size=%u", a.N, a.K, a.bits, a.group_size);
+  if (!qmm_tile_supported(a.N, a.K, a.group_size, a.bits) || (a.row_map != nullptr && !qmm_tile_maps_rows(x_rows, a.K)))
+    return fail(RMLX_INVALID_SHAPE, "grouped qmm: unsupported shape N=%u K=%u bits=%u group_size=%u, %u rows", a.N, a.K, a.bits, a.group_size, x_rows);
   if (a.max_tiles == 0) return RMLX_OK;
   if (a.tile_rows == 32) return launch_qmm_slice_grouped(a, x_rows, s);
   TileParams p{};
@@ -610,8 +610,6 @@ int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStr
   return RMLX_OK;
 }
 
-bool qmm_tile_grouped_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits, uint32_t x_rows) {
-  return qmm_tile_supported(N, K, group_size, bits) && (uint64_t)x_rows * K * 2 <= 0x80000000ull;
-}
+bool qmm_tile_maps_rows(uint32_t x_rows, uint32_t K) { return (uint64_t)x_rows * K * 2 <= 0x80000000ull; }
 
 }  // namespace rmlx

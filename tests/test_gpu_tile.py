@@ -101,3 +101,57 @@ def test_gather_on_large_tiles(hip, batch, rows, n, k, gs):
     for i in range(batch):
         ref = model.qmm(x[i].astype(np.float64), words[idx[i]], s[idx[i]], b[idx[i]], gs, 4)
         assert_close(out[i], ref, f"gather entry {i}")
+
+
+def _block(rng, experts, hidden, inter, bits=4, gs=64):
+    from rmlx_amd import ops
+    gate, up = (make_weight(rng, inter, hidden, bits, gs, (experts,)) for _ in range(2))
+    down = make_weight(rng, hidden, inter, bits, gs, (experts,))
+    return (gate, up, down), tuple(ops.QuantizedWeight.from_numpy(*w, gs, bits) for w in (gate, up, down))
+
+
+@pytest.mark.parametrize("tokens,experts,top_k,hidden,inter", [(262200, 8, 8, 512, 512), (131100, 2, 1, 8192, 512)])
+def test_routed_block_over_more_than_two_gib(hip, tokens, experts, top_k, hidden, inter):
+    """Hidden activations, and activations reached through the token map, of more than 2 GiB; the last tokens, which lie beyond it."""
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(tokens)
+    host, dev = _block(rng, experts, hidden, inter)
+    x = np.tile(make_x(rng, 600, hidden), (-(-tokens // 600), 1))[:tokens]
+    assert max(x.nbytes, tokens * top_k * inter * 2) > 2 << 30
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    out = ops.moe_forward(*dev, DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(logits), top_k).numpy()
+    rows = np.concatenate([np.arange(20), rng.integers(0, tokens, 20), np.arange(tokens - 20, tokens)])
+    idx, w, _, _ = model.topk_route(logits[rows], top_k)
+    assert_close(out[rows], model.moe_forward(x[rows], idx, w, *host, 64, top_k), f"T={tokens} D={hidden} I={inter}")
+
+
+def test_routed_block_over_activations_off_16_bytes(hip):
+    """bf16 and f32 activations are cast, so their alignment plays no part: the bits of the aligned call."""
+    import ctypes
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import BF16, DeviceBuffer
+    rng = np.random.default_rng(4)
+    _, dev = _block(rng, 4, 512, 512)
+    logits = DeviceBuffer.from_numpy(rng.standard_normal((200, 4)).astype(np.float32))
+    for dtype in ("bf16", "f32"):
+        x = make_x(rng, 200, 512, dtype)
+        kind = BF16 if dtype == "bf16" else None
+        want = ops.moe_forward(*dev, DeviceBuffer.from_numpy(x, kind), logits, 2).numpy()
+        off = DeviceBuffer.from_numpy(np.concatenate([x.reshape(-1)[:1], x.reshape(-1)]), kind)
+        xa, la, out = off.array((200, 512), 1), logits.array(), DeviceBuffer((200, 512), hip.F16)
+        hip.check(hip.lib().rmlx_hip_moe_forward(*(q.handle for q in dev), ctypes.byref(xa), ctypes.byref(la), 2, None, out.ptr, out.nbytes, None))
+        assert np.array_equal(out.numpy().view(np.uint16), want.view(np.uint16)), dtype
+
+
+def test_more_experts_than_the_grouping_kernel_sorts(hip):
+    """Portable dimensions run without grouping, whatever the number of experts."""
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(6)
+    host, dev = _block(rng, 1100, 64, 64)
+    x = make_x(rng, 3000, 64)
+    idx = rng.integers(0, 1100, 3000).astype(np.uint32)
+    w = rng.uniform(0.2, 1.0, 3000).astype(np.float32)
+    out = ops.moe_forward_grouped(*dev, DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(idx), DeviceBuffer.from_numpy(w), 1).numpy()
+    assert_close(out[::17], model.moe_forward(x[::17], idx[::17], w[::17], *host, 64, 1))
