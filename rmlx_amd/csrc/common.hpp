@@ -263,8 +263,8 @@ int32_t launch_gemm_repack(const uint32_t* w, uint32_t N, uint32_t K, uint32_t b
 // 32 x 64 tiles with K split four ways inside the workgroup (qmm_k4.hip): 4-bit weights, group size 64, K % 2048 == 0
 bool qmm_k4_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 int32_t launch_qmm_k4(const QmmArgs& a, uint32_t group_size, hipStream_t s);
-// Grouped form of the same GEMM for the expert projections of batches with many rows per expert: every
-// row tile (kGroupedTileRows rows of one expert) takes its expert and rows from a device table of
+// Grouped form of the register-weights GEMM for the expert projections of batches with some rows per expert: every
+// row tile (up to kGroupedTileRows rows of one expert) takes its expert and rows from a device table of
 // (expert, first row position, row count) triples (bit 31 of the count: write zeros instead of computing;
 // not for a pair); `n_tiles_dev` holds the table's length.  With a second
 // weight (w1 / s1 / b1: the up projection) the store writes silu(x Wg^T) * (x Wu^T).
@@ -283,7 +283,7 @@ struct GroupedQmmArgs {
   int exact;                 // tile GEMMs: see QmmArgs
   const uint32_t* tile_tab; const uint32_t* n_tiles_dev;
   uint32_t max_tiles;        // row tiles the grid covers (>= *n_tiles_dev)
-  uint32_t tile_rows;        // rows per tile the table was built for: 32 or kGroupedTileRows
+  uint32_t tile_rows;        // rows per tile the table was built for: 16, 32 or (one weight) kGroupedTileRows; tile GEMMs: 32, 64, 128 or 256
 };
 bool qmm_rw_grouped_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 int32_t launch_qmm_rw_grouped(const GroupedQmmArgs& a, hipStream_t s);
@@ -301,9 +301,6 @@ bool qmm_tile_maps_rows(uint32_t x_rows, uint32_t K);
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
 // The same over row tiles of at most 32 rows, for few rows per expert (qmm_slice.hip)
 int32_t launch_qmm_slice_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
-// The LDS-staged GEMM over the same kind of table (tile_rows == 64, one weight, f16 output; shapes: qmm_supported)
-size_t qmm_grouped_workspace_bytes(uint32_t max_tiles, uint32_t K, uint32_t tile_rows = 64);
-int32_t launch_qmm_grouped(const GroupedQmmArgs& a, void* workspace, hipStream_t s);
 
 // MoE helpers
 int32_t launch_topk_route(const float* logits, const float* bias, uint32_t T, uint32_t E, uint32_t K,
@@ -337,8 +334,6 @@ int32_t launch_identity_positions(uint32_t* tok, uint32_t* inv, uint32_t n, uint
 // out[t,:] = sum_k w[t*K+k] * y[inv[t*K+k],:]  (y f32 rows at sorted positions)
 int32_t launch_moe_combine(const float* y, const uint32_t* inv, const float* weights, uint32_t T,
                            uint32_t top_k, uint32_t D, __half* out, hipStream_t s);
-int32_t launch_moe_combine_f16(const __half* y, const uint32_t* inv, const float* weights, uint32_t T, uint32_t top_k,
-                               uint32_t D, __half* out, hipStream_t s);
 // The same over f16 rows in assignment order (row t * top_k + k is pick k of token t); idx: the assignments' experts
 // (outside [0, E): skipped)
 int32_t launch_moe_combine_rows_f16(const __half* y, const uint32_t* idx, const float* weights, uint32_t T, uint32_t top_k,

@@ -686,10 +686,11 @@ int32_t launch_qmm_rw_grouped(const GroupedQmmArgs& a, hipStream_t s) {
   if ((uint64_t)p.tiles_m * p.tiles_n > 0x7FFFFFFFull) return fail(RMLX_INVALID_SHAPE, "grouped qmm: grid too large");
   if (a.tile_rows != 16 && a.tile_rows != 32 && a.tile_rows != kGroupedTileRows)
     return fail(RMLX_RUNTIME_ERROR, "grouped qmm: row tiles of %u rows", a.tile_rows);
+  if (dual && a.tile_rows == kGroupedTileRows) return fail(RMLX_RUNTIME_ERROR, "grouped qmm: a pair takes row tiles of 16 or 32 rows");
   const dim3 grid(p.tiles_m * p.tiles_n), block(64 * nw);
   const bool tail = a.K % (kBlockK * kUnroll) != 0;
 #define RWG_FORMS(MFV, NWV, BITSV, GSV, TAILV)                                                                              \
-  if (dual) hipLaunchKernelGGL((qmm_rw_grouped_kernel<MFV, 2, BITSV, NWV, true, GSV, TAILV>), grid, block, 0, s, p);          \
+  if (MFV < 4 && dual) hipLaunchKernelGGL((qmm_rw_grouped_kernel<(MFV < 4 ? MFV : 2), 2, BITSV, NWV, true, GSV, TAILV>), grid, block, 0, s, p);          \
   else if (wide) hipLaunchKernelGGL((qmm_rw_grouped_kernel<MFV, 2, BITSV, NWV, false, GSV, TAILV>), grid, block, 0, s, p);    \
   else hipLaunchKernelGGL((qmm_rw_grouped_kernel<MFV, 1, BITSV, NWV, false, GSV, TAILV>), grid, block, 0, s, p);
 #define RWG_LAUNCH(MFV, NWV, BITSV, GSV)                                         \
