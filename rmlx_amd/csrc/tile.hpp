@@ -41,19 +41,19 @@ constexpr uint32_t kOutside = 0xC0000000u;  // an offset past every buffer (at m
 
 // 16 (4) bytes per lane from buffer r at byte offset off straight into LDS at lds + 16 (4) * lane
 __device__ __forceinline__ void dma16(uint32_t lds, uint32_t off, u4 r) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(r) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(r) : "memory", "m0");
 }
 // the same to base + at and from a uniform byte offset on top
 template <uint32_t AT>
 __device__ __forceinline__ void dma16_at(uint32_t base, uint32_t off, u4 r, uint32_t more) {
   asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(base), "v"(off), "s"(r), "s"(more), "n"(AT)
-               : "memory", "scc");
+               : "memory", "scc", "m0");
 }
 // the same where `cond` (uniform) is not zero; the branch stays inside, so that the loop body remains one block for the scheduler
 __device__ __forceinline__ void dma16_if(uint32_t cond, uint32_t lds, uint32_t off, u4 r) {
   asm volatile(
       "s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 .Ldma_skip_%=\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n"
-      ".Ldma_skip_%=:" ::"s"(lds), "v"(off), "s"(r), "s"(cond) : "memory", "scc");
+      ".Ldma_skip_%=:" ::"s"(lds), "v"(off), "s"(r), "s"(cond) : "memory", "scc", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_dma_and_barrier() {
