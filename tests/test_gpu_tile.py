@@ -57,9 +57,12 @@ def test_large_tile_gemm_plans_and_epilogues(hip, m, n, k, bits):
 
 @pytest.mark.parametrize("bits,gs", [(4, 64), (4, 32), (8, 64), (4, 128)])
 @pytest.mark.parametrize("tokens,experts,top_k,hidden,inter,fused", [(600, 4, 2, 1088, 544, True), (150, 6, 3, 1024, 1056, False), (1100, 3, 1, 1280, 1024, True),
-                                                                      (30, 8, 2, 1088, 544, True), (40, 5, 2, 1024, 1056, False)])
+                                                                      (30, 8, 2, 1088, 544, True), (40, 5, 2, 1024, 1056, False),
+                                                                      (80, 4, 2, 1088, 544, True), (80, 4, 2, 1280, 1024, False),
+                                                                      (400, 4, 2, 1280, 1024, True), (900, 3, 2, 1088, 544, False)])
 def test_routed_block_on_large_tiles(hip, bits, gs, tokens, experts, top_k, hidden, inter, fused):
-    """Row tiles of 32, 64, 128 and 256 rows of one expert, dimensions that are no whole tiles, gate / up stacked and apart; the packed
+    """Row tiles of 32 (8 and 16 rows per expert), 64 (40; 128 at group size 32), 128 (75, 300 and 366) and 256 rows (200 and 600) of one
+    expert, reached through the token map; weights in two products (1088 x 544) and rounded (1280 x 1024); dimensions that are no whole tiles, gate / up stacked and apart; the packed
     outputs of ExpertGroup over the same experts, an item of one row and an empty one among them."""
     from rmlx_amd import ops
     from rmlx_amd.runtime import DeviceBuffer
@@ -89,7 +92,23 @@ def test_routed_block_on_large_tiles(hip, bits, gs, tokens, experts, top_k, hidd
 
 
 @pytest.mark.parametrize("batch,rows,n,k,gs", [(3, 70, 130, 1056, 32), (5, 9, 129, 1088, 64), (2, 300, 260, 1024, 128), (40, 3, 72, 640, 64)])
+def test_gather_on_small_tiles(hip, batch, rows, n, k, gs):
+    """Few rows: tiles of 32 of one entry, and the single-row kernel."""
+    _gather(batch, rows, n, k, gs)
+
+
+# rows per entry -> row tiles of 64 (128 at group size 32), 128, 256 and again 128 rows, in equal shares; N in whole columns of a tile (K in whole
+# slabs: the grouped GEMM's shapes) and off them
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("batch,rows,n,k", [(45, 50, 448, 640), (45, 64, 450, 640), (45, 33, 512, 1024), (20, 100, 448, 640), (20, 128, 577, 640),
+                                            (14, 200, 448, 640), (14, 256, 512, 1024), (8, 300, 514, 640), (5, 513, 512, 640)])
 def test_gather_on_large_tiles(hip, batch, rows, n, k, gs):
+    # (a third condition keeps small launches on tiles of 32 rows)
+    assert batch * (-(-rows // 32)) * (-(-n // 64)) > 2 * hip.device_info()["compute_units"] and rows > 32
+    _gather(batch, rows, n, k, gs)
+
+
+def _gather(batch, rows, n, k, gs):
     from rmlx_amd import ops
     from rmlx_amd.runtime import DeviceBuffer
     rng = np.random.default_rng(batch + rows + n + k)
