@@ -514,7 +514,7 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
        {2, 2, 8, 1, 5.17, {{0.061, 0.452}}, 2.30, 0.00, 256},
        {4, 1, 4, 1, 4.56, {{0.032, 1.080}}, 3.39, 0.00, 256},
        {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128}}};
-  constexpr double kExactStep = 1.6;  // two products: 8 to 2000 rows 1.57 to 1.7 x, 8-bit up to 64 rows 1.35
+  constexpr double kExactStep = 1.5;  // two products: 8 to 64 rows 1.35 to 1.45 x, 300 to 2000 rows 1.55 to 1.65
   const double cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
   const uint32_t rounds = (K + 127) / 128;
   TilePlan best{4, 2, 1, 1};

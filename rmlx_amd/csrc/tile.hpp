@@ -118,13 +118,17 @@ __device__ __forceinline__ void tile_epilogue(const TileParams& p, uint64_t o, u
 // The operand of a k step: weights rounded to f16 (lo unused), or, EXACT, w = scale * q + bias rounded once to f32 and cut into hi + lo
 // of 11 bits each, multiplied one after the other (hi towards zero, so that both have one sign; 21 to 22 bits of the weight are kept, of
 // weights below 2^-4 the bits down to 2^-24).  Costs 16 vector instructions a word and a product per fragment on top:
-// 64 rows, 33001 x 2880 50.5 against 35.9 us, 2000 x 20001 x 4096 567 against 341 us; error against 64 bits 2.07e-4 of the result, that of
+// 64 rows, 33001 x 2880 47.4 against 35.8 us, 2000 x 20001 x 4096 566 against 341 us; error against 64 bits 2.07e-4 of the result, that of
 // rounding it, against 2.75e-4 (E = 16, top-2 experts: 2.2e-4 against 4.4e-4).
 struct Weights { h8 hi, lo; };
 __device__ __forceinline__ void split_pair(float w0, float w1, h2* hi, h2* lo) {
   const h2 h = __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(w0, w1));
+  // (-1 from a register that the compiler does not know: w - hi is then one instruction of mixed precision a value, not a conversion, a
+  // subtraction and a half)
+  float minus;
+  asm("s_mov_b32 %0, -1.0" : "=s"(minus));
   *hi = h;
-  *lo = (h2){(_Float16)__builtin_fmaf((float)h[0], -1.0f, w0), (_Float16)__builtin_fmaf((float)h[1], -1.0f, w1)};
+  *lo = (h2){(_Float16)__builtin_fmaf((float)h[0], minus, w0), (_Float16)__builtin_fmaf((float)h[1], minus, w1)};
 }
 __device__ __forceinline__ Weights split_q4(uint32_t w, float s, float b) {
   const uint32_t even = w & 0x0F0F0F0Fu, odd = (w >> 4) & 0x0F0F0F0Fu;

@@ -41,11 +41,37 @@ def test_linear_calls_with_exact_weights(hip, m, n, k, bits, gs, dtype):
 @pytest.mark.parametrize("bits,gs", [(4, 64), (4, 32), (4, 128), (8, 64), (8, 32), (8, 128)])
 @pytest.mark.parametrize("m,n,groups", [(1, 515, 8), (31, 127, 9), (33, 129, 21), (65, 300, 17), (130, 257, 11), (300, 1027, 8), (600, 70, 45), (40, 9, 1)])
 def test_tile_gemm_with_exact_weights(hip, bits, gs, m, n, groups):
-    """Every tile size and k split of the two-product form, remainders in each dimension."""
+    """Remainders in each dimension."""
     from rmlx_amd import runtime as rt
     out, ref = _linear(m, n, groups * gs, bits, gs, kernel=rt.KERNEL_QMM_TILE_EXACT)
     assert_close(out, ref)
     assert _ratio(out, ref) < 1.05
+
+
+# every tile, number of wave groups along k and kind of k split that the plans hold, at the smallest sizes that take them
+@pytest.mark.parametrize("m,n,k,bits", [(1, 54, 256, 4), (1, 1454, 8448, 4), (69, 5723, 512, 4), (48, 2739, 6848, 4), (36, 8704, 384, 4), (1, 55, 6080, 4),
+                                        (34, 9398, 320, 4), (1, 55, 2048, 4), (38, 8787, 256, 4), (1, 56, 4096, 4), (66, 11423, 832, 4), (37, 2860, 6720, 4),
+                                        (141, 11085, 320, 4), (141, 11859, 448, 4), (68, 6039, 6784, 4), (531, 7694, 256, 4), (1500, 9001, 320, 4),
+                                        (1, 59, 4224, 8), (68, 5815, 320, 8), (69, 1134, 8256, 8), (36, 8193, 320, 8), (1, 55, 4992, 8), (33, 9645, 320, 8),
+                                        (1, 54, 2624, 8), (1, 6954, 256, 8), (1, 55, 4032, 8), (73, 8449, 576, 8), (33, 4362, 4096, 8), (194, 8507, 320, 8),
+                                        (71, 2617, 3968, 8), (131, 11332, 256, 8), (75, 6171, 6016, 8), (1096, 3618, 256, 8), (649, 11094, 320, 8)])
+@pytest.mark.parametrize("exact", [True, False])
+def test_tile_gemm_plans(hip, m, n, k, bits, exact):
+    from rmlx_amd import ops, runtime as rt
+    from rmlx_amd.runtime import DeviceBuffer
+    gs = 64
+    rng = np.random.default_rng(m + n + k + bits)
+    w = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k)
+    out = ops.affine_quantized_matmul_batched(DeviceBuffer.from_numpy(x), ops.QuantizedWeight.from_numpy(*w, gs, bits),
+                                              kernel=rt.KERNEL_QMM_TILE_EXACT if exact else rt.KERNEL_QMM_TILE).numpy()
+    rows = np.unique(np.concatenate([np.arange(0, m, 19), [m - 1]]))
+    cols = np.unique(np.concatenate([np.arange(0, n, 7), [n - 1]]))
+    ref = model.qmm(x[rows].astype(np.float64), *(a[cols] for a in w), gs, bits)
+    got = out[rows][:, cols]
+    assert_close(got, ref)
+    if exact and got.size > 300:
+        assert _ratio(got, ref) < 1.05
 
 
 @pytest.mark.parametrize("gs", [64, 128])
