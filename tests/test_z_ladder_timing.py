@@ -21,6 +21,16 @@ LADDER_SHAPES = [(4096, 14336, 4, (3, 9, 16)), (2048, 16384, 4, (5, 16)), (4096,
 
 @pytest.mark.parametrize("n,k,bits,ms", LADDER_SHAPES)
 def test_ladder_picks_within_15_percent_of_the_fastest_family(hip, n, k, bits, ms):
+    _ladder(n, k, bits, ms)
+
+
+@pytest.mark.parametrize("n,k,bits,ms", [(4096, 4096, 8, (128, 512)), (28672, 4096, 8, (48, 256)), (12288, 4096, 4, (128, 256, 512))])
+def test_ladder_with_the_tile_contiguous_copy(hip, n, k, bits, ms):
+    """The same with a second copy of the weights, which only the K-split GEMMs read."""
+    _ladder(n, k, bits, ms, copy=True)
+
+
+def _ladder(n, k, bits, ms, copy=False):
     """The automatic dispatch on shapes its crossovers were not tuned on: against every forced kernel family that takes the
     shape and is as exact as the pick (one that multiplies the weights exactly is not compared with those that round them to
     f16), the ladder's pick is within 15 % of the fastest (trains of launches between two events, weight sets cycled), and
@@ -32,6 +42,8 @@ def test_ladder_picks_within_15_percent_of_the_fastest_family(hip, n, k, bits, m
     n_sets = max(2, min(6, (400 << 20) // (n * k * bits // 8)))
     qws = [ops.QuantizedWeight.from_numpy(np.roll(base[0], i, 0), np.roll(base[1], i, 0), np.roll(base[2], i, 0), 64, bits)
            for i in range(n_sets)]
+    if copy:
+        assert all(q.use_gemm_layout() for q in qws)
     stream, e0, e1 = rt.Stream(), rt.Event(), rt.Event()
     families = {"auto": rt.KERNEL_AUTO, "qmv": rt.KERNEL_QMV_ROWS, "single": rt.KERNEL_QMV, "qmm": rt.KERNEL_QMM, "k2": rt.KERNEL_QMM_K2,
                 "lds": rt.KERNEL_QMM_LDS,
