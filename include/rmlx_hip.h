@@ -184,7 +184,7 @@ int32_t rmlx_hip_qmm_select(const rmlx_qweight* qw, const rmlx_array* x, int32_t
  * out = silu(gate_result) * (x @ dequant(W)^T).  residual / gate_result: [M, out_features],
  * Float16 or Float32 (the reference's are Float32), same validation message as the reference
  * ("... shape must be [M, N]"); out is f16 and may be an f16 operand itself (the same address; no other overlap).  Evaluated in f32 on the accumulator with one rounding
- * in the GEMM kernel; after the GEMV / portable kernels as a separate elementwise pass.  Unlike the
+ * in the GEMM kernels (but the LDS-staged one) and the single-row GEMV; after the other kernels as a separate elementwise pass.  Unlike the
  * reference (Q4, M > 32 only) every shape the batched entry point takes is accepted. */
 int32_t rmlx_hip_qmm_add_residual(const rmlx_qweight* qw, const rmlx_array* x, const rmlx_array* residual,
                                   void* out_f16_dev, size_t out_bytes, rmlx_stream stream);
@@ -313,8 +313,8 @@ int32_t rmlx_hip_moe_forward_grouped(const rmlx_qweight* gate, const rmlx_qweigh
 
 /* Kernel choice of the expert projections (ExpertGroup and the MoeLayer entry points): batches with at least
  * `min_rows` rows per expert on average (rows / num_experts; for ExpertGroup rows / n_items) multiply with a
- * grouped MFMA GEMM -- the large-tile one (64, 128 or 256 rows of one expert, every 4- / 8-bit shape) where it is ahead
- * (with the default threshold also below it), else row tiles of 16, 32 or 64 rows of one expert, weights dequantised in registers; 4- / 8-bit,
+ * grouped MFMA GEMM -- the tile GEMM (32, 64, 128 or 256 rows of one expert, every 4- / 8-bit shape) where it is ahead
+ * (with the default threshold also below it, then with exact weights: kernel 13 of rmlx_hip_qmm_select), else row tiles of 16 or 32 rows of one expert, weights dequantised in registers; 4- / 8-bit,
  * group sizes 32 / 64 / 128 (one for the three projections), hidden and intermediate dimensions in multiples of
  * 512 -- smaller ones with the streaming GEMV, which reads an expert's weights once per 8 rows (8-bit experts
  * switch at an eighth of `min_rows`, at least 1).  0 = never the GEMM; the default (10) is the measured crossover.

@@ -13,7 +13,8 @@
 // LDS (24.3) were no faster; rings of less than two stages of distance are (latency of about 1 us per stage).
 // Measured, 4096 x 4096, 4-bit, weights from HBM, tiles of qmm_tile.hip / these: 32 rows 18.8 / 11.2 us, 64 rows 20.7 / 11.2, 256
 // rows 21.1 / 14.8; 512 rows 26.9 / 23.1; 13 rows, 14336 x 4096, 8-bit 26.0 / 17.1; 128 rows, 12288 x 4096 25.6 / 21.6, 8-bit
-// 29.2 / 27.9.  On 530 shapes of 9 to 1200 rows the best of both is 7 to 18 % ahead of the best before.
+// 29.2 / 27.9.  On 530 shapes of 9 to 1200 rows the best of both is 7 to 18 % ahead of those tiles alone (against the older GEMMs: see the
+// dispatch; 32 rows, 4096 x 4096 stay on the register-weights GEMM at 9.1).
 #include <type_traits>
 
 #include "tile.hpp"

@@ -15,10 +15,11 @@
 // us with two workgroups and a second kernel) and over workgroups.
 //
 // What bounds it: power.  At 8192^3 with random data the chip runs at 1.5 GHz instead of 2.4 (a zero-filled launch is 1.5 x as
-// fast in the same number of cycles), so time follows the energy of a step, not its cycles: 64 unpacking instructions per wave
+// fast in the same number of cycles; at 3001 x 14336 x 4096 1.6 GHz, with the matrix unit busy for 70 % of those cycles), so time follows the energy of a step, not its cycles: 64 unpacking instructions per wave
 // and step cost 15 % and the operand reads 10 % of the launch.  That is why the large tile gives each wave all 256 rows of a few
 // weight rows (2 x 4 waves of 128 x 64, half the LDS reads but every weight unpacked twice: 1143 against 1217 TFLOP/s).
-// 8192^3: 903 us (1217 TFLOP/s; the library's f16 product 1294); 4096^3 122 us against 158 us on the 128 x 128 K-split tiles;
+// 8192^3: 903 us (1217 TFLOP/s; the library's f16 product of normal values 1515 with its second operand laid out as the weights are here, 1304 with it
+// row-major, 1805 on zeros); 4096^3 122 us against 158 us on the 128 x 128 K-split tiles;
 // 3001 x 14336 x 4096 bf16 416 -> 332 us.  Small tiles are bound by the unpacking of a lone wave per SIMD (7.6 cycles per dependent
 // vector instruction: 0.33 of the 0.39 us of a 64-row step); most sizes that would use them are on qmm_slice.hip.
 #include <cmath>
