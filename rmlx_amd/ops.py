@@ -110,7 +110,7 @@ def affine_quantized_matmul_batched(x, qw, stream=None, kernel=rt.KERNEL_AUTO, o
     if out is None:
         out = DeviceBuffer((x.shape[0] if len(x.shape) == 2 else 0, qw.out_features), F16)
     a = x.view()
-    status = _entry("rmlx_hip_qmm_select")(qw.handle, a.address, kernel, out.ptr, out.nbytes, None if stream is None else stream.handle)
+    status = _entry("rmlx_hip_qmm_select")(qw.handle, a[0], kernel, out.ptr, out.nbytes, None if stream is None else stream.handle)
     if status:
         rt.check(status)
     return out
@@ -200,8 +200,8 @@ def gather_qmm(x, w_packed_buf, scales_buf, biases_buf, indices, batch, m_per_ba
     if out is None:
         out = DeviceBuffer((batch, m_per_batch, n), F16)
     xa, ia = x.view(), indices.view()
-    rt.check(_entry("rmlx_hip_gather_qmm_select")(xa.address, w_packed_buf.ptr, w_packed_buf.nbytes, scales_buf.ptr, scales_buf.nbytes,
-                                                  biases_buf.ptr, biases_buf.nbytes, ia.address, batch, m_per_batch, n, k,
+    rt.check(_entry("rmlx_hip_gather_qmm_select")(xa[0], w_packed_buf.ptr, w_packed_buf.nbytes, scales_buf.ptr, scales_buf.nbytes,
+                                                  biases_buf.ptr, biases_buf.nbytes, ia[0], batch, m_per_batch, n, k,
                                                   n_experts, group_size, kernel, out.ptr, out.nbytes, _h(stream)))
     return out
 
@@ -321,7 +321,7 @@ def moe_forward_grouped(gate, up, down, x, expert_indices, expert_weights, top_k
     if out is None:
         out = DeviceBuffer((x.shape[0], x.shape[1]), F16)
     xa = x.view()
-    rt.check(_entry("rmlx_hip_moe_forward_grouped")(gate.handle, up.handle if up is not None else None, down.handle, xa.address,
+    rt.check(_entry("rmlx_hip_moe_forward_grouped")(gate.handle, up.handle if up is not None else None, down.handle, xa[0],
                                                     expert_indices.ptr, expert_weights.ptr, top_k, out.ptr, out.nbytes, _h(stream)))
     return out
 
@@ -334,6 +334,6 @@ def moe_forward(gate, up, down, x, gate_logits, top_k, expert_bias=None, stream=
     fn = _entry("rmlx_hip_moe_forward_noalloc" if noalloc else "rmlx_hip_moe_forward")
     xa, la = x.view(), gate_logits.view()
     ba = expert_bias.view() if expert_bias is not None else None
-    rt.check(fn(gate.handle, up.handle if up is not None else None, down.handle, xa.address, la.address, top_k,
-                ba.address if ba is not None else None, out.ptr, out.nbytes, _h(stream)))
+    rt.check(fn(gate.handle, up.handle if up is not None else None, down.handle, xa[0], la[0], top_k,
+                ba[0] if ba is not None else None, out.ptr, out.nbytes, _h(stream)))
     return out

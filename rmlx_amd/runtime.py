@@ -221,15 +221,13 @@ class DeviceBuffer:
         return out
 
     def view(self):
-        """This buffer's rmlx_array (what `array()` builds) with its `address`, kept while pointer, shape and type stay the same.  A
-        call holds the object until it returns: another thread may build and keep a new one meanwhile."""
-        key = (self.ptr, self.shape, self.dtype)
-        kept = self._view
-        if kept is None or kept[0] != key:
+        """(address, rmlx_array) of this buffer's view (what `array()` builds), kept while pointer, shape and type stay the same.  A
+        call holds the pair until it returns: another thread may build and keep a new one meanwhile."""
+        kept, key = self._view, (self.ptr, self.shape, self.dtype)
+        if kept is None or kept[2] != key:
             a = self.array()
-            a.address = ctypes.addressof(a)
-            kept = self._view = (key, a)
-        return kept[1]
+            kept = self._view = (ctypes.addressof(a), a, key)
+        return kept
 
     def array(self, shape=None, offset_elems=0):
         """The rmlx_array view handed to the C ABI."""
