@@ -385,7 +385,7 @@ __global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (M
   load_activations<BITS, MR, NORM>(img, p.x, p.M, mrow0, p.norm_w, p.inv_rms, tid, xv);
   // ... the epilogue operand of the output this lane will write (lane r * MR + m) ...
   const uint32_t out_m = mrow0 + lane % MR, out_n = row0 + lane / MR;
-  const bool writes = lane < R * MR && out_m < p.M && out_n >= blk0;
+  const bool writes = lane < R * MR && out_m < p.M;
   float epi_val = 0.f;
   if (p.epi_kind != EPI_NONE && writes) {
     const uint64_t oi = (uint64_t)out_m * p.N + out_n;
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (M
       for (int q = 1; q < KP; ++q) mine += kp == 0 ? part[(wave + q) * MR + lane] : 0.f;
     }
   }
-  if (writes && kp == 0) {  // residual add / SwiGLU gate in f32, one rounding (quantized.rs:3206-3246)
+  if (writes && kp == 0 && out_n >= blk0) {  // residual add / SwiGLU gate in f32, one rounding (quantized.rs:3206-3246)
     if (p.epi_kind == EPI_RESIDUAL) mine += epi_val;
     else if (p.epi_kind == EPI_SWIGLU) mine = epi_val / (1.0f + __expf(-epi_val)) * mine;
     if (GATHER && gather_zeros) mine = 0.f;
