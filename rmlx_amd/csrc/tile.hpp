@@ -117,7 +117,7 @@ __device__ __forceinline__ void tile_epilogue(const TileParams& p, uint64_t o, u
 
 // The operand of a k step: weights rounded to f16 (lo unused), or, EXACT, w = scale * q + bias rounded once to f32 and cut into hi + lo
 // of 11 bits each, multiplied one after the other (hi towards zero, so that both have one sign; 21 to 22 bits of the weight are kept, of
-// weights below 2^-4 the bits down to 2^-24).  Costs 16 vector instructions a word and a product per fragment on top:
+// weights below 2^-4 the bits down to 2^-24; beyond 131008 the low part overflows).  Costs 16 vector instructions a word and a product per fragment on top:
 // 64 rows, 33001 x 2880 47.4 against 35.8 us, 2000 x 20001 x 4096 566 against 341 us; error against 64 bits 2.07e-4 of the result, that of
 // rounding it, against 2.75e-4 (E = 16, top-2 experts: 2.2e-4 against 4.4e-4).
 struct Weights { h8 hi, lo; };
