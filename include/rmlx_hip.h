@@ -171,8 +171,10 @@ int32_t rmlx_hip_affine_quantized_matmul_batched(const rmlx_qweight* qw, const r
  * would need more than one round of its 32 x 64 tiles; K <= 4096), 11 = the MFMA GEMM with 32 x 64 tiles and K split four
  * ways inside the workgroup (4-bit weights at group size 64, N % 64 == 0, K % 2048 == 0), 12 = the large-tile MFMA GEMM
  * (tiles of up to 256 x 256; 4- / 8-bit weights, every group size, any N and K), 13 = the same with exact weights, in two products,
- * 14 = the multi-row streaming GEMV over 4-bit matrices that kernel 6 does not take (any N, any K of whole groups of 64 or 128).
- * Precision: kernels 1, 3, 6, 13 and 14 multiply with scale * q + bias as it is (integer dot products scaled in f32, f32 weights, or two f16
+ * 14 = the multi-row streaming GEMV over 4-bit matrices that kernel 6 does not take (any N, any K of whole groups of 64 or 128),
+ * 15 = the slot-streaming GEMV (4- and 8-bit, every group size, any N from a tile on, any K of whole groups from 512 to what the
+ * registers of a workgroup hold of 16 activation rows: 8192 at 4 bits, group size 32 and 8-bit weights: 4096).
+ * Precision: kernels 1, 3, 6, 13, 14 and 15 multiply with scale * q + bias as it is (integer dot products scaled in f32, f32 weights, or two f16
  * parts of 21 bits together); the GEMMs 2, 5 and 7 to 12 round every weight to f16, which adds 1.8e-4 of the result to the 2.1e-4 of
  * rounding it.  The automatic choice rounds weights only where it has always run such a GEMM: 4- / 8-bit matrices in multiples of 64, at
  * row counts beyond the GEMVs'. */
@@ -338,7 +340,9 @@ int32_t rmlx_hip_qweight_set_gemm_layout(rmlx_qweight* qw, void* dst_dev, size_t
  * weight tile, chunks of 8 rows, 3 = a wave per tile, chunks of 16 rows, 4 = kernel 1 for the gate / up projection and
  * kernel 2 for the down projection (4-bit weights, group size 64; other weights keep kernel 1), 5 = as 4 with the gate / up
  * projection in two launches, the experts split by their row count: up to 8 rows on kernel 1, more on kernel 3, so every
- * expert is streamed once whatever the largest row count, 0 = the library's choice (4; 5 from 6 rows per expert on
+ * expert is streamed once whatever the largest row count, 6 = the slot-streaming kernel for the three projections, chunks of 16
+ * rows (4- and 8-bit weights, every group size; experts that it does not take keep the library's choice; the routed block only),
+ * 0 = the library's choice (6 for a few rows per expert where many weights are picked, else 4; 5 from 6 rows per expert on
  * average).  Kernel 3 streams an expert with 9 to 16 rows once instead of twice and is the fastest of the four from 7 rows
  * per expert on average - as long as no expert of the batch has more than 16 rows, so it is for callers whose router bounds
  * that.  Returns the previous value; the tests use it to check that the kernels agree.  (No counterpart in the reference, which has one kernel for this: gather_qmv_fast_f16_q4,

@@ -192,6 +192,10 @@ int32_t launch_qmv_q8(const uint32_t* w, const __half* s, const __half* b, const
                       int32_t x_bf16 = 0);  // 1: x holds bf16 bits, converted in registers
 // chunk-table mode for the expert projections (expert strides in u32 words / halves as for the 4-bit kernel)
 int32_t launch_qmv_q8_tab(const QmvArgs& a, hipStream_t stream);
+// Streaming GEMV over contiguous weight slots (qmv_ring.hip): up to 16 rows per chunk (M rows in chunks of 16 without a table), x of any
+// float type, 4- and 8-bit weights, every group size; x_rows: rows of x (chunks without a row map index its rows themselves)
+bool qmv_ring_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
+int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32_t x_rows, hipStream_t s);
 // Single-row GEMV (qmv_m1.hip): 4- or 8-bit weights, group size 32 / 64 / 128, f16 activations; M rows are
 // passes of up to four rows over the weights (grid.y); the store epilogue (EPI_*) is fused.
 bool qmv_m1_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);

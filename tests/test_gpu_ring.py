@@ -1,0 +1,96 @@
+"""The slot-streaming GEMV (qmv_ring.hip) at the edges of its tiles, slots and splits, against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import model
+from tests.helpers import assert_close, make_weight, make_x, x_as_f64
+from tests.test_gpu_precision import _ratio
+
+pytestmark = pytest.mark.gpu
+
+
+# Every split of a row: one to eight parts of three and of four loads, the last one full, in part empty and (8-bit K = 2240, 4-bit K = 4608) all
+# but empty, rows in two slots; 16-byte pieces of a row in multiples of 16, 8, 4 and 2; groups of a row in multiples of 32, even and odd.
+@pytest.mark.parametrize("bits,gs,k", [(4, 64, 512), (4, 64, 704), (4, 64, 1024), (4, 64, 1088), (4, 64, 1536), (4, 64, 2048), (4, 64, 2880), (4, 64, 4032),
+                                       (4, 64, 4096), (4, 64, 4608), (4, 64, 8128), (4, 64, 8192), (4, 32, 544), (4, 32, 1024), (4, 32, 2080), (4, 32, 2880),
+                                       (4, 32, 4064), (4, 32, 4096), (4, 128, 512), (4, 128, 1408), (4, 128, 2944), (4, 128, 4096), (4, 128, 6144),
+                                       (8, 64, 512), (8, 64, 1088), (8, 64, 1408), (8, 64, 2048), (8, 64, 2240), (8, 64, 4096), (8, 32, 544), (8, 32, 1504),
+                                       (8, 32, 2016), (8, 32, 2880), (8, 32, 4096), (8, 128, 640), (8, 128, 2048), (8, 128, 2944), (8, 128, 4096)])
+# fewer weight rows than workgroups and a tile's worth for each of a few, a little over one and two tiles a workgroup, many tiles with a ragged end
+@pytest.mark.parametrize("m,n,dtype", [(1, 128, "f16"), (16, 257, "bf16"), (17, 4099, "f16"), (3, 8211, "f32"), (15, 28677, "bf16")])
+def test_matrix(hip, bits, gs, k, m, n, dtype):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k + bits + gs)
+    w = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    out = ops.affine_quantized_matmul_batched(xd, ops.QuantizedWeight.from_numpy(*w, gs, bits), kernel=rt.KERNEL_QMV_RING).numpy()
+    rows = np.unique(np.concatenate([np.arange(min(n, 300)), np.arange(0, n, 61), np.arange(max(0, n - 70), n)]))
+    x64 = x_as_f64(x, dtype)
+    ref = model.qmm(x64.astype(np.float16).astype(np.float64), *(a[rows] for a in w), gs, bits)
+    assert_close(out[:, rows], ref)
+    if out[:, rows].size > 500:
+        assert _ratio(out[:, rows], ref) < 1.05
+
+
+@pytest.mark.parametrize("bits,gs,hidden,inter", [(4, 64, 1024, 1088), (4, 64, 4608, 640), (4, 32, 1056, 576), (4, 128, 1408, 4096), (8, 64, 2240, 512), (8, 32, 544, 1504),
+                                                  (8, 128, 640, 2176)])
+@pytest.mark.parametrize("tokens,experts,fused,dtype", [(3, 5, True, "f16"), (40, 6, False, "bf16"), (90, 40, True, "f32")])
+def test_routed_block(hip, bits, gs, hidden, inter, tokens, experts, fused, dtype):
+    """Experts with no row, one chunk, a little over one and several; the entry point without allocations, which routes and groups up to 8
+    tokens in one launch, returns the same bits."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(tokens + hidden + inter + bits)
+    gate, up = (make_weight(rng, inter, hidden, bits, gs, (experts,)) for _ in range(2))
+    down = make_weight(rng, hidden, inter, bits, gs, (experts,))
+    d = ops.QuantizedWeight.from_numpy(*down, gs, bits)
+    if fused:
+        g, u = ops.QuantizedWeight.from_numpy(*(np.concatenate(p, axis=1) for p in zip(gate, up)), gs, bits), None
+    else:
+        g, u = (ops.QuantizedWeight.from_numpy(*w, gs, bits) for w in (gate, up))
+    x = make_x(rng, tokens, hidden, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    logits[:, 1] -= 20.0  # no token's pick
+    logits[:17, 2] += 20.0  # 17 rows, 16 of them in the first chunk
+    logits[:, 3] += 10.0  # (nearly) every token's
+    idx, w, counts, _ = model.topk_route(logits, 2)
+    g.set_expert_stream_kernel(6)
+    ld = rt.DeviceBuffer.from_numpy(logits)
+    out = ops.moe_forward(g, u, d, xd, ld, 2).numpy()
+    print(f"slot-streaming block Q{bits} gs={gs} {hidden}/{inter} rows per expert {counts.tolist()}", flush=True)
+    x64 = x_as_f64(x, dtype).astype(np.float16)
+    ref = model.moe_forward(x64, idx, w, gate, up, down, gs, 2, bits=bits)
+    assert_close(out, ref)
+    assert _ratio(out, ref) < 1.2  # (the hidden activations are rounded to f16: about 1.08)
+    same = ops.moe_forward(g, u, d, xd, ld, 2, noalloc=True).numpy()
+    assert np.array_equal(same.view(np.uint16), out.view(np.uint16))
+
+
+@pytest.mark.parametrize("tokens,taken", [(18, False), (20, True), (40, True), (42, False)])
+def test_library_takes_it_for_a_few_rows_per_expert(hip, tokens, taken):
+    """Experts of 4M values on average 5 to 10 rows each; a threshold of the caller's for the grouped GEMM goes first."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(tokens)
+    experts, hidden = 8, 2048
+    one = [make_weight(rng, n, hidden, 4, 64, (1,)) for n in (2 * hidden, hidden)]
+    gate_up, down = (tuple(np.ascontiguousarray(np.broadcast_to(a, (experts,) + a.shape[1:])) for a in t) for t in one)
+    g, d = (ops.QuantizedWeight.from_numpy(*w, 64, 4) for w in (gate_up, down))
+    x = make_x(rng, tokens, hidden)
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    xd, ld = rt.DeviceBuffer.from_numpy(x), rt.DeviceBuffer.from_numpy(logits)
+
+    def run(kind, min_rows=None):
+        g.set_expert_stream_kernel(kind)
+        prev = g.set_expert_gemm_min_rows(min_rows) if min_rows is not None else None
+        out = ops.moe_forward(g, None, d, xd, ld, 2).numpy()
+        if prev is not None:
+            g.set_expert_gemm_min_rows(prev)
+        return out
+
+    auto, forced = run(0), run(6)
+    assert np.array_equal(auto.view(np.uint16), forced.view(np.uint16)) == taken
+    assert not np.array_equal(run(0, 2), forced)
+    idx, w, _, _ = model.topk_route(logits, 2)
+    gate, up = tuple(a[:, :hidden] for a in gate_up), tuple(a[:, hidden:] for a in gate_up)
+    assert_close(auto, model.moe_forward(x, idx, w, gate, up, down, 64, 2))
