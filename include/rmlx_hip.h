@@ -241,7 +241,8 @@ int32_t rmlx_hip_gather_qmm(const rmlx_array* x, const void* w_packed_dev, size_
  * from 512 on, the tile GEMM in its place where that is faster; other shapes: a few rows on the single-row GEMV, more on the tile GEMM;
  * the portable kernel for what neither takes), 1 = streaming GEMV (group size 64 / 128, N % 16 == 0,
  * K % 128 == 0), 2 = grouped MFMA GEMM,
- * 3 = portable kernel. */
+ * 3 = portable kernel, 4 = the slot-streaming GEMV (at most 256 entries of at most 16 rows, the matrices that kernel 15 of the matmul takes;
+ * entries of one expert share its pass over the weights; what 0 takes where that is the least to stream). */
 int32_t rmlx_hip_gather_qmm_select(const rmlx_array* x, const void* w_packed_dev, size_t w_bytes,
                                    const void* scales_dev, size_t scales_bytes,
                                    const void* biases_dev, size_t biases_bytes,

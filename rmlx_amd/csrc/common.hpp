@@ -196,6 +196,10 @@ int32_t launch_qmv_q8_tab(const QmvArgs& a, hipStream_t stream);
 // float type, 4- and 8-bit weights, every group size; x_rows: rows of x (chunks without a row map index its rows themselves)
 bool qmv_ring_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32_t x_rows, hipStream_t s);
+// gather_qmm on it (4-bit): entry i's `per` rows through expert picks[i] (outside [0, n_experts): zeros); entries of one expert share chunks
+bool qmv_ring_gather_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t entries, uint32_t per, uint32_t n_experts, int32_t x_dtype);
+int32_t launch_qmv_ring_gather(const QmvArgs& a, const uint32_t* picks, uint32_t entries, uint32_t per, uint32_t n_experts, int32_t x_dtype,
+                               hipStream_t s);
 // Single-row GEMV (qmv_m1.hip): 4- or 8-bit weights, group size 32 / 64 / 128, f16 activations; M rows are
 // passes of up to four rows over the weights (grid.y); the store epilogue (EPI_*) is fused.
 bool qmv_m1_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);

@@ -30,13 +30,17 @@ namespace {
 // Beside the arguments that the first loads need (separate ones: those arrive in scalar registers).
 struct RingParams {
   void* out;
-  uint32_t M, ld_out, x_rows, spr_inv;   // (2^20 / a row's groups of eight)
+  uint32_t ld_out, x_rows, spr_inv;   // (2^20 / a row's groups of eight)
   int32_t out_f32;
   const uint32_t* w1; const __half* s1; const __half* b1;
   const uint32_t* row_map; const uint32_t* chunk_tab; const uint32_t* n_chunks;
   uint64_t estride_w, estride_s;
+  uint32_t slack;  // weight rows that one more chunk costs a workgroup
+  const uint32_t* picks; uint32_t entries, per, per_inv, n_experts;  // GATHER; per_inv: 2^16 / per
 };
-enum { DENSE = 0, TABLE = 1, PAIR = 2 };  // rows of one matrix; of the expert that a chunk table names; of its gate and up matrices
+// rows of one matrix; of the expert that a chunk table names; of its gate and up matrices; of the experts that a list of entries picks
+enum { DENSE = 0, TABLE = 1, PAIR = 2, GATHER = 3 };
+constexpr uint32_t kMaxEntries = 256, kNoExpert = 0xFFFFFFFEu;
 // How the waves share a tile's k: `ks` parts, 2^nt_log2 tiles side by side, the tile of wave i in bits 8 + 3 i
 inline uint32_t ring_geometry(uint32_t ks, int32_t x_dtype) {
   uint32_t v = ks | (ks == 1 ? 3u : (ks == 2 ? 2u : (ks <= 4 ? 1u : 0u))) << 4 | (uint32_t)x_dtype << 6;
@@ -86,6 +90,11 @@ __device__ __forceinline__ void dma16_next(uint32_t off, u4 r) {
   asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 nt lds" ::"v"(off), "s"(r), "n"(AT) : "memory");
 }
 __device__ __forceinline__ void dma16_plain(uint32_t off, u4 r) { asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(r) : "memory"); }
+// the buffer from byte `by` on (scalar: the lanes' offsets stay as they are)
+__device__ __forceinline__ u4 later(u4 r, uint32_t by) {
+  const uint64_t a = ((uint64_t)r.y << 32 | r.x) + by;
+  return (u4){uni((uint32_t)a), uni((uint32_t)(a >> 32)), uni(r.z - by), r.w};
+}
 __device__ __forceinline__ void set_m0(uint32_t lds) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds) : "memory"); }
 template <int AT>
 __device__ __forceinline__ void load16(u4& d, uint32_t off, u4 r) {
@@ -124,7 +133,7 @@ struct Ring {
 
 template <int BITS, int GS, int U, int H, int MODE>
 __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t* w0, const __half* s0, const __half* b0, const void* x, uint32_t N,
-                                                                  uint32_t K, uint32_t geometry, uint32_t share, uint32_t over, uint32_t cpr_inv,
+                                                                  uint32_t K, uint32_t M, uint32_t geometry, uint32_t share, uint32_t over, uint32_t cpr_inv,
                                                                   RingParams p) {
   const uint32_t spr_inv = p.spr_inv;
   using C = Ring<BITS, GS, U, H>;
@@ -140,17 +149,98 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
   uint32_t lane = tid & 63;
   const uint32_t KS = geometry & 15, nt_log2 = H == 2 ? 0 : geometry >> 4 & 3, tw = geometry >> (8 + 3 * wave) & 7, kp = wave - tw * KS, NT = 1u << nt_log2;
   const int32_t x_dtype = geometry >> 6 & 3;
-  // an equal share of all (chunk, weight row) pairs for every workgroup
-  if (MODE != DENSE) {
-    const uint32_t all = uni(*p.n_chunks) * N;
-    share = all / gridDim.x;
-    over = all - share * gridDim.x;
+  // An equal share of all (chunk, weight row) pairs for every workgroup, or, where that is hardly more work for it, of one chunk (a second
+  // one starts over with empty rings and other activations: about 4 us, in which a CU streams 100 KB).
+  uint32_t pos = 0, end = 0;
+  auto take_share = [&](uint32_t chunks) {
+    const uint32_t all = chunks * N, each = all / gridDim.x, more = all - each * gridDim.x, b = blockIdx.x;
+    const uint32_t per = chunks == 0 ? 0 : gridDim.x / chunks, part = per == 0 ? 0 : N / per, rest = N - part * per;
+    if (per != 0 && part <= each + p.slack) {
+      const uint32_t c = b / per, i = b - c * per;
+      pos = c * N + i * part + (i < rest ? i : rest);
+      end = c < chunks ? pos + part + (i < rest ? 1 : 0) : pos;
+    } else {
+      pos = b * each + (b < more ? b : more);
+      end = pos + each + (b < more ? 1 : 0);
+    }
+    pos = uni(pos);
+    end = uni(end);
+  };
+  // GATHER: every workgroup groups the entries by expert itself (a launch of its own for that costs more: 3 us against about 1.5), a stable
+  // counting sort over at most 256 of them, all waves alike behind the ranks.  A chunk is 16 rows of one expert's entries one behind another;
+  // a workgroup's share lies in at most four of those (all fit in two times the workgroups): lane 16 s + i keeps row i of the s-th.
+  uint32_t seg_row = 0, seg_rows = 0, seg_expert = 0;
+  if constexpr (MODE == GATHER) {
+    uint32_t* const keys = reinterpret_cast<uint32_t*>(lds);  // in the place of the rings
+    uint32_t *const order = keys + kMaxEntries, *const run_chunks = order + kMaxEntries, *const run_rows = run_chunks + kMaxEntries;
+    uint32_t* const mine = run_rows + kMaxEntries + wave * 16;
+    if (tid < kMaxEntries) {
+      const uint32_t e = tid < p.entries ? p.picks[tid] : 0xFFFFFFFFu;
+      keys[tid] = tid < p.entries && e >= p.n_experts ? kNoExpert : e;
+      run_chunks[tid] = 0;
+    }
+    q4::lds_barrier();
+    if (tid < p.entries) {
+      const uint32_t e = keys[tid];
+      uint32_t below = 0, before = 0, same = 0;
+      for (uint32_t j = 0; j < p.entries; j += 4) {
+        const u4 v = *reinterpret_cast<const u4*>(keys + j);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+          below += v[i] < e ? 1u : 0u;
+          same += v[i] == e ? 1u : 0u;
+          before += v[i] == e && j + i < tid ? 1u : 0u;
+        }
+      }
+      order[below + before] = tid;
+      if (before == 0) {
+        run_chunks[below] = (same * p.per + 15) / 16;
+        run_rows[below] = same * p.per;
+      }
+    }
+    q4::lds_barrier();
+    const u4 v = *reinterpret_cast<const u4*>(run_chunks + lane * 4);
+    uint32_t inc = v.x + v.y + v.z + v.w;
+    const uint32_t own = inc;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t t = __shfl_up(inc, o, 64);
+      if ((int)lane >= o) inc += t;
+    }
+    take_share(uni(__builtin_amdgcn_readlane(inc, 63)));
+    const uint32_t c0 = pos / N;
+    if (lane < 16) mine[lane] = 0;
+    uint32_t base = inc - own;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+#pragma unroll
+      for (uint32_t sg = 0; sg < 4; ++sg) {
+        const uint32_t d = c0 + sg - base, q = lane * 4 + i;
+        if (c0 + sg >= base && d < v[i]) {
+          mine[4 * sg] = q * p.per + 16 * d;
+          mine[4 * sg + 1] = run_rows[q] - 16 * d < 16u ? run_rows[q] - 16 * d : 16u;
+          mine[4 * sg + 2] = keys[order[q]];
+        }
+      }
+      base += v[i];
+    }
+    const u4 m = *reinterpret_cast<const u4*>(mine + (lane >> 4) * 4);
+    const uint32_t row = m.x + (lane & 15), q = row * p.per_inv >> 16;
+    seg_rows = m.y;
+    seg_expert = m.z;
+    seg_row = (lane & 15) < m.y ? order[q] * p.per + row - q * p.per : 0;
+    wait_lds();
+    q4::lds_barrier();                                    // (the rings may be filled)
+  } else if (MODE != DENSE) {
+    take_share(uni(*p.n_chunks));
+  } else {
+    pos = uni(blockIdx.x * share + (blockIdx.x < over ? blockIdx.x : over));
+    end = uni(pos + share + (blockIdx.x < over ? 1 : 0));
   }
-  uint32_t pos = uni(blockIdx.x * share + (blockIdx.x < over ? blockIdx.x : over));
-  const uint32_t end = uni(pos + share + (blockIdx.x < over ? 1 : 0));
   const uint32_t xshift = x_dtype == RMLX_DTYPE_F32 ? 2 : 1;
   const uint32_t lds0 = uni((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds);
   if (pos >= end) return;
+  uint32_t seg = 0;
 
   do {
     // (what follows from these is worked out where it is used: kept across segments it costs more registers than there are, and the first
@@ -159,21 +249,29 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
     const uint32_t G = K / GS, row_bytes = K * BITS / 8;
     const uint32_t chunk = MODE == DENSE ? blockIdx.y : pos / N, r0 = MODE == DENSE ? pos : pos - chunk * N, r1 = end - pos < N - r0 ? r0 + (end - pos) : N;
     pos += r1 - r0;
-    uint32_t expert = 0, row0 = chunk * 16, rows = p.M - row0 < 16u ? p.M - row0 : 16u;
+    uint32_t expert = 0, row0 = chunk * 16, rows = M - row0 < 16u ? M - row0 : 16u;
     bool zeros = false;
-    if (MODE != DENSE) {
+    if constexpr (MODE == GATHER) {
+      expert = __builtin_amdgcn_readlane(seg_expert, seg * 16); rows = __builtin_amdgcn_readlane(seg_rows, seg * 16);
+      zeros = expert == kNoExpert;
+      if (zeros) expert = 0;
+    } else if (MODE != DENSE) {
       expert = uni(p.chunk_tab[3 * chunk]); row0 = uni(p.chunk_tab[3 * chunk + 1]); rows = uni(p.chunk_tab[3 * chunk + 2]);
       zeros = (rows >> 31) != 0;
       rows &= 0x7FFFFFFFu;
       if (zeros) expert = 0;
     }
     auto at = [](const void* q, uint64_t o) { return static_cast<const void*>(static_cast<const char*>(q) + o); };
-    const bool mapped = MODE != DENSE && p.row_map != nullptr;
+    const bool mapped = MODE == GATHER || (MODE != DENSE && p.row_map != nullptr);
+    auto source_row = [&](uint32_t m) -> uint32_t { return __builtin_amdgcn_ds_bpermute((seg * 16 + m) * 4, seg_row); };  // GATHER
     const uint32_t xrow = K << xshift;
     const void* const x_base = mapped ? x : at(x, (uint64_t)row0 * xrow);
     const u4 xr = rsrc(x_base, (uint64_t)(mapped ? p.x_rows : rows) * xrow);
     const uint32_t xm = lane & 15;                        // of the lane's row, and its place in a product
-    const uint32_t x_lane = xm < rows ? (mapped ? p.row_map[row0 + xm] : xm) * xrow + ((lane >> 4) * kLaneK<BITS, GS> << xshift) : kOutside;
+    uint32_t x_row = xm;
+    if constexpr (MODE == GATHER) x_row = source_row(xm);
+    else if (mapped && xm < rows) x_row = p.row_map[row0 + xm];
+    const uint32_t x_lane = xm < rows ? x_row * xrow + ((lane >> 4) * kLaneK<BITS, GS> << xshift) : kOutside;
 
     // ---- activations: this wave's part of every slot, in operand order (k past the row, rows past the chunk: zeros from the range check) ----
     u4 xv[H][U][kProducts];
@@ -261,20 +359,19 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
     const bool has_s = (wave & 3) * 1024 < C::kSBytes;
     uint32_t iq = 0, iplace = 0, splace = 0;              // the next slot to go out, its places in the rings
     auto issue = [&](bool first) {                        // (first: its tile's scales go out with it)
+      if (iq >= slots) return;                            // (an empty load costs 16 cycles of the address unit all the same)
       const uint32_t tm = iq / H, t = DUAL ? tm >> 1 : tm;
-      const bool up = DUAL && (tm & 1) != 0, ok = iq < slots;
-      const uint32_t wo = ok ? (t << (4 + nt_log2)) * row_bytes + (H == 1 ? 0 : iq % H * cpr * 16) : kOutside;
-      const u4 wr = up ? wr1 : wr0, sr = up ? sr1 : sr0;
+      const bool up = DUAL && (tm & 1) != 0;
+      const u4 wr = later(up ? wr1 : wr0, (t << (4 + nt_log2)) * row_bytes + (H == 1 ? 0 : iq % H * cpr * 16));
       if (first && has_s) {
-        const uint32_t sa = scales_at(t), so = ok ? (sa < s_last ? sa : s_last) : kOutside;
-        const uint32_t from = sa < s_last ? s_from : s_from_last;
+        const uint32_t sa = scales_at(t);
         set_m0(lds0 + C::oScales + splace * C::kScales + (wave < 4 ? 0 : C::kSBytes) + (wave & 3) * 1024);
-        dma16_plain(from + so, sr);
+        dma16_plain(sa < s_last ? s_from : s_from_last, later(up ? sr1 : sr0, sa < s_last ? sa : s_last));
       }
       if (first) splace = splace == R - 1 ? 0 : splace + 1;
       repeat<U>([&](auto u) {
         if (decltype(u)::value % 4 == 0) set_m0(lds0 + iplace * C::kWBytes + (wave * U + decltype(u)::value) * 1024);
-        dma16_next<decltype(u)::value % 4 * 1024>(w_from[u] < kOutside ? w_from[u] + wo : kOutside, wr);
+        dma16_next<decltype(u)::value % 4 * 1024>(w_from[u], wr);
       });
       iplace = iplace == R - 1 ? 0 : iplace + 1;
       ++iq;
@@ -457,7 +554,13 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
     const uint64_t out_at = (uint64_t)(row0 + out_m) * p.ld_out + r0 + out_c;
     f4 gate;
     float term[8];
+    uint32_t term_row[4];                                 // GATHER: the rows of x and of the result
     auto sums_read = [&](uint32_t tm) {
+      if constexpr (MODE == GATHER) {
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e)
+          if (e < 1u << w_log2) term_row[e] = source_row(out_m + e);
+      }
       const char* q = lds + get + (tm & 1) * C::kSums;
       if (nt_log2 == 0) {
 #pragma unroll
@@ -493,7 +596,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
       }
       const uint32_t c = (DUAL ? tm >> 1 : tm) << (4 + nt_log2);
       if (out_rows == 0 || c + out_c >= r1 - r0) return;
-      if (p.out_f32) {
+      if constexpr (MODE == GATHER) {
+        __half* q = static_cast<__half*>(p.out) + r0 + out_c + c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (e < w && (uint32_t)e < out_rows) q[(uint64_t)term_row[e] * p.ld_out] = __float2half(zeros ? 0.f : v[e]);
+      } else if (p.out_f32) {
         float* q = static_cast<float*>(p.out) + out_at + c;
 #pragma unroll
         for (int e = 0; e < 4; ++e, q += p.ld_out)
@@ -506,20 +614,24 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
       }
     };
 
-    // loads of slots q + 1 .. q + count still on their way (those of a slot: U, and one of its tile's scales with its first)
-    auto wait_but = [&](auto firsts, auto count) {
+    // `count` slots may still be on their way, `left` of them at most exist (those of a slot: U loads, and one of its tile's scales with its
+    // first; near the end the scales' loads are not counted, so one or two more loads are waited for)
+    auto wait_but = [&](auto firsts, auto count, uint32_t left) {
       constexpr int all = decltype(count)::value * U;
-      if (has_s) wait_loads<all + decltype(firsts)::value>();
-      else wait_loads<all>();
+      if (left >= (uint32_t)decltype(count)::value) {
+        if (has_s) wait_loads<all + decltype(firsts)::value>();
+        else wait_loads<all>();
+      } else if (decltype(count)::value > 1 && left != 0) wait_loads<U>();
+      else wait_loads<0>();
     };
     using std::integral_constant;
-    wait_but(integral_constant<int, (R + H - 1) / H>{}, integral_constant<int, R>{});
+    wait_but(integral_constant<int, (R + H - 1) / H>{}, integral_constant<int, R>{}, slots);
     hold_x();
     prepare_x();
     // Slot s is multiplied from registers while slot s + 1 is read from LDS; the barrier behind it says that everybody has read slot
     // s + 1, whose place the loads of slot s + 1 + R then take, and that slot s + 2 has arrived.
     Operands o[2];
-    wait_but(integral_constant<int, H == 1 ? R - 2 : (R - 2 + 1) / 2>{}, integral_constant<int, R - 2>{});
+    wait_but(integral_constant<int, H == 1 ? R - 2 : (R - 2 + 1) / 2>{}, integral_constant<int, R - 2>{}, slots > 2 ? slots - 2 : 0);
     q4::lds_barrier();
     read(o[0], integral_constant<int, 0>{});
     q4::lds_barrier();
@@ -535,7 +647,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
         if (h == H - 1) *reinterpret_cast<f4*>(lds + put + (tm & 1) * C::kSums) = idle ? (f4){0.f, 0.f, 0.f, 0.f} : acc;
         if (h == 0 && tm > 0 && ot < NT) sums_store(tm - 1);
         // slots s + 3 .. s + R may still be on their way
-        wait_but(integral_constant<int, H == 1 ? R - 2 : (R % 2 == 0 ? (R - 2) / 2 : (R - 3) / 2 + ((s + 3) % 2 == 0 ? 1 : 0))>{}, integral_constant<int, R - 2>{});
+        wait_but(integral_constant<int, H == 1 ? R - 2 : (R % 2 == 0 ? (R - 2) / 2 : (R - 3) / 2 + ((s + 3) % 2 == 0 ? 1 : 0))>{}, integral_constant<int, R - 2>{},
+                 slots > s2 + s + 3 ? slots - (s2 + s + 3) : 0);
         q4::lds_barrier();
         issue(H == 1 || (s + 1 + R) % H == 0);
       });
@@ -546,6 +659,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
     }
     wait_loads<0>();
     if (MODE != DENSE) q4::lds_barrier();  // (the rings are free again)
+    ++seg;
   } while (MODE != DENSE && pos < end);
 }
 
@@ -553,10 +667,12 @@ struct RingLaunch { const QmvArgs* a; uint32_t geometry, share, over, chunks, cp
 template <int BITS, int GS, int U, int H, int MODE>
 void launch_ring(const RingLaunch& l, hipStream_t s) {
   hipLaunchKernelGGL((qmv_ring_kernel<BITS, GS, U, H, MODE>), dim3(ctx().num_cus, l.chunks), dim3(kWaves * 64), 0, s, l.a->w0, l.a->s0, l.a->b0,
-                     static_cast<const void*>(l.a->x), l.a->N, l.a->K, l.geometry, l.share, l.over, l.cpr_inv, l.p);
+                     static_cast<const void*>(l.a->x), l.a->N, l.a->K, l.a->M, l.geometry, l.share, l.over, l.cpr_inv, l.p);
 }
 template <int BITS, int GS, int U, int H>
 void launch_mode(const RingLaunch& l, hipStream_t s) {
+  if constexpr (BITS == 4)
+    if (l.p.picks != nullptr) { launch_ring<BITS, GS, U, H, GATHER>(l, s); return; }
   if (l.a->dual) launch_ring<BITS, GS, U, H, PAIR>(l, s);
   else if (l.a->chunk_tab != nullptr) launch_ring<BITS, GS, U, H, TABLE>(l, s);
   else launch_ring<BITS, GS, U, H, DENSE>(l, s);
@@ -596,33 +712,22 @@ bool qmv_ring_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
   return N >= 16u * (8 / plan.ks) && (uint64_t)N * K * bits / 8 <= 0x80000000ull && (uint64_t)N * (K / group_size) * 2 < 0x7FFF0000ull;
 }
 
-int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32_t x_rows, hipStream_t s) {
-  const uint32_t gs = a.group_size == 0 ? 64 : a.group_size, size = x_dtype == RMLX_DTYPE_F32 ? 4 : 2;
-  if (!qmv_ring_supported(a.N, a.K, gs, bits) || (a.dual != 0 && a.chunk_tab == nullptr) || (a.row_map != nullptr && (uint64_t)x_rows * a.K * size > 0x80000000ull))
-    return fail(RMLX_INVALID_SHAPE, "streaming qmv: unsupported shape N=%u K=%u bits=%u group_size=%u, %u rows", a.N, a.K, bits, gs, x_rows);
-  RingLaunch l{};
-  l.a = &a;
-  if (a.chunk_tab != nullptr) {
-    if (a.max_chunks == 0) return RMLX_OK;
-    if ((uint64_t)a.max_chunks * a.N > 0xFFFFFFFFull) return fail(RMLX_INVALID_SHAPE, "streaming qmv: too many row chunks (%u)", a.max_chunks);
-    l.chunks = 1;
-  } else {
-    if (a.M == 0) return RMLX_OK;
-    l.chunks = (a.M + 15) / 16;
-    l.share = a.N / ctx().num_cus;
-    l.over = a.N - l.share * ctx().num_cus;
-  }
-  RingParams& p = l.p;
+// What the launches have in common: the split of a row and the constants of the kernel's divisions
+static void ring_split(const QmvArgs& a, uint32_t bits, uint32_t gs, int32_t x_dtype, RingPlan* plan, RingLaunch* l) {
+  RingParams& p = l->p;
+  l->a = &a;
   p.out = a.out; p.row_map = a.row_map; p.chunk_tab = a.chunk_tab; p.n_chunks = a.n_chunks_dev;
   p.w1 = a.w1; p.s1 = a.s1; p.b1 = a.b1;
   p.estride_w = a.expert_stride_w; p.estride_s = a.expert_stride_s;
-  p.M = a.M; p.ld_out = a.ld_out; p.x_rows = x_rows; p.out_f32 = a.out_f32;
-  RingPlan plan;
-  ring_plan(a.K, gs, bits, &plan);
-  l.geometry = ring_geometry(plan.ks, x_dtype);
-  const uint32_t cpr = plan.h == 1 ? a.K * bits / 128 : plan.ks * plan.u * 4;
-  l.cpr_inv = ((1u << 20) + cpr - 1) / cpr;
+  p.ld_out = a.ld_out; p.out_f32 = a.out_f32;
+  ring_plan(a.K, gs, bits, plan);
+  l->geometry = ring_geometry(plan->ks, x_dtype);
+  const uint32_t cpr = plan->h == 1 ? a.K * bits / 128 : plan->ks * plan->u * 4;
+  p.slack = 102400 / (a.K * bits / 8);
+  l->cpr_inv = ((1u << 20) + cpr - 1) / cpr;
   if (a.K / gs >= 8) p.spr_inv = ((1u << 20) + a.K / gs / 8 - 1) / (a.K / gs / 8);
+}
+static int32_t launch_format(const RingLaunch& l, const RingPlan& plan, uint32_t bits, uint32_t gs, hipStream_t s) {
   if (bits == 4) {
     if (gs == 32) launch_slice<4, 32>(l, plan, s);
     else if (gs == 64) launch_slice<4, 64>(l, plan, s);
@@ -634,6 +739,48 @@ int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32
   }
   RMLX_HIP_CHECK(hipGetLastError());
   return RMLX_OK;
+}
+
+int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32_t x_rows, hipStream_t s) {
+  const uint32_t gs = a.group_size == 0 ? 64 : a.group_size, size = x_dtype == RMLX_DTYPE_F32 ? 4 : 2;
+  if (!qmv_ring_supported(a.N, a.K, gs, bits) || (a.dual != 0 && a.chunk_tab == nullptr) || (a.row_map != nullptr && (uint64_t)x_rows * a.K * size > 0x80000000ull))
+    return fail(RMLX_INVALID_SHAPE, "streaming qmv: unsupported shape N=%u K=%u bits=%u group_size=%u, %u rows", a.N, a.K, bits, gs, x_rows);
+  RingLaunch l{};
+  RingPlan plan;
+  ring_split(a, bits, gs, x_dtype, &plan, &l);
+  l.p.x_rows = x_rows;
+  if (a.chunk_tab != nullptr) {
+    if (a.max_chunks == 0) return RMLX_OK;
+    if ((uint64_t)a.max_chunks * a.N > 0xFFFFFFFFull) return fail(RMLX_INVALID_SHAPE, "streaming qmv: too many row chunks (%u)", a.max_chunks);
+    l.chunks = 1;
+  } else {
+    if (a.M == 0) return RMLX_OK;
+    l.chunks = (a.M + 15) / 16;
+    l.share = a.N / ctx().num_cus;
+    l.over = a.N - l.share * ctx().num_cus;
+  }
+  return launch_format(l, plan, bits, gs, s);
+}
+
+bool qmv_ring_gather_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t entries, uint32_t per, uint32_t n_experts, int32_t x_dtype) {
+  const uint64_t rows = (uint64_t)entries * per;
+  // (a workgroup's share lies in at most four chunks: there are at most twice as many of these as workgroups)
+  const uint64_t chunks = rows / 16 + (entries < n_experts ? entries : n_experts + 1);
+  return per >= 1 && per <= 16 && entries <= kMaxEntries && n_experts < kNoExpert && qmv_ring_supported(N, K, group_size, 4) &&
+         chunks <= 2 * (uint64_t)ctx().num_cus && chunks * N <= 0xFFFFFFFFull && rows * K * (x_dtype == RMLX_DTYPE_F32 ? 4 : 2) <= 0x80000000ull;
+}
+
+int32_t launch_qmv_ring_gather(const QmvArgs& a, const uint32_t* picks, uint32_t entries, uint32_t per, uint32_t n_experts, int32_t x_dtype, hipStream_t s) {
+  const uint32_t gs = a.group_size;
+  if (!qmv_ring_gather_supported(a.N, a.K, gs, entries, per, n_experts, x_dtype))
+    return fail(RMLX_INVALID_SHAPE, "streaming qmv: unsupported gather N=%u K=%u group_size=%u, %u x %u rows", a.N, a.K, gs, entries, per);
+  RingLaunch l{};
+  RingPlan plan;
+  ring_split(a, 4, gs, x_dtype, &plan, &l);
+  l.chunks = 1;
+  l.p.x_rows = entries * per;
+  l.p.picks = picks; l.p.entries = entries; l.p.per = per; l.p.per_inv = (65536 + per - 1) / per; l.p.n_experts = n_experts;
+  return launch_format(l, plan, 4, gs, s);
 }
 
 }  // namespace rmlx

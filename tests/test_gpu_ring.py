@@ -67,9 +67,9 @@ def test_routed_block(hip, bits, gs, hidden, inter, tokens, experts, fused, dtyp
     assert np.array_equal(same.view(np.uint16), out.view(np.uint16))
 
 
-@pytest.mark.parametrize("tokens,taken", [(18, False), (20, True), (40, True), (42, False)])
+@pytest.mark.parametrize("tokens,taken", [(18, False), (20, True), (52, True), (53, False)])
 def test_library_takes_it_for_a_few_rows_per_expert(hip, tokens, taken):
-    """Experts of 4M values on average 5 to 10 rows each; a threshold of the caller's for the grouped GEMM goes first."""
+    """Experts of 6 MB, on average 5 to 13 rows each; a threshold of the caller's for the grouped GEMM goes first."""
     from rmlx_amd import ops, runtime as rt
     rng = np.random.default_rng(tokens)
     experts, hidden = 8, 2048
@@ -94,3 +94,56 @@ def test_library_takes_it_for_a_few_rows_per_expert(hip, tokens, taken):
     idx, w, _, _ = model.topk_route(logits, 2)
     gate, up = tuple(a[:, :hidden] for a in gate_up), tuple(a[:, hidden:] for a in gate_up)
     assert_close(auto, model.moe_forward(x, idx, w, gate, up, down, 64, 2))
+
+
+@pytest.mark.parametrize("gs,k,n", [(64, 512, 128), (64, 4096, 515), (64, 6208, 300), (32, 1056, 1001), (128, 2944, 4100)])
+@pytest.mark.parametrize("batch,rows,experts,dtype", [(1, 1, 3, "f16"), (5, 16, 2, "f16"), (37, 3, 4, "f32"), (256, 1, 200, "f16"), (255, 5, 7, "f32"), (160, 13, 3, "f16"),
+                                                      (129, 2, 1000, "f16")])
+def test_gather(hip, gs, k, n, batch, rows, experts, dtype):
+    """Entries of one expert share chunks of 16 rows: runs of one entry and of many, chunks that begin in the middle of an entry, more
+    chunks than workgroups; on a stream the rows of an index out of range are zero."""
+    from rmlx_amd import ops, runtime as rt
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(batch + rows + n)
+    stored = min(experts, 8)
+    w = make_weight(rng, n, k, 4, gs, (experts,) if experts == stored else (stored,))
+    if experts != stored:
+        w = tuple(np.concatenate([a] * (experts // stored), axis=0) for a in w)
+    experts = w[0].shape[0]
+    idx = rng.integers(0, experts, size=batch).astype(np.uint32)
+    bad = np.zeros(batch, bool)
+    if batch > 30:
+        bad[[3, 17, 29]] = True
+        idx[bad] = experts, 0xFFFFFFFE, 0xFFFFFFFF
+    x = make_x(rng, batch * rows, k, dtype).reshape(batch, rows, k)
+    stream = rt.Stream()
+    out = ops.gather_qmm(DeviceBuffer.from_numpy(x), *(DeviceBuffer.from_numpy(a) for a in w), DeviceBuffer.from_numpy(idx), batch, rows, n, k, experts, gs,
+                         stream=stream, kernel=rt.GATHER_SLOTS)
+    stream.sync()
+    out = out.numpy().reshape(batch, rows, n)
+    assert not out[bad].any()
+    cols = np.unique(np.concatenate([np.arange(min(n, 100)), np.arange(0, n, 29), np.arange(n - 40, n)]))
+    x64 = x.astype(np.float16).astype(np.float64)
+    ref = np.zeros((batch, rows, cols.size))
+    for e in range(stored):
+        of = ~bad & (idx % stored == e)
+        if of.any():
+            ref[of] = model.qmm(x64[of].reshape(-1, k), *(a[e][cols] for a in w), gs, 4).reshape(-1, rows, cols.size)
+    assert_close(out[..., cols], ref)
+    assert _ratio(out[..., cols], ref) < 1.05
+
+
+@pytest.mark.parametrize("batch,rows,experts,n,k,taken", [(144, 1, 8, 1536, 2048, True), (16, 1, 8, 512, 1024, False), (64, 4, 8, 3072, 4096, True),
+                                                          (6, 16, 8, 1536, 2048, False), (8, 4, 8, 6400, 1984, True)])
+def test_library_takes_it_for_gathers_of_many_weights(hip, batch, rows, experts, n, k, taken):
+    from rmlx_amd import ops, runtime as rt
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(batch + n)
+    one = make_weight(rng, n, k, 4, 64)
+    w = [DeviceBuffer.from_numpy(np.ascontiguousarray(np.broadcast_to(a, (experts,) + a.shape))) for a in one]
+    x = make_x(rng, batch * rows, k).reshape(batch, rows, k)
+    xd, idx = DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(rng.integers(0, experts, size=batch).astype(np.uint32))
+    auto, forced = (ops.gather_qmm(xd, *w, idx, batch, rows, n, k, experts, 64, kernel=q).numpy() for q in (0, rt.GATHER_SLOTS))
+    assert np.array_equal(auto.view(np.uint16), forced.view(np.uint16)) == taken
+    cols = np.arange(0, n, 37)
+    assert_close(auto.reshape(-1, n)[:, cols], model.qmm(x.reshape(-1, k).astype(np.float64), *(a[cols] for a in one), 64, 4))
