@@ -147,3 +147,25 @@ def test_library_takes_it_for_gathers_of_many_weights(hip, batch, rows, experts,
     assert np.array_equal(auto.view(np.uint16), forced.view(np.uint16)) == taken
     cols = np.arange(0, n, 37)
     assert_close(auto.reshape(-1, n)[:, cols], model.qmm(x.reshape(-1, k).astype(np.float64), *(a[cols] for a in one), 64, 4))
+
+
+# both sides of each line of the rule, one call of every kind that it takes over (odd height, ragged K, each row count class, f32 rows that it
+# reads itself and that are cast first)
+@pytest.mark.parametrize("m,n,k,bits,gs,dtype,taken", [(1, 50001, 1024, 4, 64, "f16", True), (1, 50000, 1024, 4, 64, "f16", False), (2, 33001, 2880, 4, 64, "bf16", True),
+                                                       (2, 4096, 2880, 4, 64, "f16", False), (8, 9216, 2880, 4, 64, "f16", True), (8, 9216, 4096, 4, 64, "f16", False),
+                                                       (4, 14336, 6400, 4, 64, "f16", False), (9, 9216, 2048, 4, 128, "bf16", True), (16, 4096, 4096, 4, 64, "f16", False),
+                                                       (12, 14336, 4096, 4, 64, "f32", True), (3, 2304, 1728, 8, 64, "bf16", True), (3, 2304, 1536, 8, 64, "bf16", False),
+                                                       (13, 4096, 4096, 8, 64, "f32", True), (5, 4096, 4096, 8, 32, "f32", True), (4, 4096, 1024, 4, 32, "f16", True),
+                                                       (8, 4096, 1024, 4, 32, "f16", False), (16, 4096, 1152, 4, 32, "bf16", True), (17, 4096, 1152, 4, 32, "bf16", False)])
+def test_library_takes_it_for_a_few_rows(hip, m, n, k, bits, gs, dtype, taken):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    wd = ops.QuantizedWeight.from_numpy(*w, gs, bits)
+    auto, forced = (ops.affine_quantized_matmul_batched(xd, wd, kernel=q).numpy() for q in (0, rt.KERNEL_QMV_RING))
+    assert np.array_equal(auto.view(np.uint16), forced.view(np.uint16)) == taken
+    cols = np.unique(np.concatenate([np.arange(0, n, 41), np.arange(n - 20, n)]))
+    x64 = x_as_f64(x, dtype).astype(np.float16).astype(np.float64)
+    assert_close(auto[:, cols], model.qmm(x64, *(a[cols] for a in w), gs, bits))
