@@ -33,6 +33,7 @@
 //     4 waves of the workgroup.
 #include <vector>
 
+#include "launch.hpp"
 #include "common.hpp"
 #include "route.hpp"
 
@@ -47,11 +48,10 @@ constexpr int kThreads = 512;
 constexpr int kWaves = 8;
 constexpr uint32_t kMaxK = 32768;  // (the activation image and sums must also fit the default dynamic LDS limit)
 
-struct M1Params {
-  const uint32_t* w; const __half* s; const __half* b;
-  const __half* x;
+// What only some kernels or only the end of one needs.  The rest of M1Params are plain arguments (launch.hpp).  One row, 4096 x 4096 3.97 -> 3.83 us, 9216 x 4096 6.7 -> 6.4, 8-bit
+// 4096 x 4096 5.1 -> 4.8.
+struct M1Rest {
   __half* out;
-  uint32_t N, K, M;
   int32_t epi_kind, epi_dtype;  // fused store epilogue: EPI_RESIDUAL / EPI_SWIGLU with an [M,N] f16 / f32 operand
   const void* epi;
   // fused RMSNorm prologue (null = none): x[m,k] <- (x[m,k] * half(inv_rms[m])) * norm_w[k], each product rounded to f16
@@ -66,6 +66,11 @@ struct M1Params {
   // gather_idx[(gather_row0 + m) / gather_div]; 0 or 1 = an index per row)
   uint32_t gather_div = 1, gather_row0 = 0;
   int32_t x_bf16 = 0;  // 1: the activations are bf16 bits, 2: f32 values (kernels built with the conversion prologues only, see launch_r)
+};
+struct M1Params : M1Rest {
+  const uint32_t* w; const __half* s; const __half* b;
+  const __half* x;
+  uint32_t N, K, M;
 };
 
 __device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
@@ -346,7 +351,11 @@ template <int BITS, int GS, int R, bool NT, int MR, int NORM = 0, int KP = 1, bo
 // measured 4-13 % faster.  The 4-bit kernel would spill under that bound and is slower with it.  Two activation
 // rows: without a bound the scheduler spends 124 registers on a schedule that is 12 % slower than the one it finds
 // within the 96 of five waves per SIMD.)
-__global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (MR == 2 ? 5 : 1)) void qmv_m1_kernel(M1Params p) {
+__global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (MR == 2 ? 5 : 1)) void qmv_m1_kernel(uint64_t w_, uint64_t s_, uint64_t b_, uint64_t x_, uint32_t N_, uint32_t K_, uint32_t M_,
+                                                                    int32_t x_bf16_, int32_t epi_kind_, M1Rest rest) {
+  M1Params p{rest, global_at<uint32_t>(w_), global_at<__half>(s_), global_at<__half>(b_), global_at<__half>(x_), N_, K_, M_};
+  // (two rows: loaded; preloaded these two make 4096 x 4096 4.7 us instead of 4.4)
+  if constexpr (MR == 1) { p.x_bf16 = x_bf16_; p.epi_kind = epi_kind_; }
   using Image = XImage<BITS, MR>;
   constexpr int kChunkK = Image::kChunkK, kLaneK = Image::kLaneK;
   constexpr int kLanesPerGroup = GS / kLaneK;  // whole lanes per quantisation group
@@ -485,7 +494,11 @@ __global__ __launch_bounds__(kThreads, (BITS == 8 && MR == 1 && R == 1) ? 8 : (M
 template <int BITS, int GS, int R, bool NT, int MR, int NORM = 0, bool GATHER = false>
 // (8-bit, one row: asking the compiler for eight waves per SIMD changes no register count but the schedule;
 // measured 4-13 % faster.  The 4-bit kernel would spill under that bound and is slower with it.)
-__global__ __launch_bounds__(kThreads, 1) void qmv_m1_loop_kernel(M1Params p) {
+__global__ __launch_bounds__(kThreads, 1) void qmv_m1_loop_kernel(uint64_t w_, uint64_t s_, uint64_t b_, uint64_t x_, uint32_t N_, uint32_t K_, uint32_t M_,
+                                                                    int32_t x_bf16_, int32_t epi_kind_, M1Rest rest) {
+  M1Params p{rest, global_at<uint32_t>(w_), global_at<__half>(s_), global_at<__half>(b_), global_at<__half>(x_), N_, K_, M_};
+  // (two rows: loaded; preloaded these two make 4096 x 4096 4.7 us instead of 4.4)
+  if constexpr (MR == 1) { p.x_bf16 = x_bf16_; p.epi_kind = epi_kind_; }
   using Image = XImage<BITS, MR>;
   constexpr int kChunkK = Image::kChunkK, kLaneK = Image::kLaneK;
   constexpr int kLanesPerGroup = GS / kLaneK;  // whole lanes per quantisation group
@@ -669,7 +682,8 @@ __device__ __forceinline__ uint32_t gate_up_expert(const M1GateUpParams& p, uint
 }
 
 template <int BITS, int GS, bool XBF = false>  // XBF: the activations are bf16 bits, converted while they are staged
-__global__ __launch_bounds__(kThreads, 1) void qmv_m1_gate_up_kernel(M1GateUpParams p) {
+__global__ __launch_bounds__(kThreads, 1) void qmv_m1_gate_up_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint64_t idx_, uint32_t K_, uint32_t N_, uint32_t top_k_, uint32_t n_experts_, M1GateUpParams p) {
+  p.w0 = global_at<uint32_t>(w0_); p.s0 = global_at<__half>(s0_); p.b0 = global_at<__half>(b0_); p.x = global_at<__half>(x_); p.idx = global_at<uint32_t>(idx_); p.K = K_; p.N = N_; p.top_k = top_k_; p.n_experts = n_experts_;
   using Image = XImage<BITS, 1>;
   constexpr int kChunkK = Image::kChunkK, kLaneK = Image::kLaneK;
   constexpr int kLanesPerGroup = GS / kLaneK, kGroupsPerChunk = kChunkK / GS;
@@ -742,7 +756,8 @@ __global__ __launch_bounds__(kThreads, 1) void qmv_m1_gate_up_kernel(M1GateUpPar
 // (resident workgroups / assignments, assignments) and a workgroup walks the row blocks blockIdx.x, blockIdx.x + gridDim.x,
 // ... of its assignment, staging the activations once, the next block's weights in flight while the current one is multiplied.
 template <int BITS, int GS, bool XBF = false>
-__global__ __launch_bounds__(kThreads, 1) void qmv_m1_gate_up_loop_kernel(M1GateUpParams p) {
+__global__ __launch_bounds__(kThreads, 1) void qmv_m1_gate_up_loop_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint64_t idx_, uint32_t K_, uint32_t N_, uint32_t top_k_, uint32_t n_experts_, M1GateUpParams p) {
+  p.w0 = global_at<uint32_t>(w0_); p.s0 = global_at<__half>(s0_); p.b0 = global_at<__half>(b0_); p.x = global_at<__half>(x_); p.idx = global_at<uint32_t>(idx_); p.K = K_; p.N = N_; p.top_k = top_k_; p.n_experts = n_experts_;
   using Image = XImage<BITS, 1>;
   constexpr int kChunkK = Image::kChunkK, kLaneK = Image::kLaneK;
   constexpr int kLanesPerGroup = GS / kLaneK, kGroupsPerChunk = kChunkK / GS;
@@ -845,7 +860,8 @@ struct M1DownParams {
 // -- lanes 0-31 rows n0 .. n0+R-1, lanes 32-63 the next R -- so a short row does not leave more than half of the lanes
 // without a load (K = 768 at 4 bits: 24 of 32 lanes busy instead of 24 of 64).  Same products, same summation order per row.
 template <int BITS, int GS, int NC, int R, bool HALF = false>
-__global__ __launch_bounds__(kThreads, 2) void qmv_m1_down_combine_kernel(M1DownParams p) {
+__global__ __launch_bounds__(kThreads, 2) void qmv_m1_down_combine_kernel(uint64_t w_, uint64_t s_, uint64_t b_, uint64_t h_, uint64_t idx_, uint32_t K_, uint32_t N_, uint32_t top_k_, uint32_t n_experts_, M1DownParams p) {
+  p.w = global_at<uint32_t>(w_); p.s = global_at<__half>(s_); p.b = global_at<__half>(b_); p.h = global_at<__half>(h_); p.idx = global_at<uint32_t>(idx_); p.K = K_; p.N = N_; p.top_k = top_k_; p.n_experts = n_experts_;
   static_assert(!HALF || NC == 1, "half-wave rows: one chunk");
   using Image = XImage<BITS, 1>;
   constexpr int kChunkK = Image::kChunkK, kLaneK = Image::kLaneK, kXU = Image::kXU;
@@ -956,11 +972,23 @@ uint32_t resident_workgroups(Kernel kernel, size_t lds) {
   return wgs;
 }
 
+template <auto Kernel>
+void launch_kernel(const M1Params& p, dim3 grid, size_t lds, hipStream_t s) {
+  Launch<Kernel>::go(grid, dim3(kThreads), lds, s, address(p.w), address(p.s), address(p.b), address(p.x), p.N, p.K, p.M, p.x_bf16, p.epi_kind, static_cast<const M1Rest&>(p));
+}
+template <auto Kernel>
+void launch_kernel(const M1GateUpParams& p, dim3 grid, size_t lds, hipStream_t s) {
+  Launch<Kernel>::go(grid, dim3(kThreads), lds, s, address(p.w0), address(p.s0), address(p.b0), address(p.x), address(p.idx), p.K, p.N, p.top_k, p.n_experts, p);
+}
+template <auto Kernel>
+void launch_kernel(const M1DownParams& p, dim3 grid, size_t lds, hipStream_t s) {
+  Launch<Kernel>::go(grid, dim3(kThreads), lds, s, address(p.w), address(p.s), address(p.b), address(p.h), address(p.idx), p.K, p.N, p.top_k, p.n_experts, p);
+}
+
 template <int BITS, int GS, int R, bool NT, int MR, int NORM, int KP = 1, bool GATHER = false>
 void launch_k(const M1Params& p, size_t lds, hipStream_t s) {
   if constexpr (KP > 1) {  // split rows: short matrices only, every row group has its workgroup
-    hipLaunchKernelGGL((qmv_m1_kernel<BITS, GS, R, NT, MR, NORM, KP>), dim3((p.N + kWaves / KP - 1) / (kWaves / KP), (p.M + MR - 1) / MR),
-                       dim3(kThreads), lds, s, p);
+    launch_kernel<qmv_m1_kernel<BITS, GS, R, NT, MR, NORM, KP>>(p, dim3((p.N + kWaves / KP - 1) / (kWaves / KP), (p.M + MR - 1) / MR), lds, s);
     return;
   }
   // one workgroup per row block while all of them are resident together, else as many as are (they loop)
@@ -970,8 +998,8 @@ void launch_k(const M1Params& p, size_t lds, hipStream_t s) {
   gx = gx < 1 ? 1 : gx;
   // (as many workgroups as are resident, even where that leaves some of them one block more than others: fewer
   // workgroups with equal shares are slower, 8.1 against 6.7 us at N = 9216)
-  if (gx < nblk) hipLaunchKernelGGL(looping, dim3(gx, passes), dim3(kThreads), lds, s, p);
-  else hipLaunchKernelGGL((qmv_m1_kernel<BITS, GS, R, NT, MR, NORM, 1, GATHER>), dim3(nblk, passes), dim3(kThreads), lds, s, p);
+  if (gx < nblk) launch_kernel<qmv_m1_loop_kernel<BITS, GS, R, NT, MR, NORM, GATHER>>(p, dim3(gx, passes), lds, s);
+  else launch_kernel<qmv_m1_kernel<BITS, GS, R, NT, MR, NORM, 1, GATHER>>(p, dim3(nblk, passes), lds, s);
 }
 
 template <int BITS, int R, bool NT, int MR, int KP = 1>
@@ -1081,11 +1109,11 @@ int32_t launch_qmv_m1(const uint32_t* w, const __half* s, const __half* b, const
   if (M > 65535) return fail(RMLX_INVALID_SHAPE, "qmv_m1: at most 65535 rows per launch (M=%u)", M);
   if (norm_w != nullptr && !qmv_m1_fuses_norm(M, K, bits))
     return fail(RMLX_RUNTIME_ERROR, "qmv_m1: the RMSNorm prologue is fused for at most two rows in one pass (M=%u K=%u)", M, K);
-  M1Params p{w, s, b, x, out, N, K, M, epi_kind, epi_dtype, epi, norm_w, inv_rms};
+  M1Params p{{out, epi_kind, epi_dtype, epi, norm_w, inv_rms}, w, s, b, x, N, K, M};
   p.x_bf16 = x_bf16;
   if (bits == 4) launch_bits<4>(p, group_size, stream);
   else launch_bits<8>(p, group_size, stream);
-  RMLX_HIP_CHECK(hipGetLastError());
+  RMLX_HIP_CHECK(take_launch_error());
   return RMLX_OK;
 }
 
@@ -1112,12 +1140,12 @@ int32_t launch_qmv_m1_gather(const uint32_t* w, const __half* s, const __half* b
   const bool two = (K >= 12288 || (bits == 4 && N >= 12288)) && N >= kWaves * 2;
   for (uint32_t first = 0; first < batch; first += 65535) {  // the activation row is the second grid dimension
     const uint32_t rows = batch - first < 65535 ? batch - first : 65535;
-    M1Params p{w, s, b, x + (uint64_t)first * K, out + (uint64_t)first * N, N, K, rows, EPI_NONE, 0, nullptr, nullptr, nullptr,
-               rows_per_index > 1 ? idx : idx + first, estride_w, estride_s, n_experts};
+    M1Params p{{out + (uint64_t)first * N, EPI_NONE, 0, nullptr, nullptr, nullptr, rows_per_index > 1 ? idx : idx + first, estride_w, estride_s, n_experts},
+               w, s, b, x + (uint64_t)first * K, N, K, rows};
     if (rows_per_index > 1) { p.gather_div = rows_per_index; p.gather_row0 = first; }
     if (bits == 4) launch_gather_bits<4>(p, group_size, two, stream);
     else launch_gather_bits<8>(p, group_size, two, stream);
-    RMLX_HIP_CHECK(hipGetLastError());
+    RMLX_HIP_CHECK(take_launch_error());
   }
   return RMLX_OK;
 }
@@ -1135,8 +1163,8 @@ void launch_gate_up_x(const M1GateUpParams& p, uint32_t assignments, hipStream_t
   auto looping = qmv_m1_gate_up_loop_kernel<BITS, GS, XBF>;
   uint32_t gx = resident_workgroups(looping, lds) / assignments;
   gx = gx < 1 ? 1 : gx;
-  if (gx < nblk) hipLaunchKernelGGL(looping, dim3(gx, assignments), dim3(kThreads), lds, stream, p);
-  else hipLaunchKernelGGL((qmv_m1_gate_up_kernel<BITS, GS, XBF>), dim3(nblk, assignments), dim3(kThreads), lds, stream, p);
+  if (gx < nblk) launch_kernel<qmv_m1_gate_up_loop_kernel<BITS, GS, XBF>>(p, dim3(gx, assignments), lds, stream);
+  else launch_kernel<qmv_m1_gate_up_kernel<BITS, GS, XBF>>(p, dim3(nblk, assignments), lds, stream);
 }
 template <int BITS, int GS>
 void launch_gate_up(const M1GateUpParams& p, uint32_t assignments, bool x_bf16, hipStream_t stream) {
@@ -1172,7 +1200,7 @@ int32_t launch_qmv_m1_gate_up(const QmvArgs& a, uint32_t bits, const uint32_t* i
       default: launch_gate_up<8, 128>(p, assignments, a.x_bf16 != 0, stream); break;
     }
   }
-  RMLX_HIP_CHECK(hipGetLastError());
+  RMLX_HIP_CHECK(take_launch_error());
   return RMLX_OK;
 }
 
@@ -1196,9 +1224,9 @@ void launch_down_combine(const M1DownParams& p, int chunks, uint32_t T, hipStrea
   // (four rows per wave: the weights of a pass fit the registers of two workgroups per CU)
   // (short rows, N in whole blocks of 8: two groups of four rows per wave)
   if (chunks == 1 && p.K * BITS / 8 <= 512 && p.N % 8 == 0)
-    hipLaunchKernelGGL((qmv_m1_down_combine_kernel<BITS, GS, 1, 4, true>), dim3(p.N / 8, T), dim3(kThreads), 0, stream, p);
-  else if (chunks == 1) hipLaunchKernelGGL((qmv_m1_down_combine_kernel<BITS, GS, 1, 4>), dim3(p.N / 4, T), dim3(kThreads), 0, stream, p);
-  else hipLaunchKernelGGL((qmv_m1_down_combine_kernel<BITS, GS, 2, 4>), dim3(p.N / 4, T), dim3(kThreads), 0, stream, p);
+    launch_kernel<qmv_m1_down_combine_kernel<BITS, GS, 1, 4, true>>(p, dim3(p.N / 8, T), 0, stream);
+  else if (chunks == 1) launch_kernel<qmv_m1_down_combine_kernel<BITS, GS, 1, 4>>(p, dim3(p.N / 4, T), 0, stream);
+  else launch_kernel<qmv_m1_down_combine_kernel<BITS, GS, 2, 4>>(p, dim3(p.N / 4, T), 0, stream);
 }
 }  // namespace
 
@@ -1226,7 +1254,7 @@ int32_t launch_qmv_m1_down_combine(const uint32_t* w, const __half* s, const __h
       default: launch_down_combine<4, 128>(p, chunks, T, stream); break;
     }
   }
-  RMLX_HIP_CHECK(hipGetLastError());
+  RMLX_HIP_CHECK(take_launch_error());
   return RMLX_OK;
 }
 

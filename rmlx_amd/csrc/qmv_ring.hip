@@ -21,6 +21,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "launch.hpp"
 #include "q4_stream.hpp"
 #include "tile.hpp"
 
@@ -132,9 +133,12 @@ struct Ring {
 };
 
 template <int BITS, int GS, int U, int H, int MODE>
-__global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t* w0, const __half* s0, const __half* b0, const void* x, uint32_t N,
+__global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint32_t N,
                                                                   uint32_t K, uint32_t M, uint32_t geometry, uint32_t share, uint32_t over, uint32_t cpr_inv,
                                                                   RingParams p) {
+  const uint32_t* const w0 = global_at<uint32_t>(w0_);
+  const __half *const s0 = global_at<__half>(s0_), *const b0 = global_at<__half>(b0_);
+  const char* const x = global_at<char>(x_);
   const uint32_t spr_inv = p.spr_inv;
   using C = Ring<BITS, GS, U, H>;
   constexpr bool DUAL = MODE == PAIR;
@@ -265,7 +269,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
     const bool mapped = MODE == GATHER || (MODE != DENSE && p.row_map != nullptr);
     auto source_row = [&](uint32_t m) -> uint32_t { return __builtin_amdgcn_ds_bpermute((seg * 16 + m) * 4, seg_row); };  // GATHER
     const uint32_t xrow = K << xshift;
-    const void* const x_base = mapped ? x : at(x, (uint64_t)row0 * xrow);
+    const void* const x_base = mapped ? static_cast<const void*>(x) : at(x, (uint64_t)row0 * xrow);
     const u4 xr = rsrc(x_base, (uint64_t)(mapped ? p.x_rows : rows) * xrow);
     const uint32_t xm = lane & 15;                        // of the lane's row, and its place in a product
     uint32_t x_row = xm;
@@ -666,8 +670,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(const uint32_t
 struct RingLaunch { const QmvArgs* a; uint32_t geometry, share, over, chunks, cpr_inv; RingParams p; };
 template <int BITS, int GS, int U, int H, int MODE>
 void launch_ring(const RingLaunch& l, hipStream_t s) {
-  hipLaunchKernelGGL((qmv_ring_kernel<BITS, GS, U, H, MODE>), dim3(ctx().num_cus, l.chunks), dim3(kWaves * 64), 0, s, l.a->w0, l.a->s0, l.a->b0,
-                     static_cast<const void*>(l.a->x), l.a->N, l.a->K, l.a->M, l.geometry, l.share, l.over, l.cpr_inv, l.p);
+  Launch<qmv_ring_kernel<BITS, GS, U, H, MODE>>::go(dim3(ctx().num_cus, l.chunks), dim3(kWaves * 64), 0, s, address(l.a->w0), address(l.a->s0),
+                                                    address(l.a->b0), address(l.a->x), l.a->N, l.a->K, l.a->M, l.geometry, l.share, l.over, l.cpr_inv, l.p);
 }
 template <int BITS, int GS, int U, int H>
 void launch_mode(const RingLaunch& l, hipStream_t s) {
@@ -737,7 +741,7 @@ static int32_t launch_format(const RingLaunch& l, const RingPlan& plan, uint32_t
     else if (gs == 64) launch_slice<8, 64>(l, plan, s);
     else launch_slice<8, 128>(l, plan, s);
   }
-  RMLX_HIP_CHECK(hipGetLastError());
+  RMLX_HIP_CHECK(take_launch_error());
   return RMLX_OK;
 }
 
