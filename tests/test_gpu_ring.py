@@ -169,3 +169,57 @@ def test_library_takes_it_for_a_few_rows(hip, m, n, k, bits, gs, dtype, taken):
     cols = np.unique(np.concatenate([np.arange(0, n, 41), np.arange(n - 20, n)]))
     x64 = x_as_f64(x, dtype).astype(np.float16).astype(np.float64)
     assert_close(auto[:, cols], model.qmm(x64, *(a[cols] for a in w), gs, bits))
+
+
+def test_rows_with_infinities_leave_the_others_alone(hip):
+    """A row's values meet only its own sums: not another row's through the shared operands, nor those of the rows that a chunk lacks."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(9)
+    for bits, k in ((4, 2880), (4, 6144), (8, 4096)):
+        w = make_weight(rng, 515, k, bits, 64)
+        wd = ops.QuantizedWeight.from_numpy(*w, 64, bits)
+        x = make_x(rng, 13, k)
+        clean = ops.affine_quantized_matmul_batched(rt.DeviceBuffer.from_numpy(x), wd, kernel=rt.KERNEL_QMV_RING).numpy()
+        x[3, 7], x[3, k - 1], x[8, k // 2], x[12, 0] = np.inf, -np.inf, np.nan, np.inf
+        out = ops.affine_quantized_matmul_batched(rt.DeviceBuffer.from_numpy(x), wd, kernel=rt.KERNEL_QMV_RING).numpy()
+        rest = [i for i in range(13) if i not in (3, 8, 12)]
+        assert np.array_equal(out[rest].view(np.uint16), clean[rest].view(np.uint16))
+        assert np.isnan(out[8]).all() and not np.isfinite(out[3]).any() and not np.isfinite(out[12]).any()
+
+
+def test_recorded_calls_replay_bit_for_bit(hip):
+    """A matrix, a gather and a routed block recorded into one graph, with eager work between the replays."""
+    from rmlx_amd import ops, runtime as rt
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(10)
+    n, k, experts, tokens = 520, 1088, 5, 40
+    wd = ops.QuantizedWeight.from_numpy(*make_weight(rng, n, k, 4, 64), 64, 4)
+    stacked = [DeviceBuffer.from_numpy(a) for a in make_weight(rng, n, k, 4, 64, (experts,))]
+    gate_up, down = make_weight(rng, 1280, k, 4, 64, (experts,)), make_weight(rng, k, 640, 4, 64, (experts,))
+    g, d = ops.QuantizedWeight.from_numpy(*gate_up, 64, 4), ops.QuantizedWeight.from_numpy(*down, 64, 4)
+    g.set_expert_stream_kernel(6)
+    x, rows = DeviceBuffer.from_numpy(make_x(rng, tokens, k)), DeviceBuffer.from_numpy(make_x(rng, 13, k))
+    picks = DeviceBuffer.from_numpy(rng.integers(0, experts, size=20).astype(np.uint32))
+    logits = DeviceBuffer.from_numpy(rng.standard_normal((tokens, experts)).astype(np.float32))
+    stream = rt.Stream()
+    outs = [DeviceBuffer(s, rt.F16) for s in ((13, n), (20, 2, n), (tokens, k))]
+
+    def calls(outs):
+        ops.affine_quantized_matmul_batched(rows, wd, stream=stream, kernel=rt.KERNEL_QMV_RING, out=outs[0])
+        ops.gather_qmm(x, *stacked, picks, 20, 2, n, k, experts, 64, stream=stream, kernel=rt.GATHER_SLOTS, out=outs[1])
+        ops.moe_forward(g, None, d, x, logits, 2, stream=stream, out=outs[2], noalloc=True)
+
+    calls(outs)
+    stream.sync()
+    eager = [o.numpy().copy() for o in outs]
+    with rt.Graph.record(stream) as graph:
+        calls(outs)
+    for _ in range(3):
+        for o in outs:
+            rt.check(rt.lib().rmlx_hip_memcpy_h2d(o.ptr, np.full(o.shape, np.nan, np.float16).ctypes.data, o.nbytes, None))
+        graph.launch(stream)
+        stream.sync()
+        for o, e in zip(outs, eager):
+            assert np.array_equal(o.numpy().view(np.uint16), e.view(np.uint16))
+        calls(outs)
+        stream.sync()
