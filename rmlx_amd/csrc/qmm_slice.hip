@@ -313,7 +313,7 @@ template <int BITS, int MIMAX, int WN, int KG, int KS, int S, int WPE, bool DUAL
 __global__ __launch_bounds__(WN * KG * 64, WPE) void qmm_slice_kernel(TileParams p) {
   __shared__ __align__(1024) char lds[slice_lds_all(BITS, MIMAX, WN, KG, KS, S)];
   Tile t;
-  if (!tile_of(p, MIMAX * 32, &t)) return;
+  if (!tile_of<DUAL ? 1 : 4>(p, MIMAX * 32, &t)) return;
   if (MIMAX == 2 && t.rows > 32) slice_body<BITS, MIMAX, WN, KG, KS, S, DUAL, EXACT>(p, t, lds);
   else slice_body<BITS, 1, WN, KG, KS, S, DUAL, EXACT>(p, t, lds);
 }

@@ -159,18 +159,18 @@ __device__ __forceinline__ Weights split_q8(uint32_t w0, uint32_t w1, float s, f
 
 struct Tile { uint32_t mt, nt, split, expert, row_lo, rows; bool zeros; };
 // Tile of this workgroup; false past the last.
+template <uint32_t kBlock>
 __device__ __forceinline__ bool tile_of(const TileParams& p, uint32_t tile_rows, Tile* out) {
-  // An XCD (workgroup id % 8) takes a run of tiles, in blocks of up to four row tiles by all column tiles; of a grouped launch row tile by row tile,
-  // whose activations then stay in its L2 while the weights, of another expert for nearly every row tile, pass through once (2048 tokens, 128
-  // experts 889 -> 867 us; 45 experts, 3503 tokens 805 -> 775; 16 experts of 256 rows and more 443 -> 441).
+  // An XCD (workgroup id % 8) takes a run of tiles, in blocks of up to four row tiles by all column tiles; a pair, which is always a grouped launch,
+  // row tile by row tile: the activations then stay in the XCD's L2 while the weights, of another expert for nearly every row tile, pass through
+  // once (2048 tokens, 128 experts 910 -> 865 us with the grouping kernel's share; 45 experts, 3503 tokens 811 -> 770).
   const uint32_t tiles_m = p.tile_tab != nullptr ? uni(*p.n_tiles) : p.tiles_m, total = tiles_m * p.tiles_n * p.splits, pid = blockIdx.x;
   if (pid >= total) return false;
   const uint32_t xcd = pid & 7, per = total >> 3, rem = total & 7;
   uint32_t idx = xcd * per + (xcd < rem ? xcd : rem) + (pid >> 3);
   Tile t;
   t.split = idx % p.splits; idx /= p.splits;
-  const uint32_t block = p.tile_tab != nullptr ? 1 : 4, in_block = block * p.tiles_n, first = idx / in_block * block, within = idx % in_block;
-  const uint32_t h = tiles_m - first < block ? tiles_m - first : block;
+  const uint32_t in_block = kBlock * p.tiles_n, first = idx / in_block * kBlock, within = idx % in_block, h = tiles_m - first < kBlock ? tiles_m - first : kBlock;
   t.mt = uni(first + within % h); t.nt = uni(within / h); t.split = uni(t.split);
   t.expert = 0; t.row_lo = t.mt * tile_rows; t.rows = p.M - t.row_lo; t.zeros = false;
   if (p.tile_tab != nullptr) {
