@@ -20,6 +20,7 @@
 //
 // (the device code below loads with inline assembly where the compiler would wait for the loads of a slot before it lets the next one out;
 // the counts behind wait_but are those of the loads that this kernel issues, in order)
+#include <cstddef>
 #include <type_traits>
 #include <utility>
 
@@ -134,6 +135,135 @@ struct Ring {
   static_assert(kLds <= 160 * 1024 && kSBytes <= 4096, "LDS, one load a wave for the scales");
 };
 
+// An equal share of all (chunk, weight row) pairs for every workgroup, or, where that is hardly more work for it, of one chunk (a second
+// one starts over with empty rings and other activations: about 4 us, in which a CU streams 100 KB).
+__device__ __forceinline__ void take_share(uint32_t chunks, uint32_t N, uint32_t slack, uint32_t* pos, uint32_t* end) {
+  const uint32_t all = chunks * N, each = all / gridDim.x, more = all - each * gridDim.x, b = blockIdx.x;
+  const uint32_t per = chunks == 0 ? 0 : gridDim.x / chunks, part = per == 0 ? 0 : N / per, rest = N - part * per;
+  if (per != 0 && part <= each + slack) {
+    const uint32_t c = b / per, i = b - c * per;
+    *pos = c * N + i * part + (i < rest ? i : rest);
+    *end = c < chunks ? *pos + part + (i < rest ? 1 : 0) : *pos;
+  } else {
+    *pos = b * each + (b < more ? b : more);
+    *end = *pos + each + (b < more ? 1 : 0);
+  }
+  *pos = uni(*pos);
+  *end = uni(*end);
+}
+
+// The kernel's arguments as they lie in memory.
+struct RingArgs {
+  const uint32_t* w0; const __half* s0; const __half* b0; const char* x;
+  uint32_t N, K, M, geometry, share, over, cpr_inv;
+  RingParams p;
+};
+static_assert(offsetof(RingArgs, geometry) == 44 && offsetof(RingArgs, p) == 64, "the kernel's parameters, one behind another");
+// (scale * q + bias) * x of a row in f32: the parts of it in which a value, a scale or a bias is not finite, or all of it.
+template <int BITS, int GS>
+__device__ __forceinline__ float unbounded_sum(const char* w, const __half* s, const __half* b, const char* x, int32_t x_dtype, uint32_t K, bool whole) {
+  float sum = 0.f;
+#pragma unroll 1
+  for (uint32_t k = 0; k < K && sum == sum; k += 8) {
+    const float sc = (float)s[k / GS], bi = (float)b[k / GS];
+    bool odd = whole || !__builtin_isfinite(sc) || !__builtin_isfinite(bi);
+    h8 v;
+    if (x_dtype == RMLX_DTYPE_F32) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = (_Float16)reinterpret_cast<const float*>(x)[k + e];
+    } else {
+      u4 d = *reinterpret_cast<const u4*>(x + k * 2);
+      if (x_dtype == RMLX_DTYPE_BF16) d = q4::bf16x8_to_f16(d);
+      v = __builtin_bit_cast(h8, d);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) odd = odd || !__builtin_isfinite((float)v[e]);
+    if (!odd) continue;
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(w + k * BITS / 8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t i = BITS == 4 ? q[0] >> (4 * e) & 15u : q[e >> 2] >> (8 * (e & 3)) & 255u;
+      sum = fmaf(fmaf((float)i, sc, bi), (float)v[e], sum);
+    }
+  }
+  return sum;
+}
+// Offsets and biases of both signs make a NaN of an infinite activation, (1024 + q) inf - 1024 inf, where the sum of the products is an
+// infinity (f32 and bf16 values past the range of f16 are infinities here too).  A wave that has stored a result that is not finite comes
+// here at its end and goes over its results once more: those whose sum of products is not finite are stored anew.  The arguments are
+// read again, so that nothing is kept for this (as scalar registers they made the others spill), and what it costs the others is a
+// multiply-add for each result: 13 rows, 14336 x 4096, 8-bit 14.8 -> 14.9 us, 128 tokens through 128 experts 254.4 -> 254.8.
+typedef const __attribute__((address_space(1))) RingArgs* RingArgsPtr;
+template <int BITS, int GS, int H, int MODE>
+__device__ __forceinline__ void store_unbounded(uint32_t chunks, uint32_t seg_row, uint32_t seg_rows, uint32_t seg_expert) {
+  auto args = []() -> RingArgsPtr {                       // (from memory, each time, into vector registers)
+    auto a = (RingArgsPtr)(const void*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+v"(a));
+    return a;
+  };
+  const RingArgsPtr a = args();
+  const uint32_t N = uni(a->N), geometry = a->geometry, tid = threadIdx.x, wave = uni(tid >> 6);
+  const int32_t x_dtype = geometry >> 6 & 3;
+  // (which results are this lane's: as in the kernel)
+  const uint32_t nt_log2 = H == 2 ? 0 : geometry >> 4 & 3, w_log2 = nt_log2 < 2 ? nt_log2 : 2, it = wave * 64 + (tid & 63), ot = it >> (8 - w_log2);
+  const uint32_t l = it >> (2 - w_log2) & 63, out_m = (l >> 4) * 4 + ((it & ((4 >> w_log2) - 1)) << w_log2), out_c = (ot << 4) + (l & 15);
+  uint32_t pos, end, seg = 0;
+  if (MODE != DENSE) take_share(MODE == GATHER ? uni(chunks) : uni(*a->p.n_chunks), N, uni(a->p.slack), &pos, &end);
+  else {
+    const uint32_t share = a->share, over = a->over;
+    pos = uni(blockIdx.x * share + (blockIdx.x < over ? blockIdx.x : over));
+    end = uni(pos + share + (blockIdx.x < over ? 1 : 0));
+  }
+#pragma unroll 1
+  do {
+    const RingArgsPtr a = args();
+    const uint32_t chunk = MODE == DENSE ? blockIdx.y : pos / N, r0 = MODE == DENSE ? pos : pos - chunk * N, r1 = end - pos < N - r0 ? r0 + (end - pos) : N;
+    pos += r1 - r0;
+    uint32_t expert = 0, row0 = chunk * 16, rows = a->M - row0 < 16u ? a->M - row0 : 16u;
+    if constexpr (MODE == GATHER) {
+      expert = __builtin_amdgcn_readlane(seg_expert, seg * 16);
+      rows = expert == kNoExpert ? 0u : __builtin_amdgcn_readlane(seg_rows, seg * 16);
+    } else if (MODE != DENSE) {
+      const uint32_t* const t = a->p.chunk_tab + 3 * chunk;
+      expert = uni(t[0]); row0 = uni(t[1]); rows = uni(t[2]);
+      if ((rows >> 31) != 0) rows = 0;                    // (zeros)
+    }
+#pragma unroll 1
+    for (uint32_t e = 0; e < 1u << w_log2; ++e) {
+      uint32_t m = row0 + out_m + e, from = m;
+      if constexpr (MODE == GATHER) m = from = __builtin_amdgcn_ds_bpermute((seg * 16 + out_m + e) * 4, seg_row);
+      const bool mine = out_m + e < rows && ot < 1u << nt_log2;
+      const RingArgsPtr a = args();
+      if (MODE != GATHER && MODE != DENSE && a->p.row_map != nullptr && mine) from = a->p.row_map[m];
+      const char* const x = a->x + (uint64_t)from * (a->K << (x_dtype == RMLX_DTYPE_F32 ? 2 : 1));
+#pragma unroll 1
+      for (uint32_t r = mine ? r0 + out_c : r1; r < r1; r += 16u << nt_log2) {
+        auto sum_of = [&](bool up, bool whole) {
+          const RingArgsPtr a = args();
+          const uint32_t K = a->K;
+          const uint64_t at = (uint64_t)r * (K / GS) + expert * a->p.estride_s;
+          const char* const w = reinterpret_cast<const char*>(up ? a->p.w1 : a->w0) + expert * a->p.estride_w * 4 + (uint64_t)r * (K * BITS / 8);
+          return unbounded_sum<BITS, GS>(w, (up ? a->p.s1 : a->s0) + at, (up ? a->p.b1 : a->b0) + at, x, x_dtype, K, whole);
+        };
+        float v = sum_of(false, false);
+        if constexpr (MODE == PAIR) {
+          float u = sum_of(true, false);
+          const bool v_ok = __builtin_isfinite(v), u_ok = __builtin_isfinite(u);
+          if (v_ok && u_ok) continue;
+          if (v_ok) v = sum_of(false, true);
+          if (u_ok) u = sum_of(true, true);
+          v = q4::silu_f(v) * u;
+        } else if (__builtin_isfinite(v)) continue;
+        const RingArgsPtr a = args();
+        const uint64_t o = (uint64_t)m * a->p.ld_out + r;
+        if (MODE != GATHER && a->p.out_f32) static_cast<float*>(a->p.out)[o] = v;
+        else static_cast<__half*>(a->p.out)[o] = __float2half(v);
+      }
+    }
+    ++seg;
+  } while (MODE != DENSE && pos < end);
+}
+
 template <int BITS, int GS, int U, int H, int MODE>
 __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint32_t N,
                                                                   uint32_t K, uint32_t M, uint32_t geometry, uint32_t share, uint32_t over, uint32_t cpr_inv,
@@ -155,23 +285,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
   uint32_t lane = tid & 63;
   const uint32_t KS = geometry & 15, nt_log2 = H == 2 ? 0 : geometry >> 4 & 3, tw = geometry >> (8 + 3 * wave) & 7, kp = wave - tw * KS, NT = 1u << nt_log2;
   const int32_t x_dtype = geometry >> 6 & 3;
-  // An equal share of all (chunk, weight row) pairs for every workgroup, or, where that is hardly more work for it, of one chunk (a second
-  // one starts over with empty rings and other activations: about 4 us, in which a CU streams 100 KB).
-  uint32_t pos = 0, end = 0;
-  auto take_share = [&](uint32_t chunks) {
-    const uint32_t all = chunks * N, each = all / gridDim.x, more = all - each * gridDim.x, b = blockIdx.x;
-    const uint32_t per = chunks == 0 ? 0 : gridDim.x / chunks, part = per == 0 ? 0 : N / per, rest = N - part * per;
-    if (per != 0 && part <= each + p.slack) {
-      const uint32_t c = b / per, i = b - c * per;
-      pos = c * N + i * part + (i < rest ? i : rest);
-      end = c < chunks ? pos + part + (i < rest ? 1 : 0) : pos;
-    } else {
-      pos = b * each + (b < more ? b : more);
-      end = pos + each + (b < more ? 1 : 0);
-    }
-    pos = uni(pos);
-    end = uni(end);
-  };
+  uint32_t pos = 0, end = 0, gather_chunks = 0;
   // GATHER: every workgroup groups the entries by expert itself (a launch of its own for that costs more: 3 us against about 1.5), a stable
   // counting sort over at most 256 of them, all waves alike behind the ranks.  A chunk is 16 rows of one expert's entries one behind another;
   // a workgroup's share lies in at most four of those (all fit in two times the workgroups): lane 16 s + i keeps row i of the s-th.
@@ -213,7 +327,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
       const uint32_t t = __shfl_up(inc, o, 64);
       if ((int)lane >= o) inc += t;
     }
-    take_share(uni(__builtin_amdgcn_readlane(inc, 63)));
+    gather_chunks = __shfl(inc, 63, 64);
+    take_share(uni(gather_chunks), N, p.slack, &pos, &end);
     const uint32_t c0 = pos / N;
     if (lane < 16) mine[lane] = 0;
     uint32_t base = inc - own;
@@ -238,7 +353,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
     wait_lds();
     q4::lds_barrier();                                    // (the rings may be filled)
   } else if (MODE != DENSE) {
-    take_share(uni(*p.n_chunks));
+    take_share(uni(*p.n_chunks), N, p.slack, &pos, &end);
   } else {
     pos = uni(blockIdx.x * share + (blockIdx.x < over ? blockIdx.x : over));
     end = uni(pos + share + (blockIdx.x < over ? 1 : 0));
@@ -247,6 +362,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
   const uint32_t lds0 = uni((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds);
   if (pos >= end) return;
   uint32_t seg = 0;
+  float spoiled = 0.f;                                    // NaN once the lane has stored a result that is not finite
 
   do {
     // (what follows from these is worked out where it is used: kept across segments it costs more registers than there are, and the first
@@ -602,6 +718,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
       }
       const uint32_t c = (DUAL ? tm >> 1 : tm) << (4 + nt_log2);
       if (out_rows == 0 || c + out_c >= r1 - r0) return;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < w) spoiled = fmaf(v[e], 0.f, spoiled);
       if constexpr (MODE == GATHER) {
         __half* q = static_cast<__half*>(p.out) + r0 + out_c + c;
 #pragma unroll
@@ -667,6 +786,9 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
     if (MODE != DENSE) q4::lds_barrier();  // (the rings are free again)
     ++seg;
   } while (MODE != DENSE && pos < end);
+  if (__builtin_amdgcn_ballot_w64(spoiled != spoiled) != 0) {
+    store_unbounded<BITS, GS, H, MODE>(gather_chunks, seg_row, seg_rows, seg_expert);
+  }
 }
 
 struct RingLaunch { const QmvArgs* a; uint32_t geometry, share, over, chunks, cpr_inv; RingParams p; };

@@ -187,6 +187,100 @@ def test_rows_with_infinities_leave_the_others_alone(hip):
         assert np.isnan(out[8]).all() and not np.isfinite(out[3]).any() and not np.isfinite(out[12]).any()
 
 
+def _unbounded(x, w, gs, bits):
+    """Reference of rows with infinities: NaN, +-inf by the signs of the weights that they meet (others: any finite value)."""
+    words, scales, biases = w
+    q = (words[..., None] >> np.arange(0, 32, bits, dtype=np.uint32)) & np.uint32((1 << bits) - 1)
+    q = q.reshape(words.shape[0], -1)
+    wide = scales.astype(np.float64).repeat(gs, axis=1) * q + biases.astype(np.float64).repeat(gs, axis=1)
+    odd = ~np.isfinite(x).all(axis=0)
+    with np.errstate(invalid="ignore"):
+        return sum((np.outer(x[:, k], wide[:, k]) for k in np.flatnonzero(odd)), np.zeros((x.shape[0], wide.shape[0])))
+
+
+def _assert_same_class(out, ref):
+    for of in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(of(out), of(ref)), (of.__name__, int(of(out).sum()), int(of(ref).sum()))
+
+
+@pytest.mark.parametrize("bits,gs,n,k,dtype", [(4, 32, 515, 2880, "f16"), (4, 32, 515, 4096, "bf16"), (4, 64, 5003, 704, "f32"), (4, 64, 515, 4096, "f16"),
+                                               (4, 64, 515, 6144, "bf16"), (4, 128, 5003, 1408, "f16"), (4, 128, 515, 8192, "f16"), (8, 32, 515, 1504, "f16"),
+                                               (8, 32, 515, 4096, "f32"), (8, 64, 515, 2880, "bf16"), (8, 64, 5003, 512, "f16"), (8, 128, 515, 4096, "f16")])
+@pytest.mark.parametrize("m", [13, 18])
+def test_infinite_activations_of_a_matrix(hip, bits, gs, n, k, dtype, m):
+    """A row with an infinite value, or one that f16 does not hold, is what the sum of its products is: an infinity of the weight's sign, a NaN
+    where that is zero or where two of them cancel."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, bits, gs)
+    wd = ops.QuantizedWeight.from_numpy(*w, gs, bits)
+    x = make_x(rng, m, k).astype(np.float32)
+    x[3, 7] = x[12, 0] = x[m - 1, k - 1] = np.inf if dtype == "f16" else 1e6
+    x[4, k // 2] = x[12, k // 3] = -np.inf
+    x[8, 5] = np.nan
+    x[8, 6] = np.inf
+    raw = model.f32_to_bf16_bits(x) if dtype == "bf16" else x.astype(np.float16 if dtype == "f16" else np.float32)
+    xd = rt.DeviceBuffer.from_numpy(raw, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(raw)
+    with np.errstate(over="ignore"):
+        x16 = x_as_f64(raw, dtype).astype(np.float16)
+    odd = ~np.isfinite(x16).all(axis=1)
+    out = ops.affine_quantized_matmul_batched(xd, wd, kernel=rt.KERNEL_QMV_RING).numpy()
+    _assert_same_class(out, _unbounded(x16.astype(np.float64), w, gs, bits))
+    assert_close(out[~odd], model.qmm(x16[~odd].astype(np.float64), *w, gs, bits))
+
+
+@pytest.mark.parametrize("gs,n,k,rows", [(64, 515, 4096, 3), (32, 300, 1056, 16), (128, 1001, 1408, 5)])
+def test_infinite_activations_of_a_gather(hip, gs, n, k, rows):
+    from rmlx_amd import ops, runtime as rt
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(n)
+    batch, experts = 37, 4
+    w = make_weight(rng, n, k, 4, gs, (experts,))
+    idx = rng.integers(0, experts, size=batch).astype(np.uint32)
+    idx[[3, 29]] = experts, 0xFFFFFFFF  # zeros, whatever their rows hold
+    x = make_x(rng, batch * rows, k).reshape(batch, rows, k)
+    x[3], x[0, 1, 9], x[11, 0, k - 1], x[36, rows - 1, 40] = np.inf, -np.inf, np.inf, np.inf
+    stream = rt.Stream()
+    out = ops.gather_qmm(DeviceBuffer.from_numpy(x), *(DeviceBuffer.from_numpy(a) for a in w), DeviceBuffer.from_numpy(idx), batch, rows, n, k, experts, gs,
+                         stream=stream, kernel=rt.GATHER_SLOTS)
+    stream.sync()
+    out = out.numpy().reshape(batch, rows, n)
+    assert not out[[3, 29]].any()
+    for i in [i for i in range(batch) if i not in (3, 29)]:
+        _assert_same_class(out[i], _unbounded(x[i].astype(np.float64), tuple(a[idx[i]] for a in w), gs, 4))
+
+
+@pytest.mark.parametrize("bits,gs,hidden,inter,fused", [(4, 64, 1024, 1088, True), (4, 32, 1056, 576, False), (4, 128, 4224, 512, True), (8, 64, 576, 2240, False)])
+def test_infinite_activations_of_a_routed_block(hip, bits, gs, hidden, inter, fused):
+    """Positive gate and up weights make an infinite hidden row of an infinite activation, down weights of one sign a row infinities of that sign."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(hidden)
+    experts, tokens = 6, 40
+
+    def weights(n, k):
+        words, scales, _ = make_weight(rng, n, k, bits, gs, (experts,))
+        return words, scales, scales.copy()
+
+    gate, up, down = weights(inter, hidden), weights(inter, hidden), weights(hidden, inter)
+    for a in down[1:]:
+        a[:, 1::2] *= -1
+    d = ops.QuantizedWeight.from_numpy(*down, gs, bits)
+    if fused:
+        g, u = ops.QuantizedWeight.from_numpy(*(np.concatenate(p, axis=1) for p in zip(gate, up)), gs, bits), None
+    else:
+        g, u = (ops.QuantizedWeight.from_numpy(*w, gs, bits) for w in (gate, up))
+    g.set_expert_stream_kernel(6)
+    x = (make_x(rng, tokens, hidden) * np.float16(0.01)).astype(np.float16)
+    ld = rt.DeviceBuffer.from_numpy(rng.standard_normal((tokens, experts)).astype(np.float32))
+    clean = ops.moe_forward(g, u, d, rt.DeviceBuffer.from_numpy(x), ld, 2).numpy()
+    odd = [0, 17, tokens - 1]
+    x[odd, [3, hidden // 2, hidden - 1]] = np.inf
+    out = ops.moe_forward(g, u, d, rt.DeviceBuffer.from_numpy(x), ld, 2).numpy()
+    rest = [t for t in range(tokens) if t not in odd]
+    assert np.isfinite(clean).all() and np.array_equal(out[rest].view(np.uint16), clean[rest].view(np.uint16))
+    assert np.isposinf(out[odd][:, 0::2]).all() and np.isneginf(out[odd][:, 1::2]).all()
+
+
 def test_recorded_calls_replay_bit_for_bit(hip):
     """A matrix, a gather and a routed block recorded into one graph, with eager work between the replays."""
     from rmlx_amd import ops, runtime as rt
