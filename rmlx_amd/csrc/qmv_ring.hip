@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
     auto groups_of = [&](int h) -> uint32_t { const uint32_t k0 = (h * KS + kp) * KU; return k0 < K ? (K - k0) / GS : 0; };
     auto request_x = [&]() {
       repeat<H>([&](auto h) {
-        const uint32_t groups = groups_of(h), base = x_lane + (groups != 0 ? (h * KS + kp) * KU * 2 : kOutside);
+        const uint32_t groups = groups_of(h), base = groups != 0 ? x_lane + (h * KS + kp) * KU * 2 : kOutside;  // (never a sum with x_lane: it wraps)
         if (groups >= (uint32_t)NG || groups == 0) {
           repeat<U>([&](auto u) {
             repeat<kProducts>([&](auto j) { load16<k_of<BITS, GS>(decltype(u)::value, decltype(j)::value) * 2>(xv[h][u][j], base, xr); });

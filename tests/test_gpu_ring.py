@@ -281,6 +281,26 @@ def test_infinite_activations_of_a_routed_block(hip, bits, gs, hidden, inter, fu
     assert np.isposinf(out[odd][:, 0::2]).all() and np.isneginf(out[odd][:, 1::2]).all()
 
 
+def test_rows_beyond_a_gigabyte_of_activations(hip):
+    """K = 2240 in two slots leaves a wave without k in the second: its loads stay outside the buffer wherever the row begins."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(12)
+    hidden, inter, experts, tokens = 2240, 512, 2, 239900
+    assert tokens * hidden * 2 > 1 << 30
+    gate, up = (make_weight(rng, inter, hidden, 8, 64, (experts,)) for _ in range(2))
+    down = make_weight(rng, hidden, inter, 8, 64, (experts,))
+    g, u, d = (ops.QuantizedWeight.from_numpy(*w, 64, 8) for w in (gate, up, down))
+    g.set_expert_stream_kernel(6)
+    x = np.resize(make_x(rng, 2000, hidden), (tokens, hidden))
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    out = rt.DeviceBuffer((tokens, hidden), rt.F16)
+    ops.moe_forward(g, u, d, rt.DeviceBuffer.from_numpy(x), rt.DeviceBuffer.from_numpy(logits), 1, out=out)
+    some = np.r_[np.arange(0, tokens, 30011), np.arange(tokens - 250, tokens)]
+    idx, w, _, _ = model.topk_route(logits[some], 1)
+    ref = model.moe_forward(x[some], idx, w, gate, up, down, 64, 1, bits=8)
+    assert_close(out.numpy()[some], ref)
+
+
 def test_recorded_calls_replay_bit_for_bit(hip):
     """A matrix, a gather and a routed block recorded into one graph, with eager work between the replays."""
     from rmlx_amd import ops, runtime as rt
