@@ -87,19 +87,22 @@ __device__ __forceinline__ h8 bytes8(uint32_t w0, uint32_t w1) {
   o.w = __builtin_amdgcn_perm(0x64646464u, w1, 0x04030402u);
   return __builtin_bit_cast(h8, o);
 }
-// direct loads into LDS at base + AT (of both addresses: the lane's offset is given less AT)
-template <int AT>
-__device__ __forceinline__ void dma16_next(uint32_t off, u4 r) {
-  static_assert(AT >= 0 && AT < 4096, "12 bits of offset");
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 nt lds" ::"v"(off), "s"(r), "n"(AT) : "memory");
+// 16 bytes per lane and load straight into LDS, one load behind another from `lds` on (the instruction's offset counts for both addresses, so
+// the lanes' are given less 0, 1024, 2048 .. bytes).  One statement: nothing may come between m0 and the loads that use it.
+__device__ __forceinline__ void dma_slot(uint32_t lds, const uint32_t (&off)[3], u4 r) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen nt lds\n\tbuffer_load_dwordx4 %2, %4, 0 offen offset:1024 nt lds\n\t"
+               "buffer_load_dwordx4 %3, %4, 0 offen offset:2048 nt lds" ::"s"(lds), "v"(off[0]), "v"(off[1]), "v"(off[2]), "s"(r) : "memory", "m0");
 }
-__device__ __forceinline__ void dma16_plain(uint32_t off, u4 r) { asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(r) : "memory"); }
+__device__ __forceinline__ void dma_slot(uint32_t lds, const uint32_t (&off)[4], u4 r) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %5, 0 offen nt lds\n\tbuffer_load_dwordx4 %2, %5, 0 offen offset:1024 nt lds\n\t"
+               "buffer_load_dwordx4 %3, %5, 0 offen offset:2048 nt lds\n\tbuffer_load_dwordx4 %4, %5, 0 offen offset:3072 nt lds"
+               ::"s"(lds), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(r) : "memory", "m0");
+}
 // the buffer from byte `by` on (scalar: the lanes' offsets stay as they are)
 __device__ __forceinline__ u4 later(u4 r, uint32_t by) {
   const uint64_t a = ((uint64_t)r.y << 32 | r.x) + by;
   return (u4){uni((uint32_t)a), uni((uint32_t)(a >> 32)), uni(r.z - by), r.w};
 }
-__device__ __forceinline__ void set_m0(uint32_t lds) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" ::"s"(lds) : "memory"); }
 template <int AT>
 __device__ __forceinline__ void load16(u4& d, uint32_t off, u4 r) {
   static_assert(AT >= 0 && AT < 4096, "12 bits of offset");
@@ -460,7 +463,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
       uint32_t r = i0 * cpr_inv >> 20, c = i0 - r * cpr;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        w_from[u] = r < 16u << nt_log2 ? r * row_bytes + ((c ^ (r >> kshift & kmask)) * 16) - u % 4 * 1024 : kOutside;  // (the load adds it)
+        w_from[u] = r < 16u << nt_log2 ? r * row_bytes + ((c ^ (r >> kshift & kmask)) * 16) - u * 1024 : kOutside;  // (the load adds it)
         r += dr;
         c += dc;
         if (c >= cpr) { c -= cpr; ++r; }
@@ -487,14 +490,11 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
       const u4 wr = later(up ? wr1 : wr0, (t << (4 + nt_log2)) * row_bytes + (H == 1 ? 0 : iq % H * cpr * 16));
       if (first && has_s) {
         const uint32_t sa = scales_at(t);
-        set_m0(lds0 + C::oScales + splace * C::kScales + (wave < 4 ? 0 : C::kSBytes) + (wave & 3) * 1024);
-        dma16_plain(sa < s_last ? s_from : s_from_last, later(up ? sr1 : sr0, sa < s_last ? sa : s_last));
+        dma16(lds0 + C::oScales + splace * C::kScales + (wave < 4 ? 0 : C::kSBytes) + (wave & 3) * 1024, sa < s_last ? s_from : s_from_last,
+              later(up ? sr1 : sr0, sa < s_last ? sa : s_last));
       }
       if (first) splace = splace == R - 1 ? 0 : splace + 1;
-      repeat<U>([&](auto u) {
-        if (decltype(u)::value % 4 == 0) set_m0(lds0 + iplace * C::kWBytes + (wave * U + decltype(u)::value) * 1024);
-        dma16_next<decltype(u)::value % 4 * 1024>(w_from[u], wr);
-      });
+      dma_slot(lds0 + iplace * C::kWBytes + wave * U * 1024, w_from, wr);
       iplace = iplace == R - 1 ? 0 : iplace + 1;
       ++iq;
     };
