@@ -342,7 +342,8 @@ int32_t rmlx_hip_qweight_set_gemm_layout(rmlx_qweight* qw, void* dst_dev, size_t
  * kernel 2 for the down projection (4-bit weights, group size 64; other weights keep kernel 1), 5 = as 4 with the gate / up
  * projection in two launches, the experts split by their row count: up to 8 rows on kernel 1, more on kernel 3, so every
  * expert is streamed once whatever the largest row count, 6 = the slot-streaming kernel for the three projections, chunks of 16
- * rows (4- and 8-bit weights, every group size; experts that it does not take keep the library's choice; the routed block only),
+ * rows (4- and 8-bit weights, every group size; experts that it does not take keep the library's choice; the routed block only;
+ * unlike 1 to 5 at every batch size, unless a GEMM threshold other than the default says otherwise),
  * 0 = the library's choice (6 for a few rows per expert where many weights are picked, else 4; 5 from 6 rows per expert on
  * average).  Kernel 3 streams an expert with 9 to 16 rows once instead of twice and is the fastest of the four from 7 rows
  * per expert on average - as long as no expert of the batch has more than 16 rows, so it is for callers whose router bounds

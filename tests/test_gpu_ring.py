@@ -281,6 +281,47 @@ def test_infinite_activations_of_a_routed_block(hip, bits, gs, hidden, inter, fu
     assert np.isposinf(out[odd][:, 0::2]).all() and np.isneginf(out[odd][:, 1::2]).all()
 
 
+def test_pinned_block_keeps_the_callers_gemm_threshold(hip):
+    """Pinned, it runs batches of every size; from a threshold of the caller's on the grouped GEMM does, as behind every other kernel."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(13)
+    experts, hidden, tokens = 8, 1024, 96
+    g, d = (ops.QuantizedWeight.from_numpy(*make_weight(rng, n, hidden, 4, 64, (experts,)), 64, 4) for n in (2 * hidden, hidden))
+    xd = rt.DeviceBuffer.from_numpy(make_x(rng, tokens, hidden))
+    ld = rt.DeviceBuffer.from_numpy(rng.standard_normal((tokens, experts)).astype(np.float32))
+
+    def run(kind, min_rows):
+        g.set_expert_stream_kernel(kind)
+        prev = g.set_expert_gemm_min_rows(min_rows) if min_rows is not None else None
+        out = ops.moe_forward(g, None, d, xd, ld, 2).numpy().view(np.uint16)
+        if prev is not None:
+            g.set_expert_gemm_min_rows(prev)
+        return out
+
+    slots, gemm = run(6, 0), run(1, 24)
+    assert not np.array_equal(slots, gemm)
+    assert np.array_equal(run(6, 24), gemm)  # 24 rows per expert
+    assert np.array_equal(run(6, 25), slots) and np.array_equal(run(6, None), slots)
+
+
+def test_more_chunks_than_a_grid_has_rows(hip):
+    """65552 chunks at most: their number is no grid dimension here."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(14)
+    hidden, inter, experts, tokens = 512, 512, 16, 131072
+    gate, up, down = (make_weight(rng, n, 512, 4, 64, (experts,)) for n in (inter, inter, hidden))
+    g, u, d = (ops.QuantizedWeight.from_numpy(*w, 64, 4) for w in (gate, up, down))
+    g.set_expert_stream_kernel(6)
+    x = make_x(rng, tokens, hidden)
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    stream, out, xd, ld = rt.Stream(), rt.DeviceBuffer((tokens, hidden), rt.F16), rt.DeviceBuffer.from_numpy(x), rt.DeviceBuffer.from_numpy(logits)
+    ops.moe_forward(g, u, d, xd, ld, 8, stream=stream, out=out)
+    stream.sync()
+    some = np.r_[np.arange(0, tokens, 5003), np.arange(tokens - 40, tokens)]
+    idx, w, _, _ = model.topk_route(logits[some], 8)
+    assert_close(out.numpy()[some], model.moe_forward(x[some], idx, w, gate, up, down, 64, 8))
+
+
 def test_rows_beyond_a_gigabyte_of_activations(hip):
     """K = 2240 in two slots leaves a wave without k in the second: its loads stay outside the buffer wherever the row begins."""
     from rmlx_amd import ops, runtime as rt
