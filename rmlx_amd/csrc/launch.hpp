@@ -27,6 +27,7 @@ inline hipError_t& launch_error() {
 inline hipError_t take_launch_error() {
   const hipError_t e = launch_error();
   launch_error() = hipSuccess;
+  if (e != hipSuccess) (void)hipGetLastError();  // (the runtime keeps it too, and other launches ask the runtime)
   return e;
 }
 
