@@ -342,6 +342,19 @@ def test_rows_beyond_a_gigabyte_of_activations(hip):
     assert_close(out.numpy()[some], ref)
 
 
+@pytest.mark.parametrize("bits,gs,k,taken", [(4, 64, 8192, True), (4, 64, 8256, False), (4, 128, 8192, True), (4, 128, 8320, False), (4, 32, 4096, True), (4, 32, 4128, False),
+                                             (8, 64, 4096, True), (8, 64, 4160, False), (8, 128, 512, True), (8, 128, 384, False)])
+def test_refusals_name_the_limits_of_k(hip, bits, gs, k, taken):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(k)
+    w, x = ops.QuantizedWeight.from_numpy(*make_weight(rng, 128, k, bits, gs), gs, bits), rt.DeviceBuffer.from_numpy(make_x(rng, 2, k))
+    if taken:
+        ops.affine_quantized_matmul_batched(x, w, kernel=rt.KERNEL_QMV_RING)
+        return
+    with pytest.raises(rt.KernelError, match=r"512 <= K <= 8192 \(8-bit weights and group size 32: 4096\)"):
+        ops.affine_quantized_matmul_batched(x, w, kernel=rt.KERNEL_QMV_RING)
+
+
 def test_recorded_calls_replay_bit_for_bit(hip):
     """A matrix, a gather and a routed block recorded into one graph, with eager work between the replays."""
     from rmlx_amd import ops, runtime as rt
