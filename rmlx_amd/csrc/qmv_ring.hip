@@ -162,53 +162,56 @@ struct RingArgs {
   RingParams p;
 };
 static_assert(offsetof(RingArgs, geometry) == 44 && offsetof(RingArgs, p) == 64, "the kernel's parameters, one behind another");
-// (scale * q + bias) * x of a row in f32: the parts of it in which a value, a scale or a bias is not finite, or all of it.
+// 8 activations as the products take them
+__device__ __forceinline__ h8 x_piece(const char* x, int32_t x_dtype, uint32_t k) {
+  if (x_dtype == RMLX_DTYPE_F32) {
+    h8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (_Float16)reinterpret_cast<const float*>(x)[k + e];
+    return v;
+  }
+  const u4 d = *reinterpret_cast<const u4*>(x + k * 2);
+  return __builtin_bit_cast(h8, x_dtype == RMLX_DTYPE_BF16 ? q4::bf16x8_to_f16(d) : d);
+}
+// (scale * q + bias) * x of a row in f32, over n pieces of 8: those that the list names, or all of them.
 template <int BITS, int GS>
-__device__ __forceinline__ float unbounded_sum(const char* w, const __half* s, const __half* b, const char* x, int32_t x_dtype, uint32_t K, bool whole) {
+__device__ __forceinline__ float plain_sum(const char* w, const __half* s, const __half* b, const char* x, int32_t x_dtype, const uint16_t* list, uint32_t n) {
   float sum = 0.f;
 #pragma unroll 1
-  for (uint32_t k = 0; k < K && sum == sum; k += 8) {
+  for (uint32_t i = 0; i < n && sum == sum; ++i) {
+    const uint32_t k = (list != nullptr ? list[i] : i) * 8;
     const float sc = (float)s[k / GS], bi = (float)b[k / GS];
-    bool odd = whole || !__builtin_isfinite(sc) || !__builtin_isfinite(bi);
-    h8 v;
-    if (x_dtype == RMLX_DTYPE_F32) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = (_Float16)reinterpret_cast<const float*>(x)[k + e];
-    } else {
-      u4 d = *reinterpret_cast<const u4*>(x + k * 2);
-      if (x_dtype == RMLX_DTYPE_BF16) d = q4::bf16x8_to_f16(d);
-      v = __builtin_bit_cast(h8, d);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) odd = odd || !__builtin_isfinite((float)v[e]);
-    if (!odd) continue;
+    const h8 v = x_piece(x, x_dtype, k);
     const uint32_t* q = reinterpret_cast<const uint32_t*>(w + k * BITS / 8);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const uint32_t i = BITS == 4 ? q[0] >> (4 * e) & 15u : q[e >> 2] >> (8 * (e & 3)) & 255u;
-      sum = fmaf(fmaf((float)i, sc, bi), (float)v[e], sum);
+      const uint32_t v_q = BITS == 4 ? q[0] >> (4 * e) & 15u : q[e >> 2] >> (8 * (e & 3)) & 255u;
+      sum = fmaf(fmaf((float)v_q, sc, bi), (float)v[e], sum);
     }
   }
   return sum;
 }
 // Offsets and biases of both signs make a NaN of an infinite activation, (1024 + q) inf - 1024 inf, where the sum of the products is an
 // infinity (f32 and bf16 values past the range of f16 are infinities here too).  A wave that has stored a result that is not finite comes
-// here at its end and goes over its results once more: those whose sum of products is not finite are stored anew.  The arguments are
-// read again, so that nothing is kept for this (as scalar registers they made the others spill), and what it costs the others is a
-// multiply-add for each result: 13 rows, 14336 x 4096, 8-bit 14.8 -> 14.9 us, 128 tokens through 128 experts 254.4 -> 254.8.
+// here at its end and goes over the results of such rows once more, over the pieces of the row that are not finite (the others do not change
+// the sum; over all of it where there are none: then the weights are not finite); what is not finite is stored anew.  The arguments are read again, so that nothing
+// is kept for this (as scalar registers they made the others spill), and what it costs the others is a multiply-add for each result:
+// gather of 32 x 8 rows 40.6 -> 40.9 us, 13 rows, 14336 x 4096, 8-bit 59.2 -> 58.9 for four.  A row of 100001 x 4096 with one infinity
+// 45 -> 70 us, all 16 rows 142 (3.1 ms with every lane looking through its row for itself).
 typedef const __attribute__((address_space(1))) RingArgs* RingArgsPtr;
 template <int BITS, int GS, int H, int MODE>
-__device__ __forceinline__ void store_unbounded(uint32_t chunks, uint32_t seg_row, uint32_t seg_rows, uint32_t seg_expert) {
+__device__ __forceinline__ void store_unbounded(char* lds, bool spoiled, uint32_t chunks, uint32_t seg_row, uint32_t seg_rows, uint32_t seg_expert) {
   auto args = []() -> RingArgsPtr {                       // (from memory, each time, into vector registers)
     auto a = (RingArgsPtr)(const void*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+v"(a));
     return a;
   };
   const RingArgsPtr a = args();
-  const uint32_t N = uni(a->N), geometry = a->geometry, tid = threadIdx.x, wave = uni(tid >> 6);
+  const uint32_t N = uni(a->N), K = uni(a->K), geometry = uni(a->geometry), tid = threadIdx.x, wave = uni(tid >> 6), lane = tid & 63;
   const int32_t x_dtype = geometry >> 6 & 3;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(lds) + wave * 1024;  // (in the place of the rings, which nobody reads any more)
   // (which results are this lane's: as in the kernel)
-  const uint32_t nt_log2 = H == 2 ? 0 : geometry >> 4 & 3, w_log2 = nt_log2 < 2 ? nt_log2 : 2, it = wave * 64 + (tid & 63), ot = it >> (8 - w_log2);
+  const uint32_t nt_log2 = H == 2 ? 0 : geometry >> 4 & 3, w_log2 = nt_log2 < 2 ? nt_log2 : 2, it = wave * 64 + lane, ot = it >> (8 - w_log2);
   const uint32_t l = it >> (2 - w_log2) & 63, out_m = (l >> 4) * 4 + ((it & ((4 >> w_log2) - 1)) << w_log2), out_c = (ot << 4) + (l & 15);
   uint32_t pos, end, seg = 0;
   if (MODE != DENSE) take_share(MODE == GATHER ? uni(chunks) : uni(*a->p.n_chunks), N, uni(a->p.slack), &pos, &end);
@@ -222,7 +225,7 @@ __device__ __forceinline__ void store_unbounded(uint32_t chunks, uint32_t seg_ro
     const RingArgsPtr a = args();
     const uint32_t chunk = MODE == DENSE ? blockIdx.y : pos / N, r0 = MODE == DENSE ? pos : pos - chunk * N, r1 = end - pos < N - r0 ? r0 + (end - pos) : N;
     pos += r1 - r0;
-    uint32_t expert = 0, row0 = chunk * 16, rows = a->M - row0 < 16u ? a->M - row0 : 16u;
+    uint32_t expert = 0, row0 = chunk * 16, rows = uni(a->M) - row0 < 16u ? uni(a->M) - row0 : 16u;
     if constexpr (MODE == GATHER) {
       expert = __builtin_amdgcn_readlane(seg_expert, seg * 16);
       rows = expert == kNoExpert ? 0u : __builtin_amdgcn_readlane(seg_rows, seg * 16);
@@ -232,25 +235,39 @@ __device__ __forceinline__ void store_unbounded(uint32_t chunks, uint32_t seg_ro
       if ((rows >> 31) != 0) rows = 0;                    // (zeros)
     }
 #pragma unroll 1
-    for (uint32_t e = 0; e < 1u << w_log2; ++e) {
-      uint32_t m = row0 + out_m + e, from = m;
-      if constexpr (MODE == GATHER) m = from = __builtin_amdgcn_ds_bpermute((seg * 16 + out_m + e) * 4, seg_row);
-      const bool mine = out_m + e < rows && ot < 1u << nt_log2;
+    for (uint32_t i = 0; i < rows; ++i) {
+      const bool mine = i - out_m < 1u << w_log2 && ot < 1u << nt_log2;
+      if (__builtin_amdgcn_ballot_w64(mine && spoiled) == 0) continue;
       const RingArgsPtr a = args();
-      if (MODE != GATHER && MODE != DENSE && a->p.row_map != nullptr && mine) from = a->p.row_map[m];
-      const char* const x = a->x + (uint64_t)from * (a->K << (x_dtype == RMLX_DTYPE_F32 ? 2 : 1));
+      uint32_t m = row0 + i, from = m;
+      if constexpr (MODE == GATHER) m = from = __builtin_amdgcn_readlane(seg_row, seg * 16 + i);
+      else if (MODE != DENSE && a->p.row_map != nullptr) from = uni(a->p.row_map[m]);
+      const char* const x = a->x + (uint64_t)from * (K << (x_dtype == RMLX_DTYPE_F32 ? 2 : 1));
+      uint32_t n = 0;
+#pragma unroll 1
+      for (uint32_t k = 0; k < K; k += 512) {
+        bool odd = false;
+        if (k + lane * 8 < K) {
+          const h8 v = x_piece(x, x_dtype, k + lane * 8);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) odd = odd || !__builtin_isfinite((float)v[e]);
+        }
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(odd);
+        if (odd) list[n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0))] = (uint16_t)(k / 8 + lane);
+        n += (uint32_t)__builtin_popcountll(mask);
+      }
+      wait_lds();
 #pragma unroll 1
       for (uint32_t r = mine ? r0 + out_c : r1; r < r1; r += 16u << nt_log2) {
         auto sum_of = [&](bool up, bool whole) {
           const RingArgsPtr a = args();
-          const uint32_t K = a->K;
           const uint64_t at = (uint64_t)r * (K / GS) + expert * a->p.estride_s;
           const char* const w = reinterpret_cast<const char*>(up ? a->p.w1 : a->w0) + expert * a->p.estride_w * 4 + (uint64_t)r * (K * BITS / 8);
-          return unbounded_sum<BITS, GS>(w, (up ? a->p.s1 : a->s0) + at, (up ? a->p.b1 : a->b0) + at, x, x_dtype, K, whole);
+          return plain_sum<BITS, GS>(w, (up ? a->p.s1 : a->s0) + at, (up ? a->p.b1 : a->b0) + at, x, x_dtype, whole ? nullptr : list, whole ? K / 8 : n);
         };
-        float v = sum_of(false, false);
+        float v = sum_of(false, n == 0);
         if constexpr (MODE == PAIR) {
-          float u = sum_of(true, false);
+          float u = sum_of(true, n == 0);
           const bool v_ok = __builtin_isfinite(v), u_ok = __builtin_isfinite(u);
           if (v_ok && u_ok) continue;
           if (v_ok) v = sum_of(false, true);
@@ -786,9 +803,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
     if (MODE != DENSE) q4::lds_barrier();  // (the rings are free again)
     ++seg;
   } while (MODE != DENSE && pos < end);
-  if (__builtin_amdgcn_ballot_w64(spoiled != spoiled) != 0) {
-    store_unbounded<BITS, GS, H, MODE>(gather_chunks, seg_row, seg_rows, seg_expert);
-  }
+  if (__builtin_amdgcn_ballot_w64(spoiled != spoiled) != 0)
+    store_unbounded<BITS, GS, H, MODE>(lds, spoiled != spoiled, gather_chunks, seg_row, seg_rows, seg_expert);
 }
 
 struct RingLaunch { const QmvArgs* a; uint32_t geometry, share, over, chunks, cpr_inv; RingParams p; };

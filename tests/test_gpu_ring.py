@@ -229,6 +229,25 @@ def test_infinite_activations_of_a_matrix(hip, bits, gs, n, k, dtype, m):
     assert_close(out[~odd], model.qmm(x16[~odd].astype(np.float64), *w, gs, bits))
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+def test_infinite_scales_and_biases(hip, bits):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(bits)
+    n, k = 515, 704
+    words, scales, biases = make_weight(rng, n, k, bits, 64)
+    words |= 0x11111111 if bits == 4 else 0x01010101  # (no value of zero)
+    x = np.abs(make_x(rng, 5, k)) + np.float16(0.1)
+    run = lambda s, b: ops.affine_quantized_matmul_batched(rt.DeviceBuffer.from_numpy(x), ops.QuantizedWeight.from_numpy(words, s, b, 64, bits),
+                                                           kernel=rt.KERNEL_QMV_RING).numpy()
+    clean = run(scales, biases)
+    scales, biases = scales.copy(), biases.copy()
+    scales[3, 2], scales[500, 0], biases[7, 1] = np.inf, -np.inf, -np.inf
+    out = run(scales, biases)
+    assert np.isposinf(out[:, 3]).all() and np.isneginf(out[:, 500]).all() and np.isneginf(out[:, 7]).all()
+    rest = np.setdiff1d(np.arange(n), [3, 7, 500])
+    assert np.array_equal(out[:, rest].view(np.uint16), clean[:, rest].view(np.uint16))
+
+
 @pytest.mark.parametrize("gs,n,k,rows", [(64, 515, 4096, 3), (32, 300, 1056, 16), (128, 1001, 1408, 5)])
 def test_infinite_activations_of_a_gather(hip, gs, n, k, rows):
     from rmlx_amd import ops, runtime as rt
