@@ -1,5 +1,6 @@
-// Streaming GEMV of up to 16 rows per weight row that reads the weights as they lie (4- and 8-bit, group sizes 32 / 64 / 128, any N, any K
-// of whole groups up to one row's share of the LDS): a matrix (DENSE), the rows of the expert that a chunk table names (TABLE), and the
+// Streaming GEMV of up to 16 rows per weight row that reads the weights as they lie (4- and 8-bit, group sizes 32 / 64 / 128, any N from a
+// tile on, any K of whole groups from 512 to what a workgroup's registers hold of 16 activation rows, 8192 at 4 bits, 4096 at 8 and at group
+// size 32): a matrix (DENSE), the rows of the expert that a chunk table names (TABLE), and the
 // SwiGLU of its gate and up matrices (PAIR).  The products are exact (integer dot products, scaled in f32).
 //
 // What bounds it is HBM.  The other multi-row GEMVs load a tile of 16 weight rows as the matrix instruction wants it, 64 bytes of each of
@@ -308,7 +309,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
   uint32_t pos = 0, end = 0, gather_chunks = 0;
   // GATHER: every workgroup groups the entries by expert itself (a launch of its own for that costs more: 3 us against about 1.5), a stable
   // counting sort over at most 256 of them, all waves alike behind the ranks.  A chunk is 16 rows of one expert's entries one behind another;
-  // a workgroup's share lies in at most four of those (all fit in two times the workgroups): lane 16 s + i keeps row i of the s-th.
+  // a workgroup's share lies in at most four of those (at most 256 chunks, an entry has no more than 16 rows, and twice the workgroups are
+  // let in): lane 16 s + i keeps row i of the s-th.
   uint32_t seg_row = 0, seg_rows = 0, seg_expert = 0;
   if constexpr (MODE == GATHER) {
     uint32_t* const keys = reinterpret_cast<uint32_t*>(lds);  // in the place of the rings

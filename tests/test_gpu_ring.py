@@ -100,8 +100,8 @@ def test_library_takes_it_for_a_few_rows_per_expert(hip, tokens, taken):
 @pytest.mark.parametrize("batch,rows,experts,dtype", [(1, 1, 3, "f16"), (5, 16, 2, "f16"), (37, 3, 4, "f32"), (256, 1, 200, "f16"), (255, 5, 7, "f32"), (160, 13, 3, "f16"),
                                                       (129, 2, 1000, "f16")])
 def test_gather(hip, gs, k, n, batch, rows, experts, dtype):
-    """Entries of one expert share chunks of 16 rows: runs of one entry and of many, chunks that begin in the middle of an entry, more
-    chunks than workgroups; on a stream the rows of an index out of range are zero."""
+    """Entries of one expert share chunks of 16 rows: runs of one entry and of many, chunks that begin in the middle of an entry, from one
+    chunk for the whole chip to about half a chunk for a workgroup; on a stream the rows of an index out of range are zero."""
     from rmlx_amd import ops, runtime as rt
     from rmlx_amd.runtime import DeviceBuffer
     rng = np.random.default_rng(batch + rows + n)
@@ -298,6 +298,32 @@ def test_infinite_activations_of_a_routed_block(hip, bits, gs, hidden, inter, fu
     rest = [t for t in range(tokens) if t not in odd]
     assert np.isfinite(clean).all() and np.array_equal(out[rest].view(np.uint16), clean[rest].view(np.uint16))
     assert np.isposinf(out[odd][:, 0::2]).all() and np.isneginf(out[odd][:, 1::2]).all()
+
+
+@pytest.mark.parametrize("bits,gs,hidden,inter,experts,dtype", [(4, 64, 576, 512, 600, "f16"), (8, 64, 512, 640, 560, "bf16"), (4, 32, 544, 544, 300, "f32"),
+                                                                (4, 64, 4608, 512, 540, "f16")])
+def test_more_chunks_than_workgroups(hip, bits, gs, hidden, inter, experts, dtype):
+    """A workgroup's share then holds whole chunks, one behind another, and begins and ends inside others: rings, sums and activations start over."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(experts)
+    tokens = experts * 3 // 2
+    one = [make_weight(rng, n, k, bits, gs, (20,)) for n, k in ((inter, hidden), (inter, hidden), (hidden, inter))]
+    gate, up, down = (tuple(np.ascontiguousarray(np.resize(a, (experts,) + a.shape[1:])) for a in t) for t in one)
+    g, u, d = (ops.QuantizedWeight.from_numpy(*w, gs, bits) for w in (gate, up, down))
+    g.set_expert_stream_kernel(6)
+    x = make_x(rng, tokens, hidden, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    idx = rng.integers(0, experts, size=(tokens, 2)).astype(np.uint32)
+    idx[:, 0] = np.arange(tokens) % experts  # every expert one row or two and what it is picked by at random
+    idx[7:40, 1], idx[60:77, 1] = 11, experts - 40  # three chunks, two
+    w = rng.uniform(0.2, 0.8, size=(tokens, 2)).astype(np.float32)
+    counts = np.bincount(idx.ravel(), minlength=experts)
+    chunks = int(((counts + 15) // 16).sum())
+    print(f"Q{bits} gs={gs} {hidden}/{inter}: {chunks} chunks, at most {counts.max()} rows", flush=True)
+    assert chunks > 256 and (counts > 16).sum() >= 2 and (experts < 512 or chunks > 512)
+    out = ops.moe_forward_grouped(g, u, d, xd, rt.DeviceBuffer.from_numpy(idx.ravel()), rt.DeviceBuffer.from_numpy(w.ravel()), 2).numpy()
+    x16 = x_as_f64(x, dtype).astype(np.float16)
+    assert_close(out, model.moe_forward(x16, idx.ravel(), w.ravel(), gate, up, down, gs, 2, bits=bits))
 
 
 def test_pinned_block_keeps_the_callers_gemm_threshold(hip):
