@@ -42,8 +42,8 @@ __global__ __launch_bounds__(64) void topk_route_kernel(const float* __restrict_
 // (one per expert) in LDS: it counts its run, thread e turns the counts of expert e into its offset plus an exclusive prefix over what lies
 // before the wave, and the wave walks its run once more, in order and with nobody else's cursors to wait for: position = the wave's cursor of
 // the expert + rank among the 64 lanes (by ballots over the bits of the id), so ids of one expert keep their original order
-// (numpy.argsort(kind="stable")).  Bound by the chain of one wave's iterations and its scattered stores, so beyond 1024 assignments there are
-// several workgroups (at most 32): each counts everybody's assignments itself, before and behind its portion, which costs less than
+// (numpy.argsort(kind="stable")).  Bound by the chain of one wave's iterations and its scattered stores, so from 2048 assignments on there are
+// several workgroups (at most 32, see sort_portion): each counts everybody's assignments itself, before and behind its portion, which costs less than
 // meeting in a second launch.  The first one writes the tables.  16384 assignments over 128 experts 24 to 37 us in one workgroup, 11 to 13 now.
 __device__ __forceinline__ uint32_t block_exclusive_scan_1024(uint32_t v, uint32_t* wave_tot, uint32_t* total) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -447,7 +447,9 @@ int32_t launch_route_sort_small(const float* logits, const float* bias, uint32_t
   return RMLX_OK;
 }
 
-// Assignments per workgroup of the sort: 1024 and more, at most 32 workgroups
+// Assignments per workgroup of the sort: one workgroup for every 1024 assignments, at most 32, their equal shares rounded up to whole 1024s (a
+// wave's run is whole 64s).  So a number a little past a step leaves the last ones little or nothing: 2049 are 2048 and 1, 32769 are 16 portions
+// of 2048 and one of 1.
 static uint32_t sort_portion(uint32_t n_assign) {
   const uint32_t wgs = n_assign / 1024 < 1 ? 1 : (n_assign / 1024 > 32 ? 32 : n_assign / 1024), each = (n_assign + wgs - 1) / wgs;
   return (each + 1023) / 1024 * 1024;

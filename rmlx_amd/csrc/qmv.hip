@@ -50,7 +50,7 @@ constexpr int kWaves = 8;
 constexpr int kSpwMax = 4;  // slabs (128 k) per wave per pass
 
 // What the first loads of a wave need travels a second time, as plain arguments in front of the struct (launch.hpp): 4 rows, 9216 x 4096 8.9 ->
-// 8.35 us, 8 rows 4096 x 1024 5.0 -> 4.75 (the tile GEMMs, whose waves start with long address work, lose 0.3 us by it and keep their struct).
+// 8.45 us, 8 rows 4096 x 1024 5.0 -> 4.75 (the tile GEMMs, whose waves start with long address work, lose 0.3 us by it and keep their struct).
 struct KParams {
   const uint32_t* w0;
   const __half* s0;

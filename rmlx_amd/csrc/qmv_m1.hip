@@ -48,8 +48,8 @@ constexpr int kThreads = 512;
 constexpr int kWaves = 8;
 constexpr uint32_t kMaxK = 32768;  // (the activation image and sums must also fit the default dynamic LDS limit)
 
-// What only some kernels or only the end of one needs.  The rest of M1Params are plain arguments (launch.hpp).  One row, 4096 x 4096 3.97 -> 3.83 us, 9216 x 4096 6.7 -> 6.4, 8-bit
-// 4096 x 4096 5.1 -> 4.8.
+// What only some kernels or only the end of one needs.  The rest of M1Params are plain arguments (launch.hpp).  One row, weights
+// from HBM, calls queued: 4096 x 4096 3.87 -> 3.72 us, 9216 x 4096 6.9 -> 6.6, 8-bit 4096 x 4096 5.1 -> 4.7; a call by itself is bound by the host, as before.
 struct M1Rest {
   __half* out;
   int32_t epi_kind, epi_dtype;  // fused store epilogue: EPI_RESIDUAL / EPI_SWIGLU with an [M,N] f16 / f32 operand

@@ -13,10 +13,10 @@
 // One workgroup of eight waves per CU takes an equal share of all weight rows (of all chunks, for a table): no last round that is half
 // empty, whatever the number of rows.  A slot costs one barrier; the waves' partial sums of a tile are added through LDS behind the
 // products of the next one.
-// Routed block, 128 experts, hidden 4096, inner 1536, top 8, 4-bit, group size 64: 12 / 32 / 64 / 128 / 200 tokens 142 / 219 / 246 / 264 / 302 us
-// against 166 / 249 / 286 / 347 / 382 on the kernels before (floor by its bytes: 193 at 128 tokens); 40 experts, hidden 2944, inner 3072, group
-// size 128, 15 / 120 tokens of 4 picks: 89 / 129 against 156 / 241.  8 rows, 33001 x 2880 15.3 us against 23.2; 13 rows, 14336 x 4096, 8-bit 14.6
-// against 18.7; 16 rows, 151936 x 4096 62.4 against 93.4.  A slot of 16 x 4096 takes 1.25 us with its weights in the caches, 1.35 at the floor of HBM:
+// Routed block, 128 experts, hidden 4096, inner 1536, top 8, 4-bit, group size 64: 12 / 32 / 64 / 128 / 200 tokens 143 / 221 / 247 / 264 / 303 us
+// against 165 / 247 / 287 / 348 / 390 on the kernels before (three blocks in turn; floor by its bytes: 193 at 128 tokens); 40 experts, hidden 2944,
+// inner 3072, group size 128, 15 / 120 tokens of 4 picks: 93 / 131 against 154 / 252.  8 rows, 33001 x 2880 16.2 us against 20.9; 13 rows, 14336 x 4096,
+// 8-bit, four matrices 58.8 against 75.1; 16 rows, 151936 x 4096 66 against 104.  A slot of 16 x 4096 takes 1.25 us with its weights in the caches, 1.35 at the floor of HBM:
 // 169 vector instructions per wave and slot, 80 of them unpacking, so both sides are nearly equal.
 //
 // (the device code below loads with inline assembly where the compiler would wait for the loads of a slot before it lets the next one out;
