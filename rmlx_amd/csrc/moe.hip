@@ -45,6 +45,7 @@ __global__ __launch_bounds__(64) void topk_route_kernel(const float* __restrict_
 // (numpy.argsort(kind="stable")).  Bound by the chain of one wave's iterations and its scattered stores, so from 2048 assignments on there are
 // several workgroups (at most 32, see sort_portion): each counts everybody's assignments itself, before and behind its portion, which costs less than
 // meeting in a second launch.  The first one writes the tables.  16384 assignments over 128 experts 24 to 37 us in one workgroup, 11 to 13 now.
+// A workgroup alone (SHARED: false) has no counts of others to clear and read (a routed block of 96 assignments 27.9 us with them, 27.6 without).
 __device__ __forceinline__ uint32_t block_exclusive_scan_1024(uint32_t v, uint32_t* wave_tot, uint32_t* total) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   uint32_t inc = v;
@@ -66,6 +67,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan_1024(uint32_t v, uint32
   return base + inc - v;
 }
 
+template <bool SHARED>
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const uint32_t* __restrict__ idx, uint32_t n_assign,
                                                         uint32_t E, uint32_t top_k, uint32_t* __restrict__ sorted,
                                                         uint32_t* __restrict__ sorted_tok,
@@ -77,16 +79,15 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const uint32_t* __restri
                                                         uint32_t split_cap, uint32_t portion) {
   __shared__ uint32_t wave_tot[16];
   __shared__ uint32_t cur[16][kMaxExperts];  // per wave and expert: count of the wave's run, then its running cursor
-  __shared__ uint32_t others[2][kMaxExperts];  // assignments before and behind this workgroup's
+  __shared__ uint32_t others[SHARED ? 2 * kMaxExperts : 1];  // assignments before and behind this workgroup's
   const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t first = blockIdx.x * portion, last = first + portion < n_assign ? first + portion : n_assign;
+  const uint32_t first = SHARED ? blockIdx.x * portion : 0, last = first + portion < n_assign ? first + portion : n_assign;
   const uint32_t run = portion / 16, begin = first + wave * run < last ? first + wave * run : last, end = begin + run < last ? begin + run : last;
 #pragma unroll
   for (int w = 0; w < 16; ++w) cur[w][tid] = 0;  // kMaxExperts == blockDim.x
-  others[0][tid] = 0;
-  others[1][tid] = 0;
+  if constexpr (SHARED) others[tid] = others[kMaxExperts + tid] = 0;
   __syncthreads();
-  if (gridDim.x > 1) {
+  if constexpr (SHARED) {
     auto count = [&](uint32_t from, uint32_t to, uint32_t* into) {
 #pragma unroll 8
       for (uint32_t i = from + tid; i < to; i += 1024) {
@@ -94,8 +95,8 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const uint32_t* __restri
         if (e < E) atomicAdd(&into[e], 1u);
       }
     };
-    count(0, first, others[0]);
-    count(last, n_assign, others[1]);
+    count(0, first, others);
+    count(last, n_assign, others + kMaxExperts);
   }
 #pragma unroll 4
   for (uint32_t i = begin + lane; i < end; i += 64) {
@@ -104,8 +105,11 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const uint32_t* __restri
   }
   __syncthreads();
   // thread e owns expert e: offsets, counts, its chunks of at most chunk_rows rows
-  const uint32_t earlier = others[0][tid];
-  uint32_t my_cnt = earlier + others[1][tid];
+  uint32_t earlier = 0, my_cnt = 0;
+  if constexpr (SHARED) {
+    earlier = others[tid];
+    my_cnt = earlier + others[kMaxExperts + tid];
+  }
 #pragma unroll
   for (int w = 0; w < 16; ++w) my_cnt += cur[w][tid];
   uint32_t total_rows, total_chunks;
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const uint32_t* __restri
     cur[w][tid] = before;
     before += c;
   }
-  const bool writes = blockIdx.x == 0;
+  const bool writes = !SHARED || blockIdx.x == 0;
   if (writes && tid < E) {
     if (offsets != nullptr) offsets[tid] = my_off;
     if (counts != nullptr) counts[tid] = my_cnt;
@@ -425,7 +429,7 @@ int32_t launch_topk_route(const float* logits, const float* bias, uint32_t T, ui
                        (uint32_t*)nullptr);
     RMLX_HIP_CHECK(hipGetLastError());
   } else if (counts != nullptr || offsets != nullptr) {
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, s, idx, T * K, E, K, (uint32_t*)nullptr,
+    hipLaunchKernelGGL(moe_sort_kernel<false>, dim3(1), dim3(1024), 0, s, idx, T * K, E, K, (uint32_t*)nullptr,
                        (uint32_t*)nullptr, (uint32_t*)nullptr, counts, offsets, (uint32_t*)nullptr,
                        (uint32_t*)nullptr, 8u, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u, (T * K + 1023) / 1024 * 1024);
     RMLX_HIP_CHECK(hipGetLastError());
@@ -466,8 +470,8 @@ int32_t launch_moe_sort(const uint32_t* idx, uint32_t n_assign, uint32_t E, uint
     hipLaunchKernelGGL(moe_sort_small_kernel, dim3(1), dim3(64), 0, s, idx, n_assign, E, top_k ? top_k : 1u, sorted,
                        sorted_tok, inv, counts, offsets, chunk_tab, n_chunks);
   else {
-    const uint32_t portion = sort_portion(n_assign);
-    hipLaunchKernelGGL(moe_sort_kernel, dim3(n_assign == 0 ? 1 : (n_assign + portion - 1) / portion), dim3(1024), 0, s, idx, n_assign, E, top_k ? top_k : 1u,
+    const uint32_t portion = sort_portion(n_assign), wgs = n_assign == 0 ? 1 : (n_assign + portion - 1) / portion;
+    hipLaunchKernelGGL(wgs > 1 ? moe_sort_kernel<true> : moe_sort_kernel<false>, dim3(wgs), dim3(1024), 0, s, idx, n_assign, E, top_k ? top_k : 1u,
                        sorted, sorted_tok, inv, counts, offsets, chunk_tab, n_chunks, chunk_rows, split_tab, split_n, split_cap, portion);
   }
   RMLX_HIP_CHECK(hipGetLastError());
