@@ -809,10 +809,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void qmv_ring_kernel(uint64_t w0_, 
     store_unbounded<BITS, GS, H, MODE>(lds, spoiled != spoiled, gather_chunks, seg_row, seg_rows, seg_expert);
 }
 
-struct RingLaunch { const QmvArgs* a; uint32_t geometry, share, over, chunks, cpr_inv; RingParams p; };
+struct RingLaunch { const QmvArgs* a; uint32_t geometry, share, over, wgs, chunks, cpr_inv; RingParams p; };
 template <int BITS, int GS, int U, int H, int MODE>
 void launch_ring(const RingLaunch& l, hipStream_t s) {
-  Launch<qmv_ring_kernel<BITS, GS, U, H, MODE>>::go(dim3(ctx().num_cus, l.chunks), dim3(kWaves * 64), 0, s, address(l.a->w0), address(l.a->s0),
+  Launch<qmv_ring_kernel<BITS, GS, U, H, MODE>>::go(dim3(l.wgs, l.chunks), dim3(kWaves * 64), 0, s, address(l.a->w0), address(l.a->s0),
                                                     address(l.a->b0), address(l.a->x), l.a->N, l.a->K, l.a->M, l.geometry, l.share, l.over, l.cpr_inv, l.p);
 }
 template <int BITS, int GS, int U, int H>
@@ -862,6 +862,7 @@ bool qmv_ring_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
 static void ring_split(const QmvArgs& a, uint32_t bits, uint32_t gs, int32_t x_dtype, RingPlan* plan, RingLaunch* l) {
   RingParams& p = l->p;
   l->a = &a;
+  l->wgs = ctx().num_cus;
   p.out = a.out; p.row_map = a.row_map; p.chunk_tab = a.chunk_tab; p.n_chunks = a.n_chunks_dev;
   p.w1 = a.w1; p.s1 = a.s1; p.b1 = a.b1;
   p.estride_w = a.expert_stride_w; p.estride_s = a.expert_stride_s;
@@ -887,6 +888,23 @@ static int32_t launch_format(const RingLaunch& l, const RingPlan& plan, uint32_t
   return RMLX_OK;
 }
 
+// Workgroups over the rows of a matrix: one per CU, or a few less where a workgroup's share is within 3 KB of a power of two and its 128th part
+// more, or less, from 512 KB on: walked side by side, such shares keep to a part of the memory channels (8 rows, 8-bit, us, by what the share
+// is beyond the power, KB: 512 KB, K = 2048, 0 / 2 / 4 / 6 / 8 25.9 / 28.3 / 35.3 / 26.8 / 26.7; 1 MB, K = 4096, 0 / 4 / 6 / 8 / 10 / 12 / 16 45.8 / 48.0 /
+// 51.7 / 58.6 / 52.0 / 48.2 / 47.5, -8 52.0; 2 MB, 8 / 16 / 24 89.4 / 102.6 / 90.1; 256 KB, 1 / 2 / 3 16.8 / 17.9 / 17.3).  33001 x 4096, 2 / 16 rows 33.3 /
+// 34.5 us on all CUs, 25.9 / 27.3 on two less.
+static uint32_t ring_workgroups(uint64_t bytes) {
+  const uint32_t cus = ctx().num_cus;
+  for (uint32_t w = cus; w + 8 > cus && w > 0; --w) {
+    const uint64_t share = bytes / w;
+    uint64_t p = 512 << 10;
+    while (p + p / 2 < share) p *= 2;
+    const int64_t past = (int64_t)(share > p ? share - p : p - share) - (int64_t)(p / 128);
+    if (past < -3072 || past > 3072) return w;
+  }
+  return cus;
+}
+
 int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32_t x_rows, hipStream_t s) {
   const uint32_t gs = a.group_size == 0 ? 64 : a.group_size, size = x_dtype == RMLX_DTYPE_F32 ? 4 : 2;
   if (!qmv_ring_supported(a.N, a.K, gs, bits) || (a.dual != 0 && a.chunk_tab == nullptr) || (a.row_map != nullptr && (uint64_t)x_rows * a.K * size > 0x80000000ull))
@@ -902,8 +920,9 @@ int32_t launch_qmv_ring(const QmvArgs& a, uint32_t bits, int32_t x_dtype, uint32
   } else {
     if (a.M == 0) return RMLX_OK;
     l.chunks = (a.M + 15) / 16;
-    l.share = a.N / ctx().num_cus;
-    l.over = a.N - l.share * ctx().num_cus;
+    l.wgs = ring_workgroups((uint64_t)a.N * a.K * bits / 8);
+    l.share = a.N / l.wgs;
+    l.over = a.N - l.share * l.wgs;
   }
   return launch_format(l, plan, bits, gs, s);
 }

@@ -436,3 +436,18 @@ def test_recorded_calls_replay_bit_for_bit(hip):
             assert np.array_equal(o.numpy().view(np.uint16), e.view(np.uint16))
         calls(outs)
         stream.sync()
+
+
+@pytest.mark.parametrize("bits,gs,n,k", [(8, 64, 32776, 4096), (8, 64, 33001, 4096), (8, 32, 33024, 4032), (4, 64, 33001, 8192), (4, 64, 132096, 4096)])
+def test_shares_away_from_one_part_of_the_channels(hip, bits, gs, n, k):
+    """One workgroup less or several: every row once, the same bits as in a matrix of a few rows."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(n + k)
+    base = 400
+    w = make_weight(rng, base, k, bits, gs)
+    x = make_x(rng, 3, k)
+    xd = rt.DeviceBuffer.from_numpy(x)
+    run = lambda t: ops.affine_quantized_matmul_batched(xd, ops.QuantizedWeight.from_numpy(*t, gs, bits), kernel=rt.KERNEL_QMV_RING).numpy()
+    small, out = run(w), run(tuple(np.resize(a, (n,) + a.shape[1:]) for a in w))
+    assert_close(small, model.qmm(x, *w, gs, bits))
+    assert np.array_equal(out.view(np.uint16), np.resize(small.T, (n, 3)).T.view(np.uint16))
