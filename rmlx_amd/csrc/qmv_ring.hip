@@ -17,7 +17,7 @@
 // against 165 / 247 / 287 / 348 / 390 on the kernels before (three blocks in turn; floor by its bytes: 193 at 128 tokens); 40 experts, hidden 2944,
 // inner 3072, group size 128, 15 / 120 tokens of 4 picks: 93 / 131 against 154 / 252.  8 rows, 33001 x 2880 16.2 us against 20.9; 13 rows, 14336 x 4096,
 // 8-bit, four matrices 58.8 against 75.1; 16 rows, 151936 x 4096 66 against 104.  A slot of 16 x 4096 takes 1.25 us with its weights in the caches, 1.35 at the floor of HBM:
-// 169 vector instructions per wave and slot, 80 of them unpacking, so both sides are nearly equal.
+// 171 vector instructions per wave and slot, 80 of them unpacking, so both sides are nearly equal.
 //
 // (the device code below loads with inline assembly where the compiler would wait for the loads of a slot before it lets the next one out;
 // the counts behind wait_but are those of the loads that this kernel issues, in order)
@@ -197,7 +197,7 @@ __device__ __forceinline__ float plain_sum(const char* w, const __half* s, const
 // here at its end and goes over the results of such rows once more, over the pieces of the row that are not finite (the others do not change
 // the sum; over all of it where there are none: then the weights are not finite); what is not finite is stored anew.  The arguments are read again, so that nothing
 // is kept for this (as scalar registers they made the others spill), and what it costs the others is a multiply-add for each result:
-// gather of 32 x 8 rows 40.6 -> 40.9 us, 13 rows, 14336 x 4096, 8-bit 59.2 -> 58.9 for four.  A row of 100001 x 4096 with one infinity
+// gather of 32 x 8 rows 40.6 -> 40.9 us, of 89 x 2 rows over 32 experts of 1664 x 2496 24.3 -> 24.5, 13 rows, 14336 x 4096, 8-bit 59.2 -> 58.9 for four.  A row of 100001 x 4096 with one infinity
 // 45 -> 70 us, all 16 rows 142 (3.1 ms with every lane looking through its row for itself).
 typedef const __attribute__((address_space(1))) RingArgs* RingArgsPtr;
 template <int BITS, int GS, int H, int MODE>
