@@ -158,7 +158,8 @@ def test_library_takes_it_for_gathers_of_many_weights(hip, batch, rows, experts,
                                                        (13, 4096, 4096, 8, 64, "f32", True), (5, 4096, 4096, 8, 32, "f32", True), (4, 4096, 1024, 4, 32, "f16", True),
                                                        (8, 4096, 1024, 4, 32, "f16", False), (16, 4096, 1152, 4, 32, "bf16", True), (17, 4096, 1152, 4, 32, "bf16", False),
                                                        (6, 8192, 2560, 8, 64, "f16", False), (7, 8192, 2816, 8, 64, "bf16", True), (6, 8256, 2560, 8, 64, "f32", True),
-                                                       (3, 16384, 1024, 8, 64, "f16", False), (8, 16384, 1024, 8, 64, "f16", True), (9, 8192, 2304, 8, 64, "f16", False), (10, 8192, 2304, 8, 64, "f16", True),
+                                                       (3, 16384, 1024, 8, 64, "f16", False), (3, 16384, 1024, 8, 64, "f32", True), (8, 8192, 2304, 8, 64, "f32", False),
+                                                       (8, 16384, 1024, 8, 64, "f16", True), (9, 8192, 2304, 8, 64, "f16", False), (10, 8192, 2304, 8, 64, "f16", True),
                                                        (9, 12288, 1024, 8, 64, "f16", False), (2, 14336, 3520, 4, 64, "f16", False), (2, 14345, 3520, 4, 64, "f16", True),
                                                        (4, 12288, 3264, 4, 64, "bf16", False), (3, 12289, 3264, 4, 64, "f16", True), (4, 8192, 2560, 8, 128, "f16", True)])
 def test_library_takes_it_for_a_few_rows(hip, m, n, k, bits, gs, dtype, taken):
