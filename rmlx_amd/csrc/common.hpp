@@ -292,18 +292,20 @@ struct GroupedQmmArgs {
   const uint32_t* tile_tab; const uint32_t* n_tiles_dev;
   uint32_t max_tiles;        // row tiles the grid covers (>= *n_tiles_dev)
   uint32_t tile_rows;        // rows per tile the table was built for: 16, 32 or (one weight) kGroupedTileRows; tile GEMMs: 32, 64, 128 or 256
+  int twin;                  // tile GEMMs: on qmm_twin.hip, tile_rows up to 160 (8-bit: 128)
 };
 bool qmm_rw_grouped_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 int32_t launch_qmm_rw_grouped(const GroupedQmmArgs& a, hipStream_t s);
-// GEMM of large tiles (qmm_tile.hip, qmm_slice.hip): f16 activations, 4- / 8-bit weights, group size 32 / 64 / 128, any N, any K (at
+// GEMM of large tiles (qmm_tile.hip, qmm_slice.hip, qmm_twin.hip): f16 activations, 4- / 8-bit weights, group size 32 / 64 / 128, any N, any K (at
 // least eight groups in the whole matrix).  A plan = tile of 32 mi rows by 32 wn columns, kw wave groups along k inside the workgroup
-// (kw >= 4: qmm_slice.hip, mi 1 or 2), K cut into `splits` ranges (f32 partial sums in QmmArgs::workspace, added up by a second kernel).
-struct TilePlan { uint32_t wn, mi, kw, splits; };
+// (kw >= 4: qmm_slice.hip, mi 1 or 2), K cut into `splits` ranges (f32 partial sums in QmmArgs::workspace, added up by a second kernel); twin:
+// qmm_twin.hip, wn 4 or 8.
+struct TilePlan { uint32_t wn, mi, kw, splits; bool twin = false; };
 bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us);  // us: estimated time of the launch
 size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N);
 int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s);
-// The same over a table of row tiles of 32, 64, 128 or 256 rows of one expert (x_rows: rows of x; out f16 or f32, a pair f16).  A row map
+// The same over a table of row tiles of 32, 64, 128 or 256 rows (twin: up to 160, 8-bit 128) of one expert (x_rows: rows of x; out f16 or f32, a pair f16).  A row map
 // reaches the rows of an x of at most 2 GiB.
 bool qmm_tile_maps_rows(uint32_t x_rows, uint32_t K);
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);

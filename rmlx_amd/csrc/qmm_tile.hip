@@ -494,9 +494,9 @@ bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
 // and end, a K split the kernel that adds up the partial sums.  Fitted to about 15000 timed launches (780 shapes, every plan and
 // split): 6 % mean error, and the picks are 1.3 % slower on average than the fastest plan.
 static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us) {
-  // (kw >= 4: waves along k, steps of `k` values)
-  struct Cost { uint32_t wn, mi, kw; int per_cu; double start, step[3][2], sum, sum_per_mi; uint32_t k; };
-  static const Cost costs[2][10] = {
+  // (kw >= 4: waves along k, steps of `k` values; mi_most: two workgroups per CU, qmm_twin.hip, tiles of mi to mi_most fragments)
+  struct Cost { uint32_t wn, mi, kw; int per_cu; double start, step[3][2], sum, sum_per_mi; uint32_t k, mi_most; };
+  static const Cost costs[2][12] = {
       {{8, 8, 1, 1, 8.19, {{0.503, 0.118}}, 7.46, 1.10},
        {8, 4, 1, 1, 3.71, {{0.428, 0.110}}, 4.90, 1.74},
        {4, 4, 1, 2, 4.64, {{0.270, 0.073}, {0.531, 0.083}}, 3.39, 1.59},
@@ -506,7 +506,9 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
        {2, 1, 8, 2, 4.14, {{0.256, 0.271}, {1.023, 0.000}}, 3.00, 0.10, 256},
        {2, 2, 8, 1, 5.20, {{0.089, 0.370}}, 2.80, 0.00, 256},
        {4, 1, 4, 1, 4.56, {{0.201, 0.751}}, 3.20, 1.04, 256},
-       {4, 2, 4, 1, 5.46, {{0.296, 0.467}}, 2.87, 1.33, 256}},
+       {4, 2, 4, 1, 5.46, {{0.296, 0.467}}, 2.87, 1.33, 256},
+       {8, 3, 1, 2, 5.86, {{0.365, 0.171}, {0.572, 0.278}}, 3.28, 1.29, 0, 5},
+       {4, 3, 1, 2, 4.85, {{0.269, 0.098}, {0.358, 0.153}}, 2.73, 1.52, 0, 7}},
       {{8, 8, 1, 1, 7.26, {{0.608, 0.104}}, 8.71, 1.34},
        {8, 4, 1, 1, 3.33, {{0.516, 0.102}}, 5.39, 1.89},
        {4, 4, 1, 2, 4.87, {{0.352, 0.047}, {0.628, 0.091}}, 3.44, 1.65},
@@ -516,15 +518,16 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
        {2, 1, 8, 1, 4.61, {{0.000, 0.671}}, 2.59, 0.00, 256},
        {2, 2, 8, 1, 5.17, {{0.061, 0.452}}, 2.30, 0.00, 256},
        {4, 1, 4, 1, 4.56, {{0.032, 1.080}}, 3.39, 0.00, 256},
-       {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128}}};
+       {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128},
+       {8, 3, 1, 2, 3.81, {{0.571, 0.154}, {0.722, 0.256}}, 3.89, 1.50, 0, 4},
+       {4, 3, 1, 2, 3.84, {{0.330, 0.105}, {0.395, 0.173}}, 3.25, 1.55, 0, 7}}};
   constexpr double kExactStep = 1.5;  // two products: 8 to 64 rows 1.35 to 1.45 x, 300 to 2000 rows 1.55 to 1.65
   const double cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
   const uint32_t rounds = (K + 127) / 128;
   TilePlan best{4, 2, 1, 1};
   double best_us = 1e30;
-  for (const Cost& c : costs[bits == 8]) {
-    if (c.k != 0 && c.mi == 2 && M <= 32) continue;
-    const uint64_t tm = (M + c.mi * 32 - 1) / (c.mi * 32), tiles = tm * ((N + c.wn * 32 - 1) / (c.wn * 32));
+  auto price = [&](const Cost& c, uint32_t mi) {
+    const uint64_t tm = (M + mi * 32 - 1) / (mi * 32), tiles = tm * ((N + c.wn * 32 - 1) / (c.wn * 32));
     const double frags = (double)((M + 31) / 32) / (double)tm;
     for (uint32_t splits : {1u, 2u, 3u, 4u, 6u, 8u}) {
       const uint32_t stages = c.k != 0 ? (K + c.k - 1) / c.k : 0;
@@ -538,8 +541,12 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
       }
       t = c.start + (exact ? kExactStep : 1.0) * t;
       if (splits > 1) t += c.sum + c.sum_per_mi * splits * ((double)M * N / (1 << 20));
-      if (t < best_us) { best_us = t; best = TilePlan{c.wn, c.mi, c.kw, splits}; }
+      if (t < best_us) { best_us = t; best = TilePlan{c.wn, mi, c.kw, splits, c.mi_most != 0}; }
     }
+  };
+  for (const Cost& c : costs[bits == 8]) {
+    if ((c.k != 0 && c.mi == 2 && M <= 32) || (c.mi_most != 0 && exact)) continue;
+    for (uint32_t mi = c.mi; mi <= (c.mi_most > c.mi ? c.mi_most : c.mi); ++mi) price(c, mi);
   }
   *us = best_us;
   return best;
@@ -578,7 +585,8 @@ int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s) {
   p.epi_kind = a.epi_kind; p.epi = a.epi; p.epi_dtype = a.epi_dtype; p.exact = a.exact;
   const uint64_t wgs = (uint64_t)p.tiles_m * p.tiles_n * p.splits;
   if (wgs > 0x7FFFFFFFull) return fail(RMLX_INVALID_SHAPE, "qmm: grid too large");
-  if (plan.kw >= 4) launch_qmm_slice(p, a.bits, plan, dim3((unsigned)wgs), s);
+  if (plan.twin) launch_qmm_twin(p, a.bits, plan.wn, dim3((unsigned)wgs), s);
+  else if (plan.kw >= 4) launch_qmm_slice(p, a.bits, plan, dim3((unsigned)wgs), s);
   else if (a.bits == 4) launch_tile<4>(p, plan, dim3((unsigned)wgs), s);
   else launch_tile<8>(p, plan, dim3((unsigned)wgs), s);
   RMLX_HIP_CHECK(hipGetLastError());
@@ -602,12 +610,13 @@ int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStr
   p.tile_tab = a.tile_tab; p.n_tiles = a.n_tiles_dev; p.row_map = a.row_map; p.x_rows = x_rows;
   p.estride_w = a.expert_stride_w; p.estride_s = a.expert_stride_s;
   p.splits = 1;
-  const TilePlan plan{a.tile_rows == 256 ? 8u : 4u, a.tile_rows / 32, 1, 1};
+  const TilePlan plan{a.tile_rows == 256 || a.twin ? 8u : 4u, a.tile_rows / 32, 1, 1, a.twin != 0};
   const uint32_t cols = plan.wn * 32 / (a.w1 != nullptr ? 2 : 1);
   p.tiles_n = (a.N + cols - 1) / cols;
   const uint64_t wgs = (uint64_t)a.max_tiles * p.tiles_n;
   if (wgs > 0x7FFFFFFFull) return fail(RMLX_INVALID_SHAPE, "grouped qmm: grid too large");
-  if (a.bits == 4) launch_tile<4>(p, plan, dim3((unsigned)wgs), s);
+  if (plan.twin) launch_qmm_twin(p, a.bits, plan.wn, dim3((unsigned)wgs), s);
+  else if (a.bits == 4) launch_tile<4>(p, plan, dim3((unsigned)wgs), s);
   else launch_tile<8>(p, plan, dim3((unsigned)wgs), s);
   RMLX_HIP_CHECK(hipGetLastError());
   return RMLX_OK;

@@ -1,4 +1,4 @@
-// Pieces that the two MFMA tile GEMMs (qmm_tile.hip, qmm_slice.hip) share: direct loads into LDS, weight unpacking, tile order.
+// Pieces that the MFMA tile GEMMs (qmm_tile.hip, qmm_slice.hip, qmm_twin.hip) share: direct loads into LDS, weight unpacking, tile order.
 #pragma once
 #include "common.hpp"
 
@@ -19,6 +19,8 @@ struct TileParams {
 };
 // The GEMM with waves along k (qmm_slice.hip), for the plans that have four or more (kw)
 void launch_qmm_slice(const TileParams& p, uint32_t bits, const TilePlan& plan, dim3 grid, hipStream_t s);
+// The GEMM of two workgroups per CU (qmm_twin.hip): tiles of 256 (wn = 8) or 128 columns (wn = 4; not for a pair)
+void launch_qmm_twin(const TileParams& p, uint32_t bits, uint32_t wn, dim3 grid, hipStream_t s);
 
 namespace {
 
@@ -172,7 +174,11 @@ __device__ __forceinline__ bool tile_of(const TileParams& p, uint32_t tile_rows,
   t.split = idx % p.splits; idx /= p.splits;
   const uint32_t in_block = kBlock * p.tiles_n, first = idx / in_block * kBlock, within = idx % in_block, h = tiles_m - first < kBlock ? tiles_m - first : kBlock;
   t.mt = uni(first + within % h); t.nt = uni(within / h); t.split = uni(t.split);
-  t.expert = 0; t.row_lo = t.mt * tile_rows; t.rows = p.M - t.row_lo; t.zeros = false;
+  // row tiles of equal height, to a fragment of 32 rows
+  const uint32_t frags = (p.M + 31) / 32, q = frags / tiles_m, more = frags % tiles_m;
+  t.expert = 0; t.row_lo = 32 * (t.mt * q + (t.mt < more ? t.mt : more)); t.zeros = false;
+  t.rows = p.M - t.row_lo;
+  if (t.mt + 1 < tiles_m) t.rows = 32 * (q + (t.mt < more ? 1 : 0));
   if (p.tile_tab != nullptr) {
     t.expert = uni(p.tile_tab[3 * t.mt]); t.row_lo = uni(p.tile_tab[3 * t.mt + 1]);
     const uint32_t n = uni(p.tile_tab[3 * t.mt + 2]);

@@ -129,6 +129,44 @@ def _block(rng, experts, hidden, inter, bits=4, gs=64):
     return (gate, up, down), tuple(ops.QuantizedWeight.from_numpy(*w, gs, bits) for w in (gate, up, down))
 
 
+@pytest.mark.parametrize("m,n,k,bits,gs", [(1035, 7859, 160, 4, 32), (540, 18277, 160, 4, 32), (1424, 8708, 160, 4, 32), (519, 31005, 160, 4, 32),
+                                         (550, 12011, 448, 4, 64), (1441, 6150, 384, 4, 128), (513, 3589, 160, 8, 32), (303, 3667, 5120, 8, 128),
+                                         (780, 9275, 224, 8, 32), (543, 14190, 96, 8, 32), (2698, 4894, 96, 8, 32), (411, 22650, 96, 8, 32), (532, 23055, 192, 8, 64)])
+def test_two_workgroups_per_cu(hip, m, n, k, bits, gs):
+    """Sizes that the automatic choice sends to tiles of 128 and 256 columns of the GEMM with two workgroups per CU, at every height it has and
+    with K split; K of half stages, columns and rows that are no whole tile.  Every output against the oracle's, plain and with a residual."""
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(m + n + k)
+    words, s, b = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k)
+    ref = model.qmm(x_as_f64(x, "f16"), words, s, b, gs, bits)
+    assert_close(_run(words, s, b, x, bits, gs), ref, f"M={m} N={n} K={k} bits={bits} gs={gs}")
+    e = rng.standard_normal((m, n)).astype(np.float16)
+    qw = ops.QuantizedWeight.from_numpy(words, s, b, gs, bits)
+    assert_close(ops.qmm_add_residual(DeviceBuffer.from_numpy(x), qw, DeviceBuffer.from_numpy(e)).numpy(), ref + e.astype(np.float64), "residual")
+
+
+@pytest.mark.parametrize("tokens,experts,hidden,inter,bits,gs,fused", [(1500, 32, 1088, 576, 4, 64, True), (3400, 32, 1056, 544, 4, 32, False), (5200, 32, 1088, 576, 4, 64, False),
+                                                                      (1600, 40, 1024, 512, 4, 128, True), (3400, 40, 1088, 576, 8, 64, True), (5300, 40, 1056, 544, 8, 32, False)])
+def test_routed_block_on_two_workgroups_per_cu(hip, tokens, experts, hidden, inter, bits, gs, fused):
+    """Enough tiles for two workgroups on every CU: experts of a few rows to more than one row tile (160, 128 rows)."""
+    from rmlx_amd import ops
+    from rmlx_amd.runtime import DeviceBuffer
+    rng = np.random.default_rng(bits + gs + tokens)
+    gate, up = (make_weight(rng, inter, hidden, bits, gs, (experts,)) for _ in range(2))
+    down = make_weight(rng, hidden, inter, bits, gs, (experts,))
+    both = tuple(np.concatenate([a, b], axis=1) for a, b in zip(gate, up))
+    g = ops.QuantizedWeight.from_numpy(*(both if fused else gate), gs, bits)
+    u = None if fused else ops.QuantizedWeight.from_numpy(*up, gs, bits)
+    d = ops.QuantizedWeight.from_numpy(*down, gs, bits)
+    x = make_x(rng, tokens, hidden)
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32) + 1.5 * rng.standard_normal(experts).astype(np.float32)
+    out = ops.moe_forward(g, u, d, DeviceBuffer.from_numpy(x), DeviceBuffer.from_numpy(logits), 1).numpy()
+    idx, w, _, _ = model.topk_route(logits, 1)
+    assert_close(out, model.moe_forward(x, idx, w, gate, up, down, gs, 1, bits=bits), f"E={experts} D={hidden} I={inter} T={tokens} bits={bits} gs={gs}")
+
+
 @pytest.mark.parametrize("tokens,experts,top_k,hidden,inter", [(262200, 8, 8, 512, 512), (131100, 2, 1, 8192, 512)])
 def test_routed_block_over_more_than_two_gib(hip, tokens, experts, top_k, hidden, inter):
     """Hidden activations, and activations reached through the token map, of more than 2 GiB; the last tokens, which lie beyond it."""
