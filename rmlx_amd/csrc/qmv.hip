@@ -36,6 +36,8 @@
 //     (low register count: up to three workgroups per CU).
 //   * Barriers of the tile reduction wait for LDS traffic only, and a workgroup that walks several
 //     tiles requests the next tile's weights as soon as the current accumulators have left for LDS.
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "q4_stream.hpp"
@@ -85,11 +87,17 @@ struct KParams {
 // before the tile loop (their registers are free again when the weight loads start).
 // RAGGED: any number of weight rows (those past the last repeat it, unstored) and a K of whole groups of 64: the lanes of the last
 // slab's second half, where K ends in its middle, multiply the row's last piece with activations of zero and a scale of zero.
-template <int MR, int TILES, bool TAB, int SPW, bool PAIR, int REUSE, bool RAGGED = false>
-__global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4 : 1) void qmv_q4_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint32_t K_, uint32_t ks_, uint32_t M_, uint32_t gs128_, uint32_t tpw_, uint32_t x_bf16_, KParams p) {
+// SHARE: a wave slot has p.tpw consecutive weight rows of one matrix as TILES tiles of 16 (the last one may be partly empty), all requested behind the
+// activations: one workgroup per CU.  What bounds it is two round trips to memory and, in front of the second, the address unit (64 bytes a clock; 4 rows of
+// 9216 x 4096: without the loads of the activations a tile per workgroup takes 6.4 us instead of 8.2, shares take 7.3; 4.45 is a bare read).
+// G: the group size, 0 = told by p.gs128.  Known here, the scales of group size 128 stay as loaded until the products (spread over the slabs behind their
+// loads they are waited for in front of the weights'): 8 rows 20480 x 4096 14.1 -> 12.6, 20480 x 3072 12.6 -> 11.5; one tile a workgroup gains nothing (0).
+template <int MR, int TILES, bool TAB, int SPW, bool PAIR, int REUSE, bool RAGGED = false, bool SHARE = false, int G = 0>
+__global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !SHARE) ? 4 : 1) void qmv_q4_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint32_t K_, uint32_t ks_, uint32_t M_, uint32_t gs128_, uint32_t tpw_, uint32_t x_bf16_, KParams p) {
   p.w0 = global_at<uint32_t>(w0_); p.s0 = global_at<__half>(s0_); p.b0 = global_at<__half>(b0_); p.x = global_at<__half>(x_); p.K = K_; p.ks = ks_; p.M = M_; p.gs128 = gs128_; p.tpw = tpw_; p.x_bf16 = x_bf16_;
   static_assert(!REUSE || SPW != 0, "reuse needs a uniform slab count");
-  static_assert(!PAIR || TILES == 2, "paired tiles need two tile slots");
+  static_assert(!PAIR || TILES == 2 || SHARE, "paired tiles need two tile slots");
+  static_assert(!SHARE || (PAIR && !TAB && REUSE == 1 && !RAGGED), "one matrix, one pass over K");
   static_assert(!RAGGED || (!TAB && SPW == 0 && REUSE == 0 && (TILES == 1 || PAIR)), "one matrix, guarded loads");
   constexpr int kSlots = 4 * MR;                       // 16-byte activation slots per (slab, j) block ...
   constexpr int kBlk = kSlots + 1;                     // ... followed by one slot of zeros (read by the lanes whose operand rows are empty)
@@ -127,10 +135,11 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
   // ---- which weights: tile tw of this workgroup, k-part kp of every pass --------------------
   const uint32_t K = p.K, KS = p.ks, NT = kWaves / KS;
   const uint32_t kp = wave % KS, tw = wave / KS;
-  // group size 128 (p.gs128): one scale per slab, applied to both halves of it
-  const uint32_t words_per_row = K >> 3, groups_per_row = p.gs128 ? K >> 7 : K >> 6, slabs_total = RAGGED ? (K + 127) >> 7 : K >> 7;
+  // group size 128: one scale per slab, applied to both halves of it
+  const bool gs128 = G == 128 || (G == 0 && p.gs128);
+  const uint32_t words_per_row = K >> 3, groups_per_row = gs128 ? K >> 7 : K >> 6, slabs_total = RAGGED ? (K + 127) >> 7 : K >> 7;
   constexpr bool pair = PAIR;
-  const uint32_t rows_per_slot = pair ? 32u : 16u;  // weight rows (of one matrix) per wave tile slot
+  const uint32_t rows_per_slot = SHARE ? p.tpw : (pair ? 32u : 16u);  // weight rows (of one matrix) per wave tile slot
 
   uint32_t srcs[MR];  // source rows of the activations (wave-uniform)
 #pragma unroll
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
   // ---- tiles of this workgroup: consecutive, so it streams one contiguous block of weight rows.
   //      With one pass over K the activation image (and the sums) staged for the first tile serve
   //      all of them.
-  const uint32_t ntiles = REUSE ? p.tpw : 1u;  // (without reuse the launcher gives every workgroup one tile)
+  const uint32_t ntiles = REUSE && !SHARE ? p.tpw : 1u;  // (without reuse the launcher gives every workgroup one tile)
   // every global load of one tile's slabs sl .. sl+my-1: scales / biases first (the memory counter retires in order)
   auto load_tile = [&](uint32_t wg_tile, int sl, int my, u4 (&sbv)[TILES], u4 (&wreg)[TILES][kSpwMax]) {
     const uint32_t tile_row = (wg_tile * NT + tw) * rows_per_slot;
@@ -214,6 +223,10 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
       const bool first = t == 0 || pair;                       // which matrix
       uint32_t wr = tile_row + n + (pair ? 16 * t : 0);        // which row of it
       if (RAGGED) wr = wr < p.ld_out ? wr : p.ld_out - 1;
+      if (SHARE) {  // (rows past the share repeat its last, unstored)
+        const uint32_t end = tile_row + rows_per_slot < p.ld_out ? tile_row + rows_per_slot : p.ld_out;
+        wr = wr < end ? wr : end - 1;
+      }
       wrow[t] = reinterpret_cast<const u4*>((first ? p.w0 : p.w1) + e_w + (uint64_t)wr * words_per_row) + g;
       // scales live in the lanes with even g, biases in the lanes with odd g (exchanged later)
       const __half* sb = (g & 1) ? (first ? p.b0 : p.b1) : (first ? p.s0 : p.s1);
@@ -223,7 +236,25 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
       sbv[t] = (u4){0u, 0u, 0u, 0u};
-      if (p.gs128) {  // four slabs = four halves; word `it` holds slab it's value twice
+      // (group size 128, as loaded: what spreads them over the slabs would wait for them here, in front of the weights' loads)
+      if constexpr (G == 128) {
+        const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + sl;
+        struct __attribute__((packed, aligned(2))) Pair { uint32_t v; };
+        struct __attribute__((packed, aligned(2))) Four { uint32_t v[2]; };
+        if constexpr (SPW == 4) {
+          const Four v = *reinterpret_cast<const Four*>(hp);
+          sbv[t].x = v.v[0]; sbv[t].y = v.v[1];
+        } else if constexpr (SPW == 3) {
+          sbv[t].x = reinterpret_cast<const Pair*>(hp)->v; sbv[t].y = hp[2];
+        } else {
+          if (my > 0) sbv[t].x = hp[0];
+          if (my > 1) sbv[t].y = hp[1];
+          if (my > 2) sbv[t].z = hp[2];
+          if (my > 3) sbv[t].w = hp[3];
+        }
+        continue;
+      }
+      if (gs128) {  // four slabs = four halves; word `it` holds slab it's value twice
         const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + sl;
         const uint32_t h0 = my > 0 ? hp[0] : 0u, h1 = my > 1 ? hp[1] : 0u, h2 = my > 2 ? hp[2] : 0u, h3 = my > 3 ? hp[3] : 0u;
         sbv[t] = (u4){h0 | (h0 << 16), h1 | (h1 << 16), h2 | (h2 << 16), h3 | (h3 << 16)};
@@ -279,7 +310,20 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
     return (float)__builtin_bit_cast(_Float16, h);
   };
   // the tile's slabs against the staged activations: F += scale * (dot - sum(off*x)) + bias * sum(x)
-  auto compute_tile = [&](int my, const u4 (&sbv)[TILES], const u4 (&wreg)[TILES][kSpwMax], f4 (&F)[TILES]) {
+  auto compute_tile = [&](int my, const u4 (&raw)[TILES], const u4 (&wreg)[TILES][kSpwMax], f4 (&F)[TILES]) {
+    u4 sbv[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      sbv[t] = raw[t];
+      if constexpr (G == 128) {  // word `it` holds slab it's value twice
+        constexpr bool packed = SPW != 0;
+        const uint32_t lo = 0x01000100u, hi = 0x03020302u;
+        sbv[t].x = __builtin_amdgcn_perm(0, raw[t].x, lo);
+        sbv[t].y = packed ? __builtin_amdgcn_perm(0, raw[t].x, hi) : __builtin_amdgcn_perm(0, raw[t].y, lo);
+        sbv[t].z = __builtin_amdgcn_perm(0, packed ? raw[t].y : raw[t].z, lo);
+        sbv[t].w = packed ? __builtin_amdgcn_perm(0, raw[t].y, hi) : __builtin_amdgcn_perm(0, raw[t].w, lo);
+      }
+    }
     // Slab by slab (few live registers).  The per (row, group) sums of the activations come from the matrix
     // unit: columns 0-7 of a constant B operand hold the unpack offsets (1024 for even k, 64 for odd k, in slot
     // order), columns 8-15 hold ones, so accumulator column n < 8 receives sum(off*x) and column n >= 8 sum(x)
@@ -374,6 +418,28 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
   lds_barrier();
   uint32_t tid_t = tid;
   asm volatile("" : "+v"(tid_t));
+  if constexpr (SHARE) {  // (a thread adds up one result: a tile's go to threads of their own)
+    for (uint32_t o = tid_t; o < NT * TILES * 128; o += kThreads) {
+      const uint32_t ot = o >> 7, otw = ot / TILES, t = ot - otw * TILES, m = (o >> 4) & 7, nn = o & 15;
+      const uint32_t r = 16 * t + nn, col = (wg_tile * NT + otw) * rows_per_slot + r;
+      if (m >= rows || r >= rows_per_slot || col >= p.ld_out) continue;
+      float acc = 0.f;
+      if (KS == 8) {
+#pragma unroll
+        for (uint32_t q = 0; q < 8; q += 4) {
+          const float* rp = red + ((q * TILES + t) * 8 + m) * 16 + nn;
+          const float r0 = rp[0], r1 = rp[TILES * 128], r2 = rp[2 * TILES * 128], r3 = rp[3 * TILES * 128];
+          acc += (r0 + r1) + (r2 + r3);
+        }
+      } else {
+        for (uint32_t q = 0; q < KS; ++q) acc += red[(((otw * KS + q) * TILES + t) * 8 + m) * 16 + nn];
+      }
+      const uint64_t at = (uint64_t)(row0 + m) * p.ld_out + col;
+      if (p.out_f32) reinterpret_cast<float*>(p.out)[at] = acc;
+      else reinterpret_cast<__half*>(p.out)[at] = __float2half(acc);
+    }
+    return;
+  }
   for (uint32_t o = tid_t; o < NT * 128; o += kThreads) {
     const uint32_t otw = o >> 7, m = (o >> 4) & 7, nn = o & 15;
     if (m < rows) {
@@ -412,7 +478,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2) ? 4
     reduce_parts_and_store(wg_tile);
   };
 
-  if constexpr (REUSE == 1 && MR < 8) {
+  if constexpr (SHARE || (REUSE == 1 && MR < 8)) {
     // one pass, one tile per workgroup (the launcher gives these kernels no more): straight-line code, which keeps
     // the registers low enough for a third resident workgroup per CU
     const int sl = (int)(kp * SPW);
@@ -514,35 +580,57 @@ void launch_kernel(const KParams& p, dim3 grid, hipStream_t s) {
   Launch<Kernel>::go(grid, dim3(kThreads), 0, s, address(p.w0), address(p.s0), address(p.b0), address(p.x), p.K, p.ks, p.M, p.gs128, p.tpw, p.x_bf16, p);
 }
 
-template <int MR, int TILES, int SPW, bool PAIR>
+template <int MR, int TILES, int SPW, bool PAIR, int G>
 void launch_s(const KParams& p, bool tab, dim3 grid, hipStream_t s) {
   if constexpr (SPW != 0) {
     if (p.K / 128 == p.ks * SPW) {  // one pass over K: the kernels that stage the activations once
       constexpr int kPipe = MR < 8 ? 2 : 1;
       if (p.tpw > 1) {
         if (tab) launch_kernel<qmv_q4_kernel<MR, TILES, true, SPW, PAIR, kPipe>>(p, grid, s);
-        else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, kPipe>>(p, grid, s);
+        else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, kPipe, false, false, G>>(p, grid, s);
       } else {
         if (tab) launch_kernel<qmv_q4_kernel<MR, TILES, true, SPW, PAIR, 1>>(p, grid, s);
-        else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, 1>>(p, grid, s);
+        else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, 1, false, false, G>>(p, grid, s);
       }
       return;
     }
   }
   if (tab) launch_kernel<qmv_q4_kernel<MR, TILES, true, SPW, PAIR, 0>>(p, grid, s);
-  else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, 0>>(p, grid, s);
+  else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, 0, false, false, G>>(p, grid, s);
 }
 
-template <int MR, int TILES, bool PAIR = false>
+template <int MR, int TILES>
+void launch_share(const KParams& p, uint32_t spw, dim3 grid, hipStream_t s) {
+  auto go = [&](auto g) {
+    constexpr int G = decltype(g)::value;
+    if (spw == 4) launch_kernel<qmv_q4_kernel<MR, TILES, false, 4, true, 1, false, true, G>>(p, grid, s);
+    else launch_kernel<qmv_q4_kernel<MR, TILES, false, 3, true, 1, false, true, G>>(p, grid, s);
+  };
+  if (p.gs128) go(std::integral_constant<int, 128>{});
+  else go(std::integral_constant<int, 64>{});
+}
+void launch_share_rows(const KParams& p, int mr, uint32_t spw, uint32_t tiles, dim3 grid, hipStream_t s) {
+  auto go = [&](auto m) {
+    constexpr int MR = decltype(m)::value;
+    if (tiles == 2) launch_share<MR, 2>(p, spw, grid, s);
+    else if (tiles == 3) launch_share<MR, 3>(p, spw, grid, s);
+    else if constexpr (MR < 8) launch_share<MR, 4>(p, spw, grid, s);
+  };
+  if (mr == 2) go(std::integral_constant<int, 2>{});
+  else if (mr == 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 8>{});
+}
+
+template <int MR, int TILES, bool PAIR = false, int G = 0>
 void launch_t(const KParams& p, bool tab, dim3 grid, hipStream_t s) {
   // uniform slab count per wave and pass?
   const uint32_t slabs = p.K / 128, per_pass = p.ks * kSpwMax;
   int spw = 0;
   if (slabs % per_pass == 0) spw = 4;
   else if (slabs < per_pass && slabs % p.ks == 0 && slabs / p.ks == 3) spw = 3;
-  if (spw == 4) launch_s<MR, TILES, 4, PAIR>(p, tab, grid, s);
-  else if (spw == 3) launch_s<MR, TILES, 3, PAIR>(p, tab, grid, s);
-  else launch_s<MR, TILES, 0, PAIR>(p, tab, grid, s);
+  if (spw == 4) launch_s<MR, TILES, 4, PAIR, G>(p, tab, grid, s);
+  else if (spw == 3) launch_s<MR, TILES, 3, PAIR, G>(p, tab, grid, s);
+  else launch_s<MR, TILES, 0, PAIR, G>(p, tab, grid, s);
 }
 
 __global__ void build_gather_chunks_kernel(const uint32_t* indices, uint32_t batch, uint32_t mpb,
@@ -646,6 +734,26 @@ int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s) {
   const uint32_t tiles_x = a.N / (16 * nt * (pair ? 2 : 1));
   uint32_t tpw = 1;
   const bool uniform_single_pass = slabs == ks * kSpwMax || slabs == ks * 3;  // the kernels with a fixed slab count
+  // Equal shares: one workgroup per CU with a share of the rows, as up to four tiles side by side whose weights are all requested at once.  The
+  // activations (as many bytes as a tile of weights at four rows, twice that at eight) then pass the address unit once per CU instead of
+  // once per tile, and no CU has a tile more than another.  us, a tile (8 rows: two) per workgroup / shares:
+  //   K = 4096, N = 4608 / 5120 / 6144 / 9216 / 11008 / 14336 / 16384: 2 rows 6.0 / 5.7, 6.1 / 5.8, 6.2 / 6.0, -, 8.0 / 7.6, 9.3 / 9.1, 10.3 / 9.7;
+  //     4 rows 6.4 / 5.9, 6.4 / 6.0, 6.6 / 6.1, 8.2 / 7.3, 8.5 / 7.7, 10.3 / 9.4, 10.8 / 9.9; 8 rows 7.3 / 6.3, 7.4 / 6.4, 7.5 / 6.5, 9.3 / 7.6, 9.4 / 8.2,
+  //     9.7 / 9.8, 10.2 / 10.4: up to three tiles; group size 128, 9216 / 12288: 4 rows 7.6 / 7.0, 8.0 / 7.6, 8 rows 9.6 / 7.2, 9.7 / 7.8;
+  //   K = 3072, up to 4 rows: only where the tiles leave many CUs without a last one: 3 rows 9216 / 12288 / 14336 6.7 / 6.5, 7.1 / 7.5, 8.7 / 8.2, group
+  //     size 128 6.6 / 6.4, 6.8 / 7.2; 2 rows 14336 7.6 / 8.0;
+  //   shorter rows (several waves' tiles beside each other): 3 rows 14336 x 2048 6.5 / 6.6, 14336 x 1536 5.6 / 5.7, 14336 x 1024 4.8 / 5.0;
+  //     6 rows 9216 x 3072 8.2 / 6.9, 9216 x 2048 7.1 / 6.3, 14336 x 1536 6.3 / 6.0, 14336 x 1024 5.2 / 5.3;
+  //   one tile a workgroup (3072 rows as shares of 12): 3 rows, K = 3072 4.1 / 4.2; pairs that make one even round: 8 rows 8192 x 4096 6.7 / 6.8, 16384 x 1536 6.1 / 6.2.
+  const uint32_t cus = ctx().num_cus, share = (a.N + cus * nt - 1) / (cus * nt), tiles_share = (share + 15) / 16, last_round = tiles_x % cus;
+  if (uniform_single_pass && !tab && !a.dual && chunks == 1 && a.ld_out == a.N && mr >= 2 &&
+      (mr < 8 ? (a.K >= 4096 || (mr == 4 && !p.gs128 && a.K >= 3072 && last_round != 0 && last_round * 10 <= cus * 7)) && tiles_share >= 2 && tiles_share <= 4
+              : a.K >= 1536 && tiles_share >= 2 && tiles_share <= 3 && !(pair && tiles_x <= cus))) {
+    p.tpw = share;
+    launch_share_rows(p, mr, slabs / ks, tiles_share, dim3((a.N + share * nt - 1) / (share * nt)), s);
+    RMLX_HIP_CHECK(take_launch_error());
+    return RMLX_OK;
+  }
   if (uniform_single_pass) {
     // With a chunk table, consecutive chunks often belong to one expert (more than 8 rows): a grid
     // width that is a multiple of the 8 XCDs puts their workgroups for the same tiles on one XCD,
@@ -659,7 +767,8 @@ int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s) {
   p.tpw = tpw;
   dim3 grid(tiles_x / tpw, chunks);
   if (pair) {
-    launch_t<8, 2, true>(p, tab, grid, s);
+    if (p.gs128 && !tab) launch_t<8, 2, true, 128>(p, tab, grid, s);
+    else launch_t<8, 2, true>(p, tab, grid, s);
   } else if (a.dual) {
     switch (mr) {
       case 1: launch_t<1, 2>(p, tab, grid, s); break;

@@ -1,0 +1,29 @@
+"""Multi-row GEMV with an equal share of the weight rows per CU (qmv.hip, SHARE) at the edges of its tiles, against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import model
+from tests.helpers import assert_close, make_weight, make_x, x_as_f64
+from tests.test_gpu_precision import _ratio
+
+pytestmark = pytest.mark.gpu
+
+
+# On 256 CUs, shares of one row in the last tile and of whole tiles, two to four of them, the last workgroup with fewer rows or all of its own; one
+# to four waves' tiles side by side, three and four slabs a wave; the row counts that begin and end each build (five to eight rows: up to three tiles).
+@pytest.mark.parametrize("k,gs", [(4096, 64), (4096, 128), (3072, 64), (2048, 64), (1536, 128)])
+@pytest.mark.parametrize("m,dtype", [(2, "f16"), (3, "bf16"), (4, "f16"), (5, "f16"), (8, "bf16")])
+@pytest.mark.parametrize("share", [17, 32, 33, 48, 49, 64])
+def test_shares(hip, k, gs, m, dtype, share):
+    from rmlx_amd import ops, runtime as rt
+    side = 1 if k >= 3072 else 2
+    n = (256 * side * (share - 1) // 16 + 1) * 16 if share % 16 == 1 else 256 * side * share
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, 4, gs)
+    x = make_x(rng, m, k, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    out = ops.affine_quantized_matmul_batched(xd, ops.QuantizedWeight.from_numpy(*w, gs, 4), kernel=rt.KERNEL_QMV_ROWS).numpy()
+    rows = np.unique(np.concatenate([np.arange(200), np.arange(0, n, 61), np.arange(share - 2, n, 7 * share), np.arange(n - 200, n)]))
+    ref = model.qmm(x_as_f64(x, dtype).astype(np.float16).astype(np.float64), *(a[rows] for a in w), gs, 4)
+    assert_close(out[:, rows], ref)
+    assert _ratio(out[:, rows], ref) < 1.05
