@@ -97,8 +97,8 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
   p.w0 = global_at<uint32_t>(w0_); p.s0 = global_at<__half>(s0_); p.b0 = global_at<__half>(b0_); p.x = global_at<__half>(x_); p.K = K_; p.ks = ks_; p.M = M_; p.gs128 = gs128_; p.tpw = tpw_; p.x_bf16 = x_bf16_;
   static_assert(!REUSE || SPW != 0, "reuse needs a uniform slab count");
   static_assert(!PAIR || TILES == 2 || SHARE, "paired tiles need two tile slots");
-  static_assert(!SHARE || (PAIR && !TAB && REUSE == 1 && !RAGGED), "one matrix, one pass over K");
-  static_assert(!RAGGED || (!TAB && SPW == 0 && REUSE == 0 && (TILES == 1 || PAIR)), "one matrix, guarded loads");
+  static_assert(!SHARE || (PAIR && !TAB && REUSE == 1 && G != 0), "one matrix, one pass over K");
+  static_assert(!RAGGED || SHARE || (!TAB && SPW == 0 && REUSE == 0 && (TILES == 1 || PAIR)), "one matrix, guarded loads");
   constexpr int kSlots = 4 * MR;                       // 16-byte activation slots per (slab, j) block ...
   constexpr int kBlk = kSlots + 1;                     // ... followed by one slot of zeros (read by the lanes whose operand rows are empty)
   constexpr int kXsWave = kSpwMax * 4 * kBlk * 16;     // bytes of activation image per wave
@@ -207,6 +207,11 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
   //      With one pass over K the activation image (and the sums) staged for the first tile serve
   //      all of them.
   const uint32_t ntiles = REUSE && !SHARE ? p.tpw : 1u;  // (without reuse the launcher gives every workgroup one tile)
+  // SHARE, guarded: where the loads of the scales of slabs sl .. begin, so that none reads past the row
+  auto first_group = [&](int sl, int my) -> int {
+    const int per = G == 128 ? 1 : 2, last = (int)groups_per_row - my * per;
+    return sl * per < last ? sl * per : last;
+  };
   // every global load of one tile's slabs sl .. sl+my-1: scales / biases first (the memory counter retires in order)
   auto load_tile = [&](uint32_t wg_tile, int sl, int my, u4 (&sbv)[TILES], u4 (&wreg)[TILES][kSpwMax]) {
     const uint32_t tile_row = (wg_tile * NT + tw) * rows_per_slot;
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
       sbv[t] = (u4){0u, 0u, 0u, 0u};
       // (group size 128, as loaded: what spreads them over the slabs would wait for them here, in front of the weights' loads)
       if constexpr (G == 128) {
-        const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + sl;
+        const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + (SHARE && RAGGED ? first_group(sl, my) : sl);
         struct __attribute__((packed, aligned(2))) Pair { uint32_t v; };
         struct __attribute__((packed, aligned(2))) Four { uint32_t v[2]; };
         if constexpr (SPW == 4) {
@@ -262,6 +267,19 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
       }
       if constexpr (RAGGED) {  // (rows of an odd number of groups begin at any even address)
         struct __attribute__((packed, aligned(2))) Pair { uint32_t v; };
+        if constexpr (SHARE) {  // (groups past the row: shifted out by the products, no branch between these loads and the weights')
+          const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + first_group(sl, my);
+          struct __attribute__((packed, aligned(2))) Four { uint32_t v[4]; };
+          struct __attribute__((packed, aligned(2))) Two { uint32_t v[2]; };
+          if (my == kSpwMax) {
+            const Four v = *reinterpret_cast<const Four*>(hp);
+            sbv[t] = (u4){v.v[0], v.v[1], v.v[2], v.v[3]};
+          } else {
+            const Two v = *reinterpret_cast<const Two*>(hp);
+            sbv[t].x = v.v[0]; sbv[t].y = v.v[1]; sbv[t].z = reinterpret_cast<const Pair*>(hp + 4)->v;
+          }
+          continue;
+        }
         const unsigned short* hp = reinterpret_cast<const unsigned short*>(sbrow[t]) + 2 * sl;
 #pragma unroll
         for (int it = 0; it < kSpwMax; ++it) {
@@ -310,18 +328,29 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
     return (float)__builtin_bit_cast(_Float16, h);
   };
   // the tile's slabs against the staged activations: F += scale * (dot - sum(off*x)) + bias * sum(x)
-  auto compute_tile = [&](int my, const u4 (&raw)[TILES], const u4 (&wreg)[TILES][kSpwMax], f4 (&F)[TILES]) {
+  auto compute_tile = [&](int sl, int my, const u4 (&raw)[TILES], const u4 (&wreg)[TILES][kSpwMax], f4 (&F)[TILES]) {
     u4 sbv[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
       sbv[t] = raw[t];
+      if constexpr (SHARE && RAGGED) {
+        const int past = sl * (G == 128 ? 1 : 2) - first_group(sl, my);  // groups
+        if (past > 0) {
+          u4 v = sbv[t];
+          if (past & 1) v = (u4){__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16), __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16};
+          if (past & 2) v = (u4){v.y, v.z, v.w, 0u};
+          if (past & 4) v = (u4){v.z, v.w, 0u, 0u};
+          sbv[t] = past < 8 ? v : (u4){0u, 0u, 0u, 0u};
+        }
+      }
       if constexpr (G == 128) {  // word `it` holds slab it's value twice
         constexpr bool packed = SPW != 0;
         const uint32_t lo = 0x01000100u, hi = 0x03020302u;
-        sbv[t].x = __builtin_amdgcn_perm(0, raw[t].x, lo);
-        sbv[t].y = packed ? __builtin_amdgcn_perm(0, raw[t].x, hi) : __builtin_amdgcn_perm(0, raw[t].y, lo);
-        sbv[t].z = __builtin_amdgcn_perm(0, packed ? raw[t].y : raw[t].z, lo);
-        sbv[t].w = packed ? __builtin_amdgcn_perm(0, raw[t].y, hi) : __builtin_amdgcn_perm(0, raw[t].w, lo);
+        const uint32_t r0 = sbv[t].x, r1 = sbv[t].y;
+        sbv[t].x = __builtin_amdgcn_perm(0, r0, lo);
+        sbv[t].y = packed ? __builtin_amdgcn_perm(0, r0, hi) : __builtin_amdgcn_perm(0, r1, lo);
+        sbv[t].z = __builtin_amdgcn_perm(0, packed ? r1 : sbv[t].z, lo);
+        sbv[t].w = packed ? __builtin_amdgcn_perm(0, r1, hi) : __builtin_amdgcn_perm(0, sbv[t].w, lo);
       }
     }
     // Slab by slab (few live registers).  The per (row, group) sums of the activations come from the matrix
@@ -494,7 +523,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
     f4 F[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) F[t] = (f4){0.f, 0.f, 0.f, 0.f};
-    compute_tile(SPW, sbv, wreg, F);
+    compute_tile(sl, SPW, sbv, wreg, F);
     finish_tile(blockIdx.x, F, true);
   } else if constexpr (REUSE == 1) {
     // one pass: slabs kp*SPW .. of every tile; the activations and the first tile's weights are requested together.
@@ -519,7 +548,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
       f4 F[TILES];
 #pragma unroll
       for (int t = 0; t < TILES; ++t) F[t] = (f4){0.f, 0.f, 0.f, 0.f};
-      compute_tile(SPW, sbv, wreg, F);
+      compute_tile(sl, SPW, sbv, wreg, F);
       reduce_halves(F);
       if (ti + 1 < ntiles) load_tile(first + ti + 1, sl, SPW, sbv, wreg);
       reduce_parts_and_store(first + ti);
@@ -541,13 +570,13 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
       if (ti + 1 < ntiles) load_tile(first + ti + 1, sl, SPW, sbv_b, wreg_b);
 #pragma unroll
       for (int t = 0; t < TILES; ++t) F[t] = (f4){0.f, 0.f, 0.f, 0.f};
-      compute_tile(SPW, sbv_a, wreg_a, F);
+      compute_tile(sl, SPW, sbv_a, wreg_a, F);
       finish_tile(first + ti, F, ti == 0);
       if (ti + 1 < ntiles) {
         if (ti + 2 < ntiles) load_tile(first + ti + 2, sl, SPW, sbv_a, wreg_a);
 #pragma unroll
         for (int t = 0; t < TILES; ++t) F[t] = (f4){0.f, 0.f, 0.f, 0.f};
-        compute_tile(SPW, sbv_b, wreg_b, F);
+        compute_tile(sl, SPW, sbv_b, wreg_b, F);
         finish_tile(first + ti + 1, F, false);
       }
     }
@@ -569,7 +598,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
       u4 wreg[TILES][kSpwMax];
       load_tile(wg_tile, sl, my, sbv, wreg);
       stage_x(xv);
-      compute_tile(my, sbv, wreg, F);
+      compute_tile(sl, my, sbv, wreg, F);
     }
     finish_tile(wg_tile, F, true);
   }
@@ -599,22 +628,27 @@ void launch_s(const KParams& p, bool tab, dim3 grid, hipStream_t s) {
   else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, 0, false, false, G>>(p, grid, s);
 }
 
+// spw: slabs of a wave; guarded: some waves have fewer, or K ends in the middle of one
 template <int MR, int TILES>
-void launch_share(const KParams& p, uint32_t spw, dim3 grid, hipStream_t s) {
-  auto go = [&](auto g) {
-    constexpr int G = decltype(g)::value;
-    if (spw == 4) launch_kernel<qmv_q4_kernel<MR, TILES, false, 4, true, 1, false, true, G>>(p, grid, s);
-    else launch_kernel<qmv_q4_kernel<MR, TILES, false, 3, true, 1, false, true, G>>(p, grid, s);
+void launch_share(const KParams& p, uint32_t spw, bool guarded, dim3 grid, hipStream_t s) {
+  auto go = [&](auto spw_c, auto g) {
+    constexpr int SPW = decltype(spw_c)::value, G = decltype(g)::value;
+    if (!guarded) launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, false, true, G>>(p, grid, s);
+    else if constexpr (MR >= 4) launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, true, true, G>>(p, grid, s);
   };
-  if (p.gs128) go(std::integral_constant<int, 128>{});
-  else go(std::integral_constant<int, 64>{});
+  auto with = [&](auto g) {
+    if (spw == 4) go(std::integral_constant<int, 4>{}, g);
+    else go(std::integral_constant<int, 3>{}, g);
+  };
+  if (p.gs128) with(std::integral_constant<int, 128>{});
+  else with(std::integral_constant<int, 64>{});
 }
-void launch_share_rows(const KParams& p, int mr, uint32_t spw, uint32_t tiles, dim3 grid, hipStream_t s) {
+void launch_share_rows(const KParams& p, int mr, uint32_t spw, bool guarded, uint32_t tiles, dim3 grid, hipStream_t s) {
   auto go = [&](auto m) {
     constexpr int MR = decltype(m)::value;
-    if (tiles == 2) launch_share<MR, 2>(p, spw, grid, s);
-    else if (tiles == 3) launch_share<MR, 3>(p, spw, grid, s);
-    else if constexpr (MR < 8) launch_share<MR, 4>(p, spw, grid, s);
+    if (tiles == 2) launch_share<MR, 2>(p, spw, guarded, grid, s);
+    else if (tiles == 3) launch_share<MR, 3>(p, spw, guarded, grid, s);
+    else if constexpr (MR < 8) launch_share<MR, 4>(p, spw, guarded, grid, s);
   };
   if (mr == 2) go(std::integral_constant<int, 2>{});
   else if (mr == 4) go(std::integral_constant<int, 4>{});
@@ -671,6 +705,40 @@ bool qmv_q4_ragged_supported(uint32_t N, uint32_t K, uint32_t group_size) {
   return (group_size == 64 || group_size == 128) && N > 0 && K > 0 && K % group_size == 0;
 }
 
+// Shares (the line of launch_qmv_q4) of a K whose slabs are not the same for all waves, or of any N, with clamped loads: zeros for the
+// activations and scales past the row.  us, a tile (8 rows: two) per workgroup / shares:
+//   3, 4 rows, two tiles a share: 4608 x 3840 / 2560 6.4 / 5.7, 5.3 / 4.5; 8192 x 3840 / 3200 / 2560 6.9 / 6.7, 6.3 / 6.3, 6.0 / 5.7; 4800 x 2880 6.2 / 5.1;
+//     9216 x 1984 7.3 / 6.0; 12288 x 1088 5.8 / 5.1; three, where the third is small: 9216 x 4032 / 2880 9.5 / 9.0, 7.8 / 7.0, else off the multiples of 128 or 16 at
+//     most: 11008 x 3200 7.6 / 8.0, 20480 x 1792 7.8 / 8.4, 12288 x 2880 8.1 / 8.0, 12288 x 4032 9.9 / 10.7; four: 14336 x 3200 8.9 / 10.0;
+//   5 to 8 rows, up to three tiles: 8 rows 4608 x 3840 7.5 / 6.0, 8192 x 2560 6.7 / 6.1, 11008 x 3840 11.0 / 8.9, 20480 x 1280 8.9 / 7.3; 6 rows 4800 x 2880 6.6 / 5.4,
+//     9216 x 1984 7.9 / 6.3, 20000 x 1088 9.1 / 7.0.
+struct SharePlan { uint32_t ks, rows, tiles; };
+static bool guarded_share_plan(uint32_t M, uint32_t N, uint32_t K, SharePlan* out) {
+  const uint32_t cus = ctx().num_cus, slabs = (K + 127) / 128;
+  if (M < 3 || M > 8 || slabs < 9 || slabs > 8 * kSpwMax || cus == 0) return false;
+  SharePlan s{1, 0, 0};
+  while (s.ks < 8 && s.ks * kSpwMax < slabs) s.ks *= 2;
+  const uint32_t wide = cus * (8 / s.ks);
+  s.rows = (uint32_t)(((uint64_t)N + wide - 1) / wide);
+  s.tiles = (s.rows + 15) / 16;
+  *out = s;
+  if (M > 4) return s.tiles == 2 || s.tiles == 3;
+  return s.tiles == 2 || (s.tiles == 3 && (s.rows <= 36 || ((K % 128 != 0 || N % 16 != 0) && K <= 3072)));
+}
+bool qmv_q4_takes_shares(uint32_t M, uint32_t N, uint32_t K) {
+  SharePlan plan;
+  return guarded_share_plan(M, N, K, &plan);
+}
+static bool guarded_shares(KParams& p, const QmvArgs& a, int mr, hipStream_t s) {
+  SharePlan plan;
+  if (!guarded_share_plan(a.M, a.N, a.K, &plan)) return false;
+  p.ks = plan.ks;
+  p.tpw = plan.rows;
+  const uint32_t nt = 8 / plan.ks, slabs = (a.K + 127) / 128;
+  launch_share_rows(p, mr, (slabs + plan.ks - 1) / plan.ks, true, plan.tiles, dim3((a.N + plan.rows * nt - 1) / (plan.rows * nt)), s);
+  return true;
+}
+
 // Rows of x over a matrix off the multiples above: one tile of 16 or, where those fill the chip, 32 weight rows per wave.
 int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s) {
   if (!qmv_q4_ragged_supported(a.N, a.K, a.group_size) || a.dual || a.chunk_tab != nullptr || a.out_f32 || a.ld_out != a.N)
@@ -683,6 +751,10 @@ int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s) {
   p.K = a.K; p.ld_out = a.ld_out; p.M = a.M;
   p.gs128 = a.group_size == 128 ? 1u : 0u;
   p.x_bf16 = a.x_bf16 ? 1u : 0u;
+  if (guarded_shares(p, a, a.M > 4 ? 8 : 4, s)) {
+    RMLX_HIP_CHECK(take_launch_error());
+    return RMLX_OK;
+  }
   p.tpw = 1;
   p.ks = 1;
   while (p.ks < 8 && p.ks * kSpwMax * 128 < a.K) p.ks *= 2;
@@ -750,7 +822,11 @@ int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s) {
       (mr < 8 ? (a.K >= 4096 || (mr == 4 && !p.gs128 && a.K >= 3072 && last_round != 0 && last_round * 10 <= cus * 7)) && tiles_share >= 2 && tiles_share <= 4
               : a.K >= 1536 && tiles_share >= 2 && tiles_share <= 3 && !(pair && tiles_x <= cus))) {
     p.tpw = share;
-    launch_share_rows(p, mr, slabs / ks, tiles_share, dim3((a.N + share * nt - 1) / (share * nt)), s);
+    launch_share_rows(p, mr, slabs / ks, false, tiles_share, dim3((a.N + share * nt - 1) / (share * nt)), s);
+    RMLX_HIP_CHECK(take_launch_error());
+    return RMLX_OK;
+  }
+  if (!uniform_single_pass && !tab && !a.dual && a.ld_out == a.N && mr >= 4 && guarded_shares(p, a, mr, s)) {
     RMLX_HIP_CHECK(take_launch_error());
     return RMLX_OK;
   }

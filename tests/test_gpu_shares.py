@@ -27,3 +27,23 @@ def test_shares(hip, k, gs, m, dtype, share):
     ref = model.qmm(x_as_f64(x, dtype).astype(np.float16).astype(np.float64), *(a[rows] for a in w), gs, 4)
     assert_close(out[:, rows], ref)
     assert _ratio(out[:, rows], ref) < 1.05
+
+
+# K of waves with fewer slabs than others, with none, that ends in the middle of a slab; one to four waves' tiles side by side; N of any kind
+@pytest.mark.parametrize("k,gs", [(3968, 64), (3648, 64), (2880, 64), (2304, 128), (2176, 64), (1984, 64), (1088, 64), (896, 128)])
+@pytest.mark.parametrize("m,dtype", [(3, "f16"), (4, "bf16"), (5, "bf16"), (8, "f16")])
+@pytest.mark.parametrize("share,odd", [(17, 5), (32, 0), (33, 16), (48, 37), (49, 1), (64, 7)])
+def test_guarded_shares(hip, k, gs, m, dtype, share, odd):
+    from rmlx_amd import ops, runtime as rt
+    side = 1 if k > 2048 else (2 if k > 1024 else 4)
+    n = 256 * side * (share - 1) + 256 * side - odd if odd != 1 else 256 * side * (share - 1) + 1
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, 4, gs)
+    x = make_x(rng, m, k, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    kernel = rt.KERNEL_QMV_ROWS if n % 16 == 0 and k % 128 == 0 else rt.KERNEL_QMV_RAGGED
+    out = ops.affine_quantized_matmul_batched(xd, ops.QuantizedWeight.from_numpy(*w, gs, 4), kernel=kernel).numpy()
+    rows = np.unique(np.concatenate([np.arange(200), np.arange(0, n, 61), np.arange(share - 2, n, 7 * share), np.arange(n - 200, n)]))
+    ref = model.qmm(x_as_f64(x, dtype).astype(np.float16).astype(np.float64), *(a[rows] for a in w), gs, 4)
+    assert_close(out[:, rows], ref)
+    assert _ratio(out[:, rows], ref) < 1.05
