@@ -28,6 +28,7 @@
 #include "launch.hpp"
 #include "q4_stream.hpp"
 #include "tile.hpp"
+#include "unbounded.hpp"
 
 namespace rmlx {
 namespace {
@@ -163,35 +164,6 @@ struct RingArgs {
   RingParams p;
 };
 static_assert(offsetof(RingArgs, geometry) == 44 && offsetof(RingArgs, p) == 64, "the kernel's parameters, one behind another");
-// 8 activations as the products take them
-__device__ __forceinline__ h8 x_piece(const char* x, int32_t x_dtype, uint32_t k) {
-  if (x_dtype == RMLX_DTYPE_F32) {
-    h8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (_Float16)reinterpret_cast<const float*>(x)[k + e];
-    return v;
-  }
-  const u4 d = *reinterpret_cast<const u4*>(x + k * 2);
-  return __builtin_bit_cast(h8, x_dtype == RMLX_DTYPE_BF16 ? q4::bf16x8_to_f16(d) : d);
-}
-// (scale * q + bias) * x of a row in f32, over n pieces of 8: those that the list names, or all of them.
-template <int BITS, int GS>
-__device__ __forceinline__ float plain_sum(const char* w, const __half* s, const __half* b, const char* x, int32_t x_dtype, const uint16_t* list, uint32_t n) {
-  float sum = 0.f;
-#pragma unroll 1
-  for (uint32_t i = 0; i < n && sum == sum; ++i) {
-    const uint32_t k = (list != nullptr ? list[i] : i) * 8;
-    const float sc = (float)s[k / GS], bi = (float)b[k / GS];
-    const h8 v = x_piece(x, x_dtype, k);
-    const uint32_t* q = reinterpret_cast<const uint32_t*>(w + k * BITS / 8);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t v_q = BITS == 4 ? q[0] >> (4 * e) & 15u : q[e >> 2] >> (8 * (e & 3)) & 255u;
-      sum = fmaf(fmaf((float)v_q, sc, bi), (float)v[e], sum);
-    }
-  }
-  return sum;
-}
 // Offsets and biases of both signs make a NaN of an infinite activation, (1024 + q) inf - 1024 inf, where the sum of the products is an
 // infinity (f32 and bf16 values past the range of f16 are infinities here too).  A wave that has stored a result that is not finite comes
 // here at its end and goes over the results of such rows once more, over the pieces of the row that are not finite (the others do not change
@@ -244,27 +216,14 @@ __device__ __forceinline__ void store_unbounded(char* lds, bool spoiled, uint32_
       if constexpr (MODE == GATHER) m = from = __builtin_amdgcn_readlane(seg_row, seg * 16 + i);
       else if (MODE != DENSE && a->p.row_map != nullptr) from = uni(a->p.row_map[m]);
       const char* const x = a->x + (uint64_t)from * (K << (x_dtype == RMLX_DTYPE_F32 ? 2 : 1));
-      uint32_t n = 0;
-#pragma unroll 1
-      for (uint32_t k = 0; k < K; k += 512) {
-        bool odd = false;
-        if (k + lane * 8 < K) {
-          const h8 v = x_piece(x, x_dtype, k + lane * 8);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) odd = odd || !__builtin_isfinite((float)v[e]);
-        }
-        const uint64_t mask = __builtin_amdgcn_ballot_w64(odd);
-        if (odd) list[n + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0))] = (uint16_t)(k / 8 + lane);
-        n += (uint32_t)__builtin_popcountll(mask);
-      }
-      wait_lds();
+      const uint32_t n = q4::odd_pieces(x, x_dtype, K, lane, list);
 #pragma unroll 1
       for (uint32_t r = mine ? r0 + out_c : r1; r < r1; r += 16u << nt_log2) {
         auto sum_of = [&](bool up, bool whole) {
           const RingArgsPtr a = args();
           const uint64_t at = (uint64_t)r * (K / GS) + expert * a->p.estride_s;
           const char* const w = reinterpret_cast<const char*>(up ? a->p.w1 : a->w0) + expert * a->p.estride_w * 4 + (uint64_t)r * (K * BITS / 8);
-          return plain_sum<BITS, GS>(w, (up ? a->p.s1 : a->s0) + at, (up ? a->p.b1 : a->b0) + at, x, x_dtype, whole ? nullptr : list, whole ? K / 8 : n);
+          return q4::plain_sum<BITS>(GS == 32 ? 5 : (GS == 64 ? 6 : 7), w, (up ? a->p.s1 : a->s0) + at, (up ? a->p.b1 : a->b0) + at, x, x_dtype, whole ? nullptr : list, whole ? K / 8 : n);
         };
         float v = sum_of(false, n == 0);
         if constexpr (MODE == PAIR) {

@@ -9,9 +9,13 @@ from tests.test_gpu_ring import _assert_same_class, _unbounded
 pytestmark = pytest.mark.gpu
 
 
-# Aligned shapes that the slot-streaming kernel takes from the multi-row GEMV: 3 and 4 rows from 30 MiB on, more rows from 18.
-@pytest.mark.parametrize("m,n,k,gs,dtype", [(4, 22528, 3328, 64, "f16"), (3, 28672, 3200, 128, "bf16"), (4, 28672, 3328, 64, "f32"), (3, 23040, 2816, 64, "f32"),
-                                            (6, 12288, 4032, 64, "f16")])
+# Shapes that the slot-streaming kernel and the multi-row GEMVs share among them, both sides of the lines: equal shares of the weight rows per CU (with
+# whole and with clamped loads, two and three tiles, one and two waves' tiles beside each other), and the slot-streaming kernel.
+@pytest.mark.parametrize("m,n,k,gs,dtype", [(8, 11008, 3840, 64, "f16"), (8, 12288, 3200, 128, "bf16"), (8, 9001, 4096, 64, "f32"), (8, 24001, 1984, 64, "bf16"),
+                                            (7, 9216, 2880, 64, "f16"), (6, 9216, 2880, 64, "f32"), (5, 16001, 1088, 64, "f16"), (6, 12001, 4032, 64, "bf16"),
+                                            (4, 16001, 1984, 64, "f16"), (3, 9001, 4096, 128, "f16"), (4, 22528, 3328, 64, "f16"), (3, 28672, 3200, 128, "bf16"),
+                                            (4, 28672, 3328, 64, "f32"), (3, 23040, 2816, 64, "f32"), (6, 15680, 1088, 64, "f16"), (4, 9216, 4096, 64, "f16"),
+                                            (8, 9216, 4096, 128, "bf16"), (8, 9216, 2880, 64, "f16"), (6, 12288, 4032, 64, "f16")])
 def test_infinite_activations(hip, m, n, k, gs, dtype):
     from rmlx_amd import ops, runtime as rt
     rng = np.random.default_rng(m + n + k)
@@ -34,7 +38,7 @@ def test_infinite_activations(hip, m, n, k, gs, dtype):
         assert_close(out[np.ix_(rest, cols)], model.qmm(x16[rest].astype(np.float64), *part, gs, 4))
 
 
-@pytest.mark.parametrize("m,n,k,gs", [(4, 22528, 3328, 64), (3, 28672, 3200, 128)])
+@pytest.mark.parametrize("m,n,k,gs", [(8, 9001, 4096, 64), (4, 9216, 4096, 128), (6, 9216, 2880, 64), (4, 22528, 3328, 64), (3, 28672, 3200, 128)])
 def test_infinite_scales_and_biases(hip, m, n, k, gs):
     from rmlx_amd import ops, runtime as rt
     rng = np.random.default_rng(n)
