@@ -151,8 +151,8 @@ int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s);
 bool qmv_q4_supported(uint32_t N, uint32_t K, uint32_t group_size);
 // The same over any N and any K of whole groups (64 or 128): plain matrices, f16 output
 bool qmv_q4_ragged_supported(uint32_t N, uint32_t K, uint32_t group_size);
-// (whether 3 to 8 rows, off the multiples of the kernels with a fixed slab count, are taken as an equal share of weight rows per CU)
-bool qmv_q4_takes_shares(uint32_t M, uint32_t N, uint32_t K);
+// (whether both take the rows as an equal share of weight rows per CU)
+bool qmv_q4_takes_shares(uint32_t M, uint32_t N, uint32_t K, uint32_t group_size);
 int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s);
 // Gate / up projection of single rows through chosen experts (qmv_m1.hip): position a = activation row a / top_k (x, no
 // row map) through expert idx[a] (idx == null: pick a % top_k of the ranking the kernel makes itself, see route_logits) of the two stacked matrices of `a` (w0 / w1, expert strides), out[a, :] = silu(gate) * up

@@ -665,31 +665,45 @@ void launch_s(const KParams& p, bool tab, dim3 grid, hipStream_t s) {
   else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, PAIR, 0, false, false, G>>(p, grid, s);
 }
 
-// spw: slabs of a wave; guarded: some waves have fewer, or K ends in the middle of one
-template <int MR, int TILES>
-void launch_share(const KParams& p, uint32_t spw, bool guarded, dim3 grid, hipStream_t s) {
-  auto go = [&](auto spw_c, auto g) {
-    constexpr int SPW = decltype(spw_c)::value, G = decltype(g)::value;
-    if (!guarded) launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, false, true, G>>(p, grid, s);
-    else if constexpr (MR >= 4) launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, true, true, G>>(p, grid, s);
-  };
-  auto with = [&](auto g) {
-    if (spw == 4) go(std::integral_constant<int, 4>{}, g);
-    else go(std::integral_constant<int, 3>{}, g);
-  };
-  if (p.gs128) with(std::integral_constant<int, 128>{});
-  else with(std::integral_constant<int, 64>{});
+// Rows taken as equal shares: a row's slabs over ks waves, spw a wave; rows: weight rows of a wave's share, in tiles of 16; guarded: some waves have
+// fewer slabs, K ends in the middle of one, or N is no multiple of 16.
+struct SharePlan { uint32_t ks, spw, rows, tiles; bool guarded; };
+
+// false: no kernel for the plan (share_plan makes none of these)
+template <int MR, int TILES, int SPW, int G>
+bool launch_share(const KParams& p, bool guarded, dim3 grid, hipStream_t s) {
+  if constexpr (MR >= 4 && TILES <= 3) {
+    if (guarded) { launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, true, true, G>>(p, grid, s); return true; }
+  }
+  if constexpr (SPW == 4 || MR == 8 || (MR == 4 && G == 64)) {
+    if (!guarded) { launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, false, true, G>>(p, grid, s); return true; }
+  }
+  return false;
 }
-void launch_share_rows(const KParams& p, int mr, uint32_t spw, bool guarded, uint32_t tiles, dim3 grid, hipStream_t s) {
-  auto go = [&](auto m) {
-    constexpr int MR = decltype(m)::value;
-    if (tiles == 2) launch_share<MR, 2>(p, spw, guarded, grid, s);
-    else if (tiles == 3) launch_share<MR, 3>(p, spw, guarded, grid, s);
-    else if constexpr (MR < 8) launch_share<MR, 4>(p, spw, guarded, grid, s);
-  };
-  if (mr == 2) go(std::integral_constant<int, 2>{});
-  else if (mr == 4) go(std::integral_constant<int, 4>{});
-  else go(std::integral_constant<int, 8>{});
+template <int MR, int TILES>
+bool launch_share_k(const KParams& p, const SharePlan& plan, dim3 grid, hipStream_t s) {
+  if (plan.spw == 4) return p.gs128 ? launch_share<MR, TILES, 4, 128>(p, plan.guarded, grid, s) : launch_share<MR, TILES, 4, 64>(p, plan.guarded, grid, s);
+  if (plan.spw == 3) return p.gs128 ? launch_share<MR, TILES, 3, 128>(p, plan.guarded, grid, s) : launch_share<MR, TILES, 3, 64>(p, plan.guarded, grid, s);
+  return false;
+}
+template <int MR>
+bool launch_share_rows(const KParams& p, const SharePlan& plan, dim3 grid, hipStream_t s) {
+  if (plan.tiles == 2) return launch_share_k<MR, 2>(p, plan, grid, s);
+  if (plan.tiles == 3) return launch_share_k<MR, 3>(p, plan, grid, s);
+  if constexpr (MR < 8) {
+    if (plan.tiles == 4) return launch_share_k<MR, 4>(p, plan, grid, s);
+  }
+  return false;
+}
+int32_t launch_shares(KParams& p, const SharePlan& plan, hipStream_t s) {
+  p.ks = plan.ks;
+  p.tpw = plan.rows;
+  const uint32_t per_wg = plan.rows * (8 / plan.ks);
+  const dim3 grid((p.ld_out + per_wg - 1) / per_wg);
+  if (!(p.M > 4 ? launch_share_rows<8>(p, plan, grid, s) : (p.M > 2 ? launch_share_rows<4>(p, plan, grid, s) : launch_share_rows<2>(p, plan, grid, s))))
+    return fail(RMLX_RUNTIME_ERROR, "qmv_q4: no kernel for shares of %u rows in %u tiles, %u slabs a wave (M=%u K=%u)", plan.rows, plan.tiles, plan.spw, p.M, p.K);
+  RMLX_HIP_CHECK(take_launch_error());
+  return RMLX_OK;
 }
 
 template <int MR, int TILES, bool PAIR = false, int G = 0>
@@ -742,38 +756,65 @@ bool qmv_q4_ragged_supported(uint32_t N, uint32_t K, uint32_t group_size) {
   return (group_size == 64 || group_size == 128) && N > 0 && K > 0 && K % group_size == 0;
 }
 
-// Shares (the line of launch_qmv_q4) of a K whose slabs are not the same for all waves, or of any N, with clamped loads: zeros for the
+// k-parts per pass: 8 for K >= 4096; for smaller K the fewest parts of at most 4 slabs each, the remaining waves take further 16-row tiles (as long as
+// N divides)
+static uint32_t k_parts(uint32_t N, uint32_t slabs) {
+  uint32_t ks = slabs < 32 ? 1 : 8;
+  while (ks < 8 && ks * kSpwMax < slabs) ks *= 2;
+  while (ks < 8 && N % (16 * (8 / ks)) != 0) ks *= 2;
+  return ks;
+}
+// With 8 rows every wave takes two tiles (rows r and r+16) for the same staged activations when that still gives every CU a workgroup: the activation
+// traffic and staging work per weight byte halve.
+static bool pairs_pay(uint32_t N, uint32_t nt, uint32_t chunks) {
+  return N % (32 * nt) == 0 && (uint64_t)(N / (32 * nt)) * chunks >= 1ull * (uint32_t)ctx().num_cus;
+}
+
+// Equal shares: one workgroup per CU with a share of the rows, as up to four tiles side by side whose weights are all requested at once.  The
+// activations (as many bytes as a tile of weights at four rows, twice that at eight) then pass the address unit once per CU instead of
+// once per tile, and no CU has a tile more than another.  us, a tile (8 rows: two) per workgroup / shares:
+//   K = 4096, N = 4608 / 5120 / 6144 / 9216 / 11008 / 14336 / 16384: 2 rows 6.0 / 5.7, 6.1 / 5.8, 6.2 / 6.0, -, 8.0 / 7.6, 9.3 / 9.1, 10.3 / 9.7;
+//     4 rows 6.4 / 5.9, 6.4 / 6.0, 6.6 / 6.1, 8.2 / 7.3, 8.5 / 7.7, 10.3 / 9.4, 10.8 / 9.9; 8 rows 7.3 / 6.3, 7.4 / 6.4, 7.5 / 6.5, 9.3 / 7.6, 9.4 / 8.2,
+//     9.7 / 9.8, 10.2 / 10.4: up to three tiles; group size 128, 9216 / 12288: 4 rows 7.6 / 7.0, 8.0 / 7.6, 8 rows 9.6 / 7.2, 9.7 / 7.8;
+//   K = 3072, up to 4 rows: only where the tiles leave many CUs without a last one: 3 rows 9216 / 12288 / 14336 6.7 / 6.5, 7.1 / 7.5, 8.7 / 8.2, group
+//     size 128 6.6 / 6.4, 6.8 / 7.2; 2 rows 14336 7.6 / 8.0;
+//   shorter rows (several waves' tiles beside each other): 3 rows 14336 x 2048 6.5 / 6.6, 14336 x 1536 5.6 / 5.7, 14336 x 1024 4.8 / 5.0;
+//     6 rows 9216 x 3072 8.2 / 6.9, 9216 x 2048 7.1 / 6.3, 14336 x 1536 6.3 / 6.0, 14336 x 1024 5.2 / 5.3;
+//   one tile a workgroup (3072 rows as shares of 12): 3 rows, K = 3072 4.1 / 4.2; pairs that make one even round: 8 rows 8192 x 4096 6.7 / 6.8, 16384 x 1536 6.1 / 6.2.
+// Of a K whose slabs are not the same for all waves, or of any N, with clamped loads: zeros for the
 // activations and scales past the row.  us, a tile (8 rows: two) per workgroup / shares:
 //   3, 4 rows, two tiles a share: 4608 x 3840 / 2560 6.4 / 5.7, 5.3 / 4.5; 8192 x 3840 / 3200 / 2560 6.9 / 6.7, 6.3 / 6.3, 6.0 / 5.7; 4800 x 2880 6.2 / 5.1;
 //     9216 x 1984 7.3 / 6.0; 12288 x 1088 5.8 / 5.1; three, where the third is small: 9216 x 4032 / 2880 9.5 / 9.0, 7.8 / 7.0, else off the multiples of 128 or 16 at
 //     most: 11008 x 3200 7.6 / 8.0, 20480 x 1792 7.8 / 8.4, 12288 x 2880 8.1 / 8.0, 12288 x 4032 9.9 / 10.7; four: 14336 x 3200 8.9 / 10.0;
 //   5 to 8 rows, up to three tiles: 8 rows 4608 x 3840 7.5 / 6.0, 8192 x 2560 6.7 / 6.1, 11008 x 3840 11.0 / 8.9, 20480 x 1280 8.9 / 7.3; 6 rows 4800 x 2880 6.6 / 5.4,
 //     9216 x 1984 7.9 / 6.3, 20000 x 1088 9.1 / 7.0.
-struct SharePlan { uint32_t ks, rows, tiles; };
-static bool guarded_share_plan(uint32_t M, uint32_t N, uint32_t K, SharePlan* out) {
+static bool share_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t group_size, SharePlan* out) {
   const uint32_t cus = ctx().num_cus, slabs = (K + 127) / 128;
-  if (M < 3 || M > 8 || slabs < 9 || slabs > 8 * kSpwMax || cus == 0) return false;
-  SharePlan s{1, 0, 0};
-  while (s.ks < 8 && s.ks * kSpwMax < slabs) s.ks *= 2;
-  const uint32_t wide = cus * (8 / s.ks);
-  s.rows = (uint32_t)(((uint64_t)N + wide - 1) / wide);
-  s.tiles = (s.rows + 15) / 16;
-  *out = s;
-  if (M > 4) return s.tiles == 2 || s.tiles == 3;
-  return s.tiles == 2 || (s.tiles == 3 && (s.rows <= 36 || ((K % 128 != 0 || N % 16 != 0) && K <= 3072)));
+  if (M < 2 || M > 8 || cus == 0 || slabs > 8 * kSpwMax || (group_size != 64 && group_size != 128)) return false;
+  auto shares = [&](uint32_t ks, bool guarded) {
+    const uint32_t wide = cus * (8 / ks), rows = (uint32_t)(((uint64_t)N + wide - 1) / wide);
+    *out = SharePlan{ks, (slabs + ks - 1) / ks, rows, (rows + 15) / 16, guarded};
+  };
+  if (qmv_q4_supported(N, K, group_size)) {
+    const uint32_t ks = k_parts(N, slabs), nt = 8 / ks;
+    if (slabs == ks * kSpwMax || slabs == ks * 3) {  // (the kernels with a fixed slab count)
+      shares(ks, false);
+      const bool pair = M > 4 && pairs_pay(N, nt, 1);
+      const uint32_t tiles_x = N / (16 * nt * (pair ? 2 : 1)), last_round = tiles_x % cus;
+      if (M > 4) return K >= 1536 && out->tiles >= 2 && out->tiles <= 3 && !(pair && tiles_x <= cus);
+      return (K >= 4096 || (M > 2 && group_size == 64 && K >= 3072 && last_round != 0 && last_round * 10 <= cus * 7)) && out->tiles >= 2 && out->tiles <= 4;
+    }
+  }
+  if (M < 3 || slabs < 9) return false;
+  uint32_t ks = 1;
+  while (ks < 8 && ks * kSpwMax < slabs) ks *= 2;
+  shares(ks, true);
+  if (M > 4) return out->tiles == 2 || out->tiles == 3;
+  return out->tiles == 2 || (out->tiles == 3 && (out->rows <= 36 || ((K % 128 != 0 || N % 16 != 0) && K <= 3072)));
 }
-bool qmv_q4_takes_shares(uint32_t M, uint32_t N, uint32_t K) {
+bool qmv_q4_takes_shares(uint32_t M, uint32_t N, uint32_t K, uint32_t group_size) {
   SharePlan plan;
-  return guarded_share_plan(M, N, K, &plan);
-}
-static bool guarded_shares(KParams& p, const QmvArgs& a, int mr, hipStream_t s) {
-  SharePlan plan;
-  if (!guarded_share_plan(a.M, a.N, a.K, &plan)) return false;
-  p.ks = plan.ks;
-  p.tpw = plan.rows;
-  const uint32_t nt = 8 / plan.ks, slabs = (a.K + 127) / 128;
-  launch_share_rows(p, mr, (slabs + plan.ks - 1) / plan.ks, true, plan.tiles, dim3((a.N + plan.rows * nt - 1) / (plan.rows * nt)), s);
-  return true;
+  return share_plan(M, N, K, group_size, &plan);
 }
 
 // Rows of x over a matrix off the multiples above: one tile of 16 or, where those fill the chip, 32 weight rows per wave.
@@ -788,10 +829,8 @@ int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s) {
   p.K = a.K; p.ld_out = a.ld_out; p.M = a.M;
   p.gs128 = a.group_size == 128 ? 1u : 0u;
   p.x_bf16 = a.x_bf16 ? 1u : 0u;
-  if (guarded_shares(p, a, a.M > 4 ? 8 : 4, s)) {
-    RMLX_HIP_CHECK(take_launch_error());
-    return RMLX_OK;
-  }
+  SharePlan shares;
+  if (share_plan(a.M, a.N, a.K, a.group_size, &shares)) return launch_shares(p, shares, s);
   p.tpw = 1;
   p.ks = 1;
   while (p.ks < 8 && p.ks * kSpwMax * 128 < a.K) p.ks *= 2;
@@ -819,54 +858,20 @@ int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s) {
   const bool tab = a.chunk_tab != nullptr;
   uint32_t chunks = tab ? a.max_chunks : (a.M + 7) / 8;
   if (chunks == 0) return RMLX_OK;
-  // k-parts per pass: 8 for K >= 4096; for smaller K the fewest parts of at most 4 slabs each,
-  // the remaining waves take further 16-row tiles (as long as N divides)
-  uint32_t ks = 8;
-  const uint32_t slabs = a.K / 128;
-  if (slabs < 32) {
-    ks = 1;
-    while (ks * kSpwMax < slabs) ks *= 2;
-    while (ks < 8 && a.N % (16 * (8 / ks)) != 0) ks *= 2;
-  }
+  SharePlan shares;
+  if (!tab && !a.dual && a.mr == 0 && a.ld_out == a.N && share_plan(a.M, a.N, a.K, a.group_size, &shares)) return launch_shares(p, shares, s);
+  const uint32_t slabs = a.K / 128, ks = k_parts(a.N, slabs);
   p.ks = ks;
   int mr = a.mr;
   if (mr == 0) mr = tab ? 8 : (a.M >= 5 ? 8 : (a.M >= 3 ? 4 : (a.M == 2 ? 2 : 1)));
-  // With 8 rows every wave takes two tiles (rows r and r+16) for the same staged activations when
-  // that still gives every CU a workgroup: the activation traffic and staging work per
-  // weight byte halve.
   const uint32_t nt = 8 / ks;
-  const bool pair = !a.dual && mr == 8 && a.N % (32 * nt) == 0 &&
-                    (uint64_t)(a.N / (32 * nt)) * chunks >= 1ull * (uint32_t)ctx().num_cus;
+  const bool pair = !a.dual && mr == 8 && pairs_pay(a.N, nt, chunks);
   // Tiles per workgroup: with one pass over K a workgroup keeps its staged activations for several
   // consecutive tiles (staging 8 rows costs as many bytes as the two tiles it serves), as long as
   // every CU still gets two workgroups.
   const uint32_t tiles_x = a.N / (16 * nt * (pair ? 2 : 1));
   uint32_t tpw = 1;
   const bool uniform_single_pass = slabs == ks * kSpwMax || slabs == ks * 3;  // the kernels with a fixed slab count
-  // Equal shares: one workgroup per CU with a share of the rows, as up to four tiles side by side whose weights are all requested at once.  The
-  // activations (as many bytes as a tile of weights at four rows, twice that at eight) then pass the address unit once per CU instead of
-  // once per tile, and no CU has a tile more than another.  us, a tile (8 rows: two) per workgroup / shares:
-  //   K = 4096, N = 4608 / 5120 / 6144 / 9216 / 11008 / 14336 / 16384: 2 rows 6.0 / 5.7, 6.1 / 5.8, 6.2 / 6.0, -, 8.0 / 7.6, 9.3 / 9.1, 10.3 / 9.7;
-  //     4 rows 6.4 / 5.9, 6.4 / 6.0, 6.6 / 6.1, 8.2 / 7.3, 8.5 / 7.7, 10.3 / 9.4, 10.8 / 9.9; 8 rows 7.3 / 6.3, 7.4 / 6.4, 7.5 / 6.5, 9.3 / 7.6, 9.4 / 8.2,
-  //     9.7 / 9.8, 10.2 / 10.4: up to three tiles; group size 128, 9216 / 12288: 4 rows 7.6 / 7.0, 8.0 / 7.6, 8 rows 9.6 / 7.2, 9.7 / 7.8;
-  //   K = 3072, up to 4 rows: only where the tiles leave many CUs without a last one: 3 rows 9216 / 12288 / 14336 6.7 / 6.5, 7.1 / 7.5, 8.7 / 8.2, group
-  //     size 128 6.6 / 6.4, 6.8 / 7.2; 2 rows 14336 7.6 / 8.0;
-  //   shorter rows (several waves' tiles beside each other): 3 rows 14336 x 2048 6.5 / 6.6, 14336 x 1536 5.6 / 5.7, 14336 x 1024 4.8 / 5.0;
-  //     6 rows 9216 x 3072 8.2 / 6.9, 9216 x 2048 7.1 / 6.3, 14336 x 1536 6.3 / 6.0, 14336 x 1024 5.2 / 5.3;
-  //   one tile a workgroup (3072 rows as shares of 12): 3 rows, K = 3072 4.1 / 4.2; pairs that make one even round: 8 rows 8192 x 4096 6.7 / 6.8, 16384 x 1536 6.1 / 6.2.
-  const uint32_t cus = ctx().num_cus, share = (a.N + cus * nt - 1) / (cus * nt), tiles_share = (share + 15) / 16, last_round = tiles_x % cus;
-  if (uniform_single_pass && !tab && !a.dual && chunks == 1 && a.ld_out == a.N && mr >= 2 &&
-      (mr < 8 ? (a.K >= 4096 || (mr == 4 && !p.gs128 && a.K >= 3072 && last_round != 0 && last_round * 10 <= cus * 7)) && tiles_share >= 2 && tiles_share <= 4
-              : a.K >= 1536 && tiles_share >= 2 && tiles_share <= 3 && !(pair && tiles_x <= cus))) {
-    p.tpw = share;
-    launch_share_rows(p, mr, slabs / ks, false, tiles_share, dim3((a.N + share * nt - 1) / (share * nt)), s);
-    RMLX_HIP_CHECK(take_launch_error());
-    return RMLX_OK;
-  }
-  if (!uniform_single_pass && !tab && !a.dual && a.ld_out == a.N && mr >= 4 && guarded_shares(p, a, mr, s)) {
-    RMLX_HIP_CHECK(take_launch_error());
-    return RMLX_OK;
-  }
   if (uniform_single_pass) {
     // With a chunk table, consecutive chunks often belong to one expert (more than 8 rows): a grid
     // width that is a multiple of the 8 XCDs puts their workgroups for the same tiles on one XCD,

@@ -47,3 +47,42 @@ def test_guarded_shares(hip, k, gs, m, dtype, share, odd):
     ref = model.qmm(x_as_f64(x, dtype).astype(np.float16).astype(np.float64), *(a[rows] for a in w), gs, 4)
     assert_close(out[:, rows], ref)
     assert _ratio(out[:, rows], ref) < 1.05
+
+
+def _builds():
+    """(rows of x, K, group size, weight rows of a share, weight rows that the last one lacks): every build of the kernel, two waves' tiles beside each
+    other (K up to 2048)."""
+    whole = [(2, 4096, gs, s) for gs in (64, 128) for s in (17, 33, 49)] + [(4, 4096, gs, s) for gs in (64, 128) for s in (32, 48, 64)]
+    whole += [(3, 3072, 64, s) for s in (17, 33, 49)] + [(8, k, gs, s) for k in (4096, 3072, 2048, 1536) for gs in (64, 128) for s in (17, 33)]
+    guarded = [(4, 3968, gs, s) for gs in (64, 128) for s in (17, 33)] + [(3, k, gs, s) for k, gs in ((2880, 64), (2304, 128)) for s in (32, 36)]
+    guarded += [(5, 3968, gs, s) for gs in (64, 128) for s in (32, 48)] + [(8, k, gs, s) for k, gs in ((2880, 64), (2304, 128), (1984, 64), (1088, 64)) for s in (17, 48)]
+    return [b + (0,) for b in whole + guarded] + [b + (16,) for b in whole] + [b + (13,) for b in guarded]
+
+
+# Selector 16 runs the shares or refuses: a rule that leaves a shape to another kernel fails here.
+@pytest.mark.parametrize("m,k,gs,share,short", _builds())
+def test_every_build(hip, m, k, gs, share, short):
+    from rmlx_amd import ops, runtime as rt
+    sides = 1 if k > 2048 else 2
+    n = hip.device_info()["compute_units"] * sides * share - short
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, 4, gs)
+    dtype = "bf16" if (share + m) % 2 else "f16"
+    x = make_x(rng, m, k, dtype)
+    xd = rt.DeviceBuffer.from_numpy(x, rt.BF16) if dtype == "bf16" else rt.DeviceBuffer.from_numpy(x)
+    out = ops.affine_quantized_matmul_batched(xd, ops.QuantizedWeight.from_numpy(*w, gs, 4), kernel=rt.KERNEL_QMV_SHARES).numpy()
+    rows = np.unique(np.concatenate([np.arange(2 * share), np.arange(0, n, 61), np.arange(share - 1, n, 7 * share), np.arange(n - 2 * share, n)]))
+    ref = model.qmm(x_as_f64(x, dtype).astype(np.float16).astype(np.float64), *(a[rows] for a in w), gs, 4)
+    assert_close(out[:, rows], ref)
+    assert _ratio(out[:, rows], ref) < 1.05
+
+
+# eight rows of four tiles, seven slabs, two rows of K < 4096, one tile, two slots, more rows, other weights
+@pytest.mark.parametrize("m,k,gs,share,bits", [(8, 4096, 64, 49, 4), (4, 896, 128, 17, 4), (2, 3072, 64, 33, 4), (4, 4096, 64, 16, 4), (4, 8192, 64, 33, 4),
+                                               (9, 4096, 64, 33, 4), (1, 4096, 64, 33, 4), (4, 4096, 32, 33, 4), (4, 4096, 64, 33, 8), (3, 3200, 64, 48, 4)])
+def test_shares_are_refused(hip, m, k, gs, share, bits):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(k)
+    w = make_weight(rng, hip.device_info()["compute_units"] * share, k, bits, gs)
+    with pytest.raises(rt.KernelError):
+        ops.affine_quantized_matmul_batched(rt.DeviceBuffer.from_numpy(make_x(rng, m, k)), ops.QuantizedWeight.from_numpy(*w, gs, bits), kernel=rt.KERNEL_QMV_SHARES)
