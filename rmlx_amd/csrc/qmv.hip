@@ -93,12 +93,15 @@ struct KParams {
 // 9216 x 4096: without the loads of the activations a tile per workgroup takes 6.4 us instead of 8.2, shares take 7.3; 4.45 is a bare read).
 // G: the group size, 0 = told by p.gs128.  Known here, the scales of group size 128 stay as loaded until the products (spread over the slabs behind their
 // loads they are waited for in front of the weights'): 8 rows 20480 x 4096 14.1 -> 12.6, 20480 x 3072 12.6 -> 11.5; one tile a workgroup gains nothing (0).
-template <int MR, int TILES, bool TAB, int SPW, bool PAIR, int REUSE, bool RAGGED = false, bool SHARE = false, int G = 0>
+// XF32 (SHARE): x holds f32 values.  8 rows 11008 x 3840 11.0 us with a cast in front, 12.8 on the slot-streaming kernel, which reads them itself too, here
+// 9.3; 6 rows 9216 x 2880 9.4 / 9.7 / 7.5; 3 rows 9001 x 4096, group size 128 9.6 with the cast, here 7.8.
+template <int MR, int TILES, bool TAB, int SPW, bool PAIR, int REUSE, bool RAGGED = false, bool SHARE = false, int G = 0, bool XF32 = false>
 __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !SHARE) ? 4 : 1) void qmv_q4_kernel(uint64_t w0_, uint64_t s0_, uint64_t b0_, uint64_t x_, uint32_t K_, uint32_t ks_, uint32_t M_, uint32_t gs128_, uint32_t tpw_, uint32_t x_bf16_, KParams p) {
   p.w0 = global_at<uint32_t>(w0_); p.s0 = global_at<__half>(s0_); p.b0 = global_at<__half>(b0_); p.x = global_at<__half>(x_); p.K = K_; p.ks = ks_; p.M = M_; p.gs128 = gs128_; p.tpw = tpw_; p.x_bf16 = x_bf16_;
   static_assert(!REUSE || SPW != 0, "reuse needs a uniform slab count");
   static_assert(!PAIR || TILES == 2 || SHARE, "paired tiles need two tile slots");
   static_assert(!SHARE || (PAIR && !TAB && REUSE == 1 && G != 0), "one matrix, one pass over K");
+  static_assert(!XF32 || SHARE, "f32 rows: equal shares");
   static_assert(!RAGGED || SHARE || (!TAB && SPW == 0 && REUSE == 0 && (TILES == 1 || PAIR)), "one matrix, guarded loads");
   constexpr int kSlots = 4 * MR;                       // 16-byte activation slots per (slab, j) block ...
   constexpr int kBlk = kSlots + 1;                     // ... followed by one slot of zeros (read by the lanes whose operand rows are empty)
@@ -175,7 +178,7 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
   // this wave's activations -> its LDS image in operand order
   auto stage_x = [&](const u4 (&xv)[MR]) {
     const int ls = lane >> 4, gg = (lane >> 2) & 3, j = lane & 3;
-    if (p.x_bf16) {  // (wave-uniform; the f16 path pays a scalar compare)
+    if (!XF32 && p.x_bf16) {  // (wave-uniform; the f16 path pays a scalar compare)
 #pragma unroll
       for (int m = 0; m < MR; ++m)
         *reinterpret_cast<u4*>(xs + ((ls * 4 + j) * kBlk + gg * MR + m) * 16) = permute_x8(bf16x8_to_f16(xv[m]));
@@ -184,6 +187,21 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
 #pragma unroll
     for (int m = 0; m < MR; ++m)
       *reinterpret_cast<u4*>(xs + ((ls * 4 + j) * kBlk + gg * MR + m) * 16) = permute_x8(xv[m]);
+  };
+  // XF32: f32 rows as they are (16 more bytes a lane and row), rounded to f16 as the cast kernel does before the weights are asked for.  No branch
+  // between the loads: rows past the last repeat it (unstored), k past the row its last piece (zeros instead).
+  auto load_x_f32 = [&](int sl, u4 (&lo)[MR], u4 (&hi)[MR]) {
+    const uint32_t k = (uint32_t)(sl * 16 + lane) * 8, from = k < K ? k : K - 8;
+#pragma unroll
+    for (int m = 0; m < MR; ++m) {
+      const u4* q = reinterpret_cast<const u4*>(reinterpret_cast<const float*>(p.x) + (uint64_t)(row0 + ((uint32_t)m < rows ? m : rows - 1)) * K + from);
+      lo[m] = q[0]; hi[m] = q[1];
+    }
+  };
+  auto round_x = [&](const u4& lo, const u4& hi) -> u4 {
+    const f4 a = __builtin_bit_cast(f4, lo), b = __builtin_bit_cast(f4, hi);
+    const h8 v = {(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w, (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
+    return __builtin_bit_cast(u4, v);
   };
   auto stage_sums = [&]() {
     if constexpr (kPreSums) {
@@ -496,8 +514,8 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
       for (uint32_t i = 0; i < rows; ++i) {
         const bool mine = spoiled && a.m == i;
         if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
-        const char* const x = reinterpret_cast<const char*>(p.x + (uint64_t)(row0 + i) * K);
-        const int32_t x_dtype = p.x_bf16 ? RMLX_DTYPE_BF16 : RMLX_DTYPE_F16;
+        const char* const x = reinterpret_cast<const char*>(p.x) + (((uint64_t)(row0 + i) * K) << (XF32 ? 2 : 1));
+        const int32_t x_dtype = XF32 ? RMLX_DTYPE_F32 : (p.x_bf16 ? RMLX_DTYPE_BF16 : RMLX_DTYPE_F16);
         const uint32_t n = odd_pieces(x, x_dtype, K, (uint32_t)lane, list);
         if (mine)
           store(a, plain_sum<4>(G == 128 ? 7 : 6, reinterpret_cast<const char*>(p.w0 + (uint64_t)a.col * words_per_row), p.s0 + (uint64_t)a.col * groups_per_row,
@@ -552,7 +570,14 @@ __global__ __launch_bounds__(kThreads, (REUSE != 0 && MR == 8 && TILES == 2 && !
     u4 wreg[TILES][kSpwMax];
     {
       u4 xv[MR];
-      load_x(sl, SPW, xv);
+      if constexpr (XF32) {
+        u4 hi[MR];
+        load_x_f32(sl, xv, hi);
+#pragma unroll
+        for (int m = 0; m < MR; ++m) xv[m] = (uint32_t)(sl * 16 + lane) * 8 < K ? round_x(xv[m], hi[m]) : (u4){0u, 0u, 0u, 0u};
+      } else {
+        load_x(sl, SPW, xv);
+      }
       load_tile(blockIdx.x, sl, SPW, sbv, wreg);
       stage_x(xv);
       stage_sums();
@@ -671,36 +696,44 @@ struct SharePlan { uint32_t ks, spw, rows, tiles; bool guarded; };
 
 // false: no kernel for the plan (share_plan makes none of these)
 template <int MR, int TILES, int SPW, int G>
-bool launch_share(const KParams& p, bool guarded, dim3 grid, hipStream_t s) {
+bool launch_share(const KParams& p, bool x_f32, bool guarded, dim3 grid, hipStream_t s) {
+  auto go = [&](auto guarded_c) {
+    constexpr bool kGuarded = decltype(guarded_c)::value;
+    if (x_f32) launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, kGuarded, true, G, true>>(p, grid, s);
+    else launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, kGuarded, true, G>>(p, grid, s);
+    return true;
+  };
   if constexpr (MR >= 4 && TILES <= 3) {
-    if (guarded) { launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, true, true, G>>(p, grid, s); return true; }
+    if (guarded) return go(std::true_type{});
   }
   if constexpr (SPW == 4 || MR == 8 || (MR == 4 && G == 64)) {
-    if (!guarded) { launch_kernel<qmv_q4_kernel<MR, TILES, false, SPW, true, 1, false, true, G>>(p, grid, s); return true; }
+    if (!guarded) return go(std::false_type{});
   }
   return false;
 }
 template <int MR, int TILES>
-bool launch_share_k(const KParams& p, const SharePlan& plan, dim3 grid, hipStream_t s) {
-  if (plan.spw == 4) return p.gs128 ? launch_share<MR, TILES, 4, 128>(p, plan.guarded, grid, s) : launch_share<MR, TILES, 4, 64>(p, plan.guarded, grid, s);
-  if (plan.spw == 3) return p.gs128 ? launch_share<MR, TILES, 3, 128>(p, plan.guarded, grid, s) : launch_share<MR, TILES, 3, 64>(p, plan.guarded, grid, s);
+bool launch_share_k(const KParams& p, bool x_f32, const SharePlan& plan, dim3 grid, hipStream_t s) {
+  if (plan.spw == 4)
+    return p.gs128 ? launch_share<MR, TILES, 4, 128>(p, x_f32, plan.guarded, grid, s) : launch_share<MR, TILES, 4, 64>(p, x_f32, plan.guarded, grid, s);
+  if (plan.spw == 3)
+    return p.gs128 ? launch_share<MR, TILES, 3, 128>(p, x_f32, plan.guarded, grid, s) : launch_share<MR, TILES, 3, 64>(p, x_f32, plan.guarded, grid, s);
   return false;
 }
 template <int MR>
-bool launch_share_rows(const KParams& p, const SharePlan& plan, dim3 grid, hipStream_t s) {
-  if (plan.tiles == 2) return launch_share_k<MR, 2>(p, plan, grid, s);
-  if (plan.tiles == 3) return launch_share_k<MR, 3>(p, plan, grid, s);
+bool launch_share_rows(const KParams& p, bool x_f32, const SharePlan& plan, dim3 grid, hipStream_t s) {
+  if (plan.tiles == 2) return launch_share_k<MR, 2>(p, x_f32, plan, grid, s);
+  if (plan.tiles == 3) return launch_share_k<MR, 3>(p, x_f32, plan, grid, s);
   if constexpr (MR < 8) {
-    if (plan.tiles == 4) return launch_share_k<MR, 4>(p, plan, grid, s);
+    if (plan.tiles == 4) return launch_share_k<MR, 4>(p, x_f32, plan, grid, s);
   }
   return false;
 }
-int32_t launch_shares(KParams& p, const SharePlan& plan, hipStream_t s) {
+int32_t launch_shares(KParams& p, bool x_f32, const SharePlan& plan, hipStream_t s) {
   p.ks = plan.ks;
   p.tpw = plan.rows;
   const uint32_t per_wg = plan.rows * (8 / plan.ks);
   const dim3 grid((p.ld_out + per_wg - 1) / per_wg);
-  if (!(p.M > 4 ? launch_share_rows<8>(p, plan, grid, s) : (p.M > 2 ? launch_share_rows<4>(p, plan, grid, s) : launch_share_rows<2>(p, plan, grid, s))))
+  if (!(p.M > 4 ? launch_share_rows<8>(p, x_f32, plan, grid, s) : (p.M > 2 ? launch_share_rows<4>(p, x_f32, plan, grid, s) : launch_share_rows<2>(p, x_f32, plan, grid, s))))
     return fail(RMLX_RUNTIME_ERROR, "qmv_q4: no kernel for shares of %u rows in %u tiles, %u slabs a wave (M=%u K=%u)", plan.rows, plan.tiles, plan.spw, p.M, p.K);
   RMLX_HIP_CHECK(take_launch_error());
   return RMLX_OK;
@@ -828,9 +861,10 @@ int32_t launch_qmv_q4_ragged(const QmvArgs& a, hipStream_t s) {
   p.x = a.x; p.out = a.out;
   p.K = a.K; p.ld_out = a.ld_out; p.M = a.M;
   p.gs128 = a.group_size == 128 ? 1u : 0u;
-  p.x_bf16 = a.x_bf16 ? 1u : 0u;
+  p.x_bf16 = a.x_bf16 == 1 ? 1u : 0u;
   SharePlan shares;
-  if (share_plan(a.M, a.N, a.K, a.group_size, &shares)) return launch_shares(p, shares, s);
+  if (share_plan(a.M, a.N, a.K, a.group_size, &shares)) return launch_shares(p, a.x_bf16 == 2, shares, s);
+  if (a.x_bf16 == 2) return fail(RMLX_RUNTIME_ERROR, "qmv_q4: f32 activations must be cast to f16 first");
   p.tpw = 1;
   p.ks = 1;
   while (p.ks < 8 && p.ks * kSpwMax * 128 < a.K) p.ks *= 2;
@@ -854,12 +888,13 @@ int32_t launch_qmv_q4(const QmvArgs& a, hipStream_t s) {
   p.out = a.out; p.estride_w = a.expert_stride_w; p.estride_s = a.expert_stride_s;
   p.K = a.K; p.ld_out = a.ld_out; p.M = a.M; p.out_f32 = a.out_f32;
   p.gs128 = a.group_size == 128 ? 1u : 0u;
-  p.x_bf16 = a.x_bf16 ? 1u : 0u;
+  p.x_bf16 = a.x_bf16 == 1 ? 1u : 0u;
   const bool tab = a.chunk_tab != nullptr;
   uint32_t chunks = tab ? a.max_chunks : (a.M + 7) / 8;
   if (chunks == 0) return RMLX_OK;
   SharePlan shares;
-  if (!tab && !a.dual && a.mr == 0 && a.ld_out == a.N && share_plan(a.M, a.N, a.K, a.group_size, &shares)) return launch_shares(p, shares, s);
+  if (!tab && !a.dual && a.mr == 0 && a.ld_out == a.N && share_plan(a.M, a.N, a.K, a.group_size, &shares)) return launch_shares(p, a.x_bf16 == 2, shares, s);
+  if (a.x_bf16 == 2) return fail(RMLX_RUNTIME_ERROR, "qmv_q4: f32 activations must be cast to f16 first");
   const uint32_t slabs = a.K / 128, ks = k_parts(a.N, slabs);
   p.ks = ks;
   int mr = a.mr;

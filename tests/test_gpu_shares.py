@@ -86,3 +86,25 @@ def test_shares_are_refused(hip, m, k, gs, share, bits):
     w = make_weight(rng, hip.device_info()["compute_units"] * share, k, bits, gs)
     with pytest.raises(rt.KernelError):
         ops.affine_quantized_matmul_batched(rt.DeviceBuffer.from_numpy(make_x(rng, m, k)), ops.QuantizedWeight.from_numpy(*w, gs, bits), kernel=rt.KERNEL_QMV_SHARES)
+
+
+# f32 rows, 3 to 8 of them: read and rounded by the kernel itself on both sides of the line to the slot-streaming kernel, the builds of each form
+@pytest.mark.parametrize("m,n,k,gs", [(8, 11008, 3840, 64), (6, 9216, 2880, 64), (5, 14336, 1984, 64), (7, 24001, 1984, 64), (3, 9001, 4096, 128), (4, 28672, 3328, 64),
+                                      (4, 9216, 4096, 64), (2, 9216, 4096, 128), (8, 9216, 4096, 128), (3, 8448, 3072, 64), (8, 8704, 1536, 64), (4, 4608, 2304, 128)])
+def test_f32_rows_take_no_scratch(hip, m, n, k, gs):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, 4, gs)
+    wd = ops.QuantizedWeight.from_numpy(*w, gs, 4)
+    x = make_x(rng, m, k, "f32")
+    x16 = x.astype(np.float16)
+    xd, xh = rt.DeviceBuffer.from_numpy(x), rt.DeviceBuffer.from_numpy(x16)
+    stream = rt.Stream()
+    before = rt.scratch_allocations()
+    out = ops.affine_quantized_matmul_batched(xd, wd, stream=stream)
+    stream.sync()
+    assert rt.scratch_allocations() == before
+    same = ops.affine_quantized_matmul_batched(xh, wd).numpy()
+    assert np.array_equal(out.numpy().view(np.uint16), same.view(np.uint16))
+    rows = np.unique(np.concatenate([np.arange(0, n, 61), np.arange(n - 40, n)]))
+    assert_close(same[:, rows], model.qmm(x16.astype(np.float64), *(a[rows] for a in w), gs, 4))
