@@ -4,7 +4,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from tests.helpers import make_weight, make_x
+from tests.helpers import assert_close, make_weight, make_x
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +87,26 @@ def test_fused_in_the_store_of_one_launch(hip, m, n, k, bits):
     assert hip.scratch_allocations() == before
     p, got = plain.numpy().astype(np.float64), out.numpy().astype(np.float64)
     assert np.all(np.abs(got - (p + e)) <= 2.0 ** -11 * (np.abs(p) + np.abs(got)) * 1.01 + 1e-7)
+
+
+@pytest.mark.parametrize("m,n,k", [(6, 15680, 1088), (8, 15936, 1088), (5, 11968, 1472), (8, 12800, 1088), (6, 10496, 1472)])
+def test_few_rows_keep_the_fused_epilogue(hip, m, n, k):
+    """Shapes that a plain product takes as equal shares of the multi-row GEMV: an epilogue stays in the store of the tile GEMM, which needs no block for the
+    product where the output is the operand."""
+    from oracle import model
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k)
+    qw = ops.QuantizedWeight.from_numpy(*w, 64, 4)
+    x = make_x(rng, m, k)
+    xd = rt.DeviceBuffer.from_numpy(x)
+    plain, shares = (ops.affine_quantized_matmul_batched(xd, qw, kernel=q).numpy() for q in (0, rt.KERNEL_QMV_SHARES))
+    assert np.array_equal(plain.view(np.uint16), shares.view(np.uint16))
+    e = rng.standard_normal((m, n)).astype(np.float16)
+    own, stream, xa = rt.DeviceBuffer.from_numpy(e), rt.Stream(), xd.array()
+    oa, before = own.array(), rt.scratch_allocations()
+    rt.check(_calls(rt)["residual"](qw.handle, ctypes.byref(xa), ctypes.byref(oa), own.ptr, own.nbytes, ops._h(stream)))
+    stream.sync()
+    assert rt.scratch_allocations() == before
+    cols = np.arange(0, n, 61)
+    assert_close(own.numpy()[:, cols], model.qmm(x.astype(np.float64), *(a[cols] for a in w), 64, 4) + e[:, cols].astype(np.float64))
