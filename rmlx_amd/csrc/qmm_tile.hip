@@ -544,11 +544,12 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
       if (t < best_us) { best_us = t; best = TilePlan{c.wn, mi, c.kw, splits, c.mi_most != 0}; }
     }
   };
-  for (const Cost& c : costs[bits == 8]) {
-    if ((c.k != 0 && c.mi == 2 && M <= 32) || (c.mi_most != 0 && exact)) continue;
-    for (uint32_t mi = c.mi; mi <= (c.mi_most > c.mi ? c.mi_most : c.mi); ++mi) price(c, mi);
-  }
-  *us = best_us;
+  for (const Cost& c : costs[bits == 8])
+    if (c.mi_most == 0 && !(c.k != 0 && c.mi == 2 && M <= 32)) price(c, c.mi);
+  *us = best_us;  // (the dispatch's lines were drawn for these: a shorter estimate must not send a call to a kernel that is longer still)
+  if (exact) return best;
+  for (const Cost& c : costs[bits == 8])
+    for (uint32_t mi = c.mi; mi <= c.mi_most; ++mi) price(c, mi);
   return best;
 }
 

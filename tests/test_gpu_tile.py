@@ -147,6 +147,20 @@ def test_two_workgroups_per_cu(hip, m, n, k, bits, gs):
     assert_close(ops.qmm_add_residual(DeviceBuffer.from_numpy(x), qw, DeviceBuffer.from_numpy(e)).numpy(), ref + e.astype(np.float64), "residual")
 
 
+@pytest.mark.parametrize("m,n,k,bits,gs", [(188, 62528, 512, 4, 128), (923, 12864, 512, 4, 64), (404, 32320, 512, 4, 32), (451, 18624, 512, 8, 64), (714, 14528, 512, 8, 128)])
+def test_short_rows_of_bf16_stay_on_the_tile_gemm(hip, m, n, k, bits, gs):
+    """Rows of up to 1024 values over wide matrices, where the estimate of the GEMM with two workgroups per CU lies below the line to the GEMMs of before."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n)
+    w = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k, "bf16")
+    xd, qw = rt.DeviceBuffer.from_numpy(x, rt.BF16), ops.QuantizedWeight.from_numpy(*w, gs, bits)
+    auto, tile, other = (ops.affine_quantized_matmul_batched(xd, qw, kernel=q).numpy().view(np.uint16) for q in (0, rt.KERNEL_QMM_TILE, rt.KERNEL_QMM))
+    assert np.array_equal(auto, tile) and not np.array_equal(auto, other)
+    cols = np.arange(0, n, 97)
+    assert_close(auto.view(np.float16)[:, cols], model.qmm(x_as_f64(x, "bf16"), *(a[cols] for a in w), gs, bits))
+
+
 @pytest.mark.parametrize("tokens,experts,hidden,inter,bits,gs,fused", [(1500, 32, 1088, 576, 4, 64, True), (3400, 32, 1056, 544, 4, 32, False), (5200, 32, 1088, 576, 4, 64, False),
                                                                       (1600, 40, 1024, 512, 4, 128, True), (3400, 40, 1088, 576, 8, 64, True), (5300, 40, 1056, 544, 8, 32, False)])
 def test_routed_block_on_two_workgroups_per_cu(hip, tokens, experts, hidden, inter, bits, gs, fused):
