@@ -10,7 +10,7 @@ struct TileParams {
   const __half* x; void* out;
   float* partial;                   // not null: f32 partial sums [splits, M, N]
   uint32_t M, N, K, group_size, tiles_m, tiles_n, splits;
-  uint32_t frags_each, frags_more;  // fragments of 32 rows in a row tile, the first frags_more with one more (not a table's)
+  uint32_t tile_rows;               // rows of a row tile (not of a table's)
   int32_t exact, out_f32, epi_kind, epi_dtype;
   const void* epi;
   // grouped: (expert, first row, rows) per row tile, their number, optional gather of the activation rows, strides per expert
@@ -175,11 +175,8 @@ __device__ __forceinline__ bool tile_of(const TileParams& p, uint32_t tile_rows,
   t.split = idx % p.splits; idx /= p.splits;
   const uint32_t in_block = kBlock * p.tiles_n, first = idx / in_block * kBlock, within = idx % in_block, h = tiles_m - first < kBlock ? tiles_m - first : kBlock;
   t.mt = uni(first + within % h); t.nt = uni(within / h); t.split = uni(t.split);
-  // row tiles of equal height, to a fragment of 32 rows
-  const uint32_t q = p.frags_each, more = p.frags_more;
-  t.expert = 0; t.row_lo = 32 * (t.mt * q + (t.mt < more ? t.mt : more)); t.zeros = false;
-  t.rows = p.M - t.row_lo;
-  if (t.mt + 1 < tiles_m) t.rows = 32 * (q + (t.mt < more ? 1 : 0));
+  t.expert = 0; t.row_lo = t.mt * p.tile_rows; t.zeros = false;
+  t.rows = p.M - t.row_lo < p.tile_rows ? p.M - t.row_lo : p.tile_rows;
   if (p.tile_tab != nullptr) {
     t.expert = uni(p.tile_tab[3 * t.mt]); t.row_lo = uni(p.tile_tab[3 * t.mt + 1]);
     const uint32_t n = uni(p.tile_tab[3 * t.mt + 2]);
