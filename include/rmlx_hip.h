@@ -174,9 +174,10 @@ int32_t rmlx_hip_affine_quantized_matmul_batched(const rmlx_qweight* qw, const r
  * 14 = the multi-row streaming GEMV over 4-bit matrices that kernel 6 does not take (any N, any K of whole groups of 64 or 128),
  * 15 = the slot-streaming GEMV (4- and 8-bit, every group size, any N from a tile on, any K of whole groups from 512 to what the
  * registers of a workgroup hold of 16 activation rows: 8192 at 4 bits, group size 32 and 8-bit weights: 4096),
- * 16 = the multi-row streaming GEMV (6, 14) where it takes the rows as an equal share of weight rows per CU (refused where it does not).
+ * 16 = the multi-row streaming GEMV (6, 14) where it takes the rows as an equal share of weight rows per CU (refused where it does not),
+ * 17 = the large-tile MFMA GEMM (12) on its kernel of two workgroups per CU, whatever the size.
  * Precision: kernels 1, 3, 6 and 13 to 16 multiply with scale * q + bias as it is (integer dot products scaled in f32, f32 weights, or two f16
- * parts of 21 bits together); the GEMMs 2, 5 and 7 to 12 round every weight to f16, which adds 1.8e-4 of the result to the 2.1e-4 of
+ * parts of 21 bits together); the GEMMs 2, 5, 7 to 12 and 17 round every weight to f16, which adds 1.8e-4 of the result to the 2.1e-4 of
  * rounding it.  The automatic choice rounds weights only where it has always run such a GEMM: 4- / 8-bit matrices in multiples of 64, at
  * row counts beyond the GEMVs'. */
 int32_t rmlx_hip_qmm_select(const rmlx_qweight* qw, const rmlx_array* x, int32_t kernel,

@@ -305,6 +305,7 @@ int32_t launch_qmm_rw_grouped(const GroupedQmmArgs& a, hipStream_t s);
 struct TilePlan { uint32_t wn, mi, kw, splits; bool twin = false; };
 bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bits);
 TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us);  // us: estimated time of the launch, two workgroups per CU left out
+TilePlan qmm_twin_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits);  // the same among the plans of qmm_twin.hip only
 size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N);
 int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s);
 // The same over a table of row tiles of 32, 64, 128 or 256 rows (twin: up to 160, 8-bit 128) of one expert (x_rows: rows of x; out f16 or f32, a pair f16).  A row map

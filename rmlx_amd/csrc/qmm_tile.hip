@@ -492,8 +492,20 @@ bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
 // grows with the 32-row fragments of the tile and with the workgroups that share a CU (`step` holds (constant, per fragment) for
 // 1, 2, .. of them); fragments cost half as much on an idle chip as on a full one, where the clock falls.  A launch adds its start
 // and end, a K split the kernel that adds up the partial sums.  Fitted to about 15000 timed launches (780 shapes, every plan and
-// split): 6 % mean error, and the picks are 1.3 % slower on average than the fastest plan.
-static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool exact, double* us) {
+// split): 6 % mean error, and the picks are 1.3 % slower on average than the fastest plan; the rows of two workgroups per CU to 200 shapes of 17 rows and more.
+// What the estimate of two workgroups per CU, in `wn` * 32 columns, may be of the best other plan's for them to be ahead: the table's errors differ from
+// tile to tile (it has the 256 x 256 tile too long against the others and the tiles of 128 rows by 256 columns too short, over short rows above all).  Of 615
+// shapes of 65 to 4096 rows timed in both forms these lines take 205, 12 % faster on average, four of them 2 to 5 % slower (the best choice: 311, 10 %).
+static double twin_limit(const TilePlan& other, uint32_t wn, uint32_t M, uint32_t K) {
+  const bool is_short = K <= 640;
+  if (other.kw > 1 || other.splits > 1) return 0.95;
+  if (other.wn == 8 && other.mi == 8) return wn == 8 ? (is_short ? 1.03 : 0.98) : (M <= 320 ? 0.8 : 0.87);
+  if (other.wn == 8) return wn == 8 ? (is_short ? 1.13 : 1.03) : (is_short ? 1.07 : 1.01);
+  return wn == 8 ? (is_short ? 1.02 : 0.98) : 0.95;
+}
+enum { PLAN_ROUNDED = 0, PLAN_EXACT = 1, PLAN_TWIN = 2 };  // any kernel, those with exact weights, two workgroups per CU only
+static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, int kind, double* us) {
+  const bool exact = kind == PLAN_EXACT;
   // (kw >= 4: waves along k, steps of `k` values; mi_most: two workgroups per CU, qmm_twin.hip, tiles of mi to mi_most fragments)
   struct Cost { uint32_t wn, mi, kw; int per_cu; double start, step[3][2], sum, sum_per_mi; uint32_t k, mi_most; };
   static const Cost costs[2][12] = {
@@ -507,8 +519,8 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
        {2, 2, 8, 1, 5.20, {{0.089, 0.370}}, 2.80, 0.00, 256},
        {4, 1, 4, 1, 4.56, {{0.201, 0.751}}, 3.20, 1.04, 256},
        {4, 2, 4, 1, 5.46, {{0.296, 0.467}}, 2.87, 1.33, 256},
-       {8, 3, 1, 2, 5.86, {{0.365, 0.171}, {0.572, 0.278}}, 3.28, 1.29, 0, 5},
-       {4, 3, 1, 2, 4.85, {{0.269, 0.098}, {0.358, 0.153}}, 2.73, 1.52, 0, 7}},
+       {8, 3, 1, 2, 5.86, {{0.365, 0.171}, {0.572, 0.278}}, 0, 0, 0, 5},
+       {4, 3, 1, 2, 4.85, {{0.269, 0.098}, {0.358, 0.153}}, 0, 0, 0, 7}},
       {{8, 8, 1, 1, 7.26, {{0.608, 0.104}}, 8.71, 1.34},
        {8, 4, 1, 1, 3.33, {{0.516, 0.102}}, 5.39, 1.89},
        {4, 4, 1, 2, 4.87, {{0.352, 0.047}, {0.628, 0.091}}, 3.44, 1.65},
@@ -519,8 +531,8 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
        {2, 2, 8, 1, 5.17, {{0.061, 0.452}}, 2.30, 0.00, 256},
        {4, 1, 4, 1, 4.56, {{0.032, 1.080}}, 3.39, 0.00, 256},
        {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128},
-       {8, 3, 1, 2, 3.81, {{0.571, 0.154}, {0.722, 0.256}}, 3.89, 1.50, 0, 4},
-       {4, 3, 1, 2, 3.84, {{0.330, 0.105}, {0.395, 0.173}}, 3.25, 1.55, 0, 7}}};
+       {8, 3, 1, 2, 3.81, {{0.571, 0.154}, {0.722, 0.256}}, 0, 0, 0, 4},
+       {4, 3, 1, 2, 3.84, {{0.330, 0.105}, {0.395, 0.173}}, 0, 0, 0, 7}}};
   constexpr double kExactStep = 1.5;  // two products: 8 to 64 rows 1.35 to 1.45 x, 300 to 2000 rows 1.55 to 1.65
   const double cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
   const uint32_t rounds = (K + 127) / 128;
@@ -531,7 +543,7 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
     const double frags = (double)((M + 31) / 32) / (double)tm;
     for (uint32_t splits : {1u, 2u, 3u, 4u, 6u, 8u}) {
       const uint32_t stages = c.k != 0 ? (K + c.k - 1) / c.k : 0;
-      if (splits > 1 && (rounds < 2 * splits * c.kw || (double)(tiles * splits) > 1.6 * c.per_cu * cus || (uint64_t)splits * M * N > (1u << 27))) break;
+      if (splits > 1 && (c.mi_most != 0 || rounds < 2 * splits * c.kw || (double)(tiles * splits) > 1.6 * c.per_cu * cus || (uint64_t)splits * M * N > (1u << 27))) break;
       const double load = (double)(tiles * splits) / cus, full = std::floor(load / c.per_cu), rest = load - full * c.per_cu;
       const double steps = c.k != 0 ? (stages + splits - 1) / splits : 2.0 * ((((rounds + splits - 1) / splits) + c.kw - 1) / c.kw);
       double t = steps * full * (c.step[c.per_cu - 1][0] + c.step[c.per_cu - 1][1] * frags);
@@ -545,12 +557,22 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
     }
   };
   for (const Cost& c : costs[bits == 8])
-    if (c.mi_most == 0 && !(c.k != 0 && c.mi == 2 && M <= 32)) price(c, c.mi);
+    if (kind != PLAN_TWIN && c.mi_most == 0 && !(c.k != 0 && c.mi == 2 && M <= 32)) price(c, c.mi);
   *us = best_us;  // (the dispatch's lines were drawn for these: a shorter estimate must not send a call to a kernel that is longer still)
   if (exact) return best;
+  // Two workgroups per CU (rounded weights only), without a K split (timed 4 to 15 % slower than the plans of the other kernels: 2398 rows, 896 x 10432 76
+  // against 68 us).  Up to 64 rows only over rows of up to 1024 values (8 rows, 117760 x 640, 8-bit 24.6 / 21.7; but 9 rows, 22016 x 14336 41 / 57, 21 rows, 62144 x
+  // 11328 108 / 153), in 256 columns.
+  const TilePlan other = best;
+  const double other_us = best_us;
+  best_us = 1e30;
   for (const Cost& c : costs[bits == 8])
-    for (uint32_t mi = c.mi; mi <= c.mi_most; ++mi) price(c, mi);
-  return best;
+    for (uint32_t mi = c.mi; mi <= c.mi_most; ++mi)
+      if (M > 64 || c.wn == 8 || kind == PLAN_TWIN) price(c, mi);
+  if (kind == PLAN_TWIN) return best;
+  if (M <= 64) return K <= 1024 && best_us < 1.05 * other_us ? best : other;
+  if (M <= 96 && K > 2048) return other;  // (72 rows, 117312 x 3200, group size 32 91 / 102)
+  return best_us < twin_limit(other, best.wn, M, K) * other_us ? best : other;
 }
 
 // (about 1 us of arithmetic, asked for twice per call by launches that take 5: the last plans of a thread are kept)
@@ -560,11 +582,16 @@ TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool e
   const uint32_t kind = bits + (exact ? 1 : 0);
   Kept& e = kept[(M * 31 + N * 7 + K + kind) & 63];
   if (e.M != M || e.N != N || e.K != K || e.bits != kind) {
-    e.plan = estimate_plan(M, N, K, bits, exact, &e.us);
+    e.plan = estimate_plan(M, N, K, bits, exact ? PLAN_EXACT : PLAN_ROUNDED, &e.us);
     e.M = M; e.N = N; e.K = K; e.bits = kind;
   }
   if (us != nullptr) *us = e.us;
   return e.plan;
+}
+
+TilePlan qmm_twin_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits) {
+  double us;
+  return estimate_plan(M, N, K, bits, PLAN_TWIN, &us);
 }
 
 size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N) {

@@ -161,6 +161,40 @@ def test_short_rows_of_bf16_stay_on_the_tile_gemm(hip, m, n, k, bits, gs):
     assert_close(auto.view(np.float16)[:, cols], model.qmm(x_as_f64(x, "bf16"), *(a[cols] for a in w), gs, bits))
 
 
+# Row tiles of one to seven fragments of 128 columns (8-bit too) and of one to five of 256 (8-bit: four), the last of them shorter; rows of several units
+# of scales, the last one early, half a stage at the end; columns that are no whole tile.
+@pytest.mark.parametrize("m,n,bits", [(5, 301, 4), (42, 1001, 4), (79, 300, 4), (301, 9001, 4), (153, 17001, 4), (190, 17000, 4), (1189, 5203, 4), (20, 110001, 4), (42, 33000, 4),
+                                      (79, 33001, 4), (116, 33003, 4), (412, 33000, 4), (5, 301, 8), (42, 1001, 8), (116, 17003, 8), (412, 9001, 8), (486, 9001, 8),
+                                      (1226, 5203, 8), (20, 70001, 8), (42, 70001, 8), (227, 33001, 8), (338, 33003, 8)])
+@pytest.mark.parametrize("k,gs", [(2112, 64), (1056, 32), (1408, 128)])
+def test_two_workgroups_at_every_height(hip, m, n, bits, k, gs):
+    """Selector 17 runs the kernel whatever the estimate says."""
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k + bits)
+    w = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k)
+    out = ops.affine_quantized_matmul_batched(rt.DeviceBuffer.from_numpy(x), ops.QuantizedWeight.from_numpy(*w, gs, bits), kernel=rt.KERNEL_QMM_TWIN).numpy()
+    cols = np.unique(np.concatenate([np.arange(0, n, 331), np.arange(max(0, n - 70), n)]))
+    assert_close(out[:, cols], model.qmm(x_as_f64(x, "f16"), *(a[cols] for a in w), gs, bits), f"M={m} N={n} K={k} bits={bits} gs={gs}")
+
+
+# The library's choice on both sides of its lines to that kernel, where the other plan splits K (over waves or workgroups, so its sums round differently): a few
+# rows over short and long ones, 10432 values in three ranges.
+@pytest.mark.parametrize("m,n,k,bits,gs,taken", [(30, 106240, 1024, 8, 128, True), (24, 130688, 1024, 4, 64, True), (9, 22016, 14336, 4, 64, False),
+                                                 (21, 62144, 2048, 4, 64, False), (48, 32768, 4096, 8, 64, False), (2398, 896, 10432, 4, 64, False)])
+def test_library_takes_two_workgroups(hip, m, n, k, bits, gs, taken):
+    from rmlx_amd import ops, runtime as rt
+    rng = np.random.default_rng(m + n + k)
+    w = make_weight(rng, n, k, bits, gs)
+    x = make_x(rng, m, k)
+    xd, qw = rt.DeviceBuffer.from_numpy(x), ops.QuantizedWeight.from_numpy(*w, gs, bits)
+    auto, tile, twin = (ops.affine_quantized_matmul_batched(xd, qw, kernel=q).numpy().view(np.uint16) for q in (0, rt.KERNEL_QMM_TILE, rt.KERNEL_QMM_TWIN))
+    assert np.array_equal(auto, tile) and np.array_equal(auto, twin) == taken
+    cols = np.arange(0, n, 331)
+    rows = np.arange(0, m, 7)
+    assert_close(auto.view(np.float16)[np.ix_(rows, cols)], model.qmm(x_as_f64(x, "f16")[rows], *(a[cols] for a in w), gs, bits))
+
+
 @pytest.mark.parametrize("tokens,experts,hidden,inter,bits,gs,fused", [(1500, 32, 1088, 576, 4, 64, True), (3400, 32, 1056, 544, 4, 32, False), (5200, 32, 1088, 576, 4, 64, False),
                                                                       (1600, 40, 1024, 512, 4, 128, True), (3400, 40, 1088, 576, 8, 64, True), (5300, 40, 1056, 544, 8, 32, False)])
 def test_routed_block_on_two_workgroups_per_cu(hip, tokens, experts, hidden, inter, bits, gs, fused):
