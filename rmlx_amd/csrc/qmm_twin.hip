@@ -43,7 +43,7 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
   const uint32_t lds0 = uni((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds);
   const uint32_t K = p.K, G = K / p.group_size, row_bytes = K * BITS / 8;
   const uint32_t rows = t_.rows, row_lo = t_.row_lo, n0 = t_.nt * BNO, cols = p.N - n0 < BNO ? p.N - n0 : BNO;
-  const uint32_t stages = (K + KB - 1) / KB;
+  const uint32_t stages = (K + KB - 1) / KB, s0 = uni(stages * t_.split / p.splits), s1 = uni(stages * (t_.split + 1) / p.splits);
 
   // ---- where a wave's loads come from -----------------------------------------------------------------------------------
   // Chunks of a row lie xor-ed with its number, on the address that a lane loads from, so that operand reads spread over the banks.
@@ -91,9 +91,10 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
     if constexpr (NI == 2) dma16_if(uni(cond), to + BN * 16, from, br);
   };
 
-  // what goes out next: activations ta bytes and weights tw bytes into their rows.  Past the end of the row a lane's offset goes out of range for good
-  const uint32_t base = lds0 + wave * 1024, a_end = K * 2, w_end = row_bytes;
-  uint32_t ta = 0, tw = 0, w_slot = 0;
+  // what goes out next: activations ta bytes and weights tw bytes into their rows.  Past the end of the row, or of this split, a lane's
+  // offset goes out of range for good
+  const uint32_t base = lds0 + wave * 1024, a_end = s1 * kARow < K * 2 ? s1 * kARow : K * 2, w_end = s1 * kWRow < row_bytes ? s1 * kWRow : row_bytes;
+  uint32_t ta = s0 * kARow, tw = s0 * kWRow, w_slot = 0;
   auto dma_a = [&](auto slotc, auto qc) {
     constexpr int q = decltype(qc)::value;
     if constexpr (q < NA) dma16_at<decltype(slotc)::value * kABytes + q * kRound>(base, aoff[q], xr, ta);
@@ -139,7 +140,7 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
   const uint32_t own_group = p.group_size == 32 ? hh * 2 : 0;  // (the lane's half of a stage is a group of its own)
   // bytes of the group's place in its row (of the last group, past the end), and what a unit that starts earlier adds
   const uint32_t gb_last = (G - 1) * 2, unit_last = (G - 1) / 8 * 16, early = unit_last - unit_start((G - 1) / 8) * 2;
-  uint32_t t_read = 0;
+  uint32_t t_read = s0;
   uint32_t wq[NI][WW], sraw[NI], braw[NI];
   uint32_t r_slot = 0;
   auto load_w = [&] {
@@ -198,9 +199,9 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
   const uint32_t umask = (1u << ushift) - 1;
   {
     clip();
-    dma_sb(1, 0);
+    dma_sb(1, s0 >> ushift);
 #pragma unroll
-    for (uint32_t i = 1; i < kNS; ++i) dma_sb((i & umask) == 0, i >> ushift);
+    for (uint32_t i = 1; i < kNS; ++i) dma_sb(((s0 + i) & umask) == 0, (s0 + i) >> ushift);
     using std::integral_constant;
     auto weights = [&] { each(integral_constant<int, NW>{}, dma_w); w_next(); };
     weights();
@@ -225,7 +226,7 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
   pick_sb();
 #pragma unroll
   for (int c = 0; c < 4 * NI; ++c) unpack(wf[c / 4], c / 4, 0, c % 4);
-  uint32_t t = 0;
+  uint32_t t = s0;
   auto step = [&](auto ic) -> bool {
     constexpr int I = decltype(ic)::value;
     auto kstep = [&](auto jc) {
@@ -269,7 +270,7 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
     kstep(std::integral_constant<int, 2>{});
     kstep(std::integral_constant<int, 3>{});
     clip();
-    return ++t < stages;
+    return ++t < s1;
   };
   while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
   }
@@ -286,8 +287,10 @@ __device__ __forceinline__ void twin_body(const TileParams p, const Tile t_, cha
 
   // ---- store: fragment (i, ni) of a lane holds activation row 32 i + r, weight rows 8 eg + 4 hh + 0 .. 3 of the wave's 32
   constexpr uint32_t U = BNO / 8, kKey = U < 32 ? U - 1 : 31;
-  const bool f32 = !DUAL && p.out_f32;
-  float* const o32 = static_cast<float*>(p.out);
+  // (no plan splits K; without the choice of partial sums here the f32 store is laid out otherwise and down projections are slower, 15 experts of 1024 x 512,
+  // group size 32, 343 rows each 56.6 / 62.4 us, 128 of 4096 x 1536, 128 rows 770 / 778)
+  const bool f32 = !DUAL && (p.partial != nullptr || p.out_f32);
+  float* const o32 = p.partial != nullptr ? p.partial + (uint64_t)t_.split * p.M * p.N : static_cast<float*>(p.out);
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const uint32_t m = i * 32 + r;
