@@ -312,6 +312,8 @@ int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s);
 // reaches the rows of an x of at most 2 GiB.
 bool qmm_tile_maps_rows(uint32_t x_rows, uint32_t K);
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
+// Estimated time of such a launch: `row_tiles` of them, `frags` fragments of 32 rows high on average, over N weight rows (of a pair: of both)
+double qmm_tile_grouped_us(uint32_t bits, bool twin, uint32_t tile_rows, double row_tiles, double frags, uint32_t N, uint32_t K);
 // The same over row tiles of at most 32 rows, for few rows per expert (qmm_slice.hip)
 int32_t launch_qmm_slice_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s);
 

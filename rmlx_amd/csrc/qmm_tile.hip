@@ -493,6 +493,45 @@ bool qmm_tile_supported(uint32_t N, uint32_t K, uint32_t group_size, uint32_t bi
 // 1, 2, .. of them); fragments cost half as much on an idle chip as on a full one, where the clock falls.  A launch adds its start
 // and end, a K split the kernel that adds up the partial sums.  Fitted to about 15000 timed launches (780 shapes, every plan and
 // split): 6 % mean error, and the picks are 1.3 % slower on average than the fastest plan; the rows of two workgroups per CU to 200 shapes of 17 rows and more.
+// (kw >= 4: waves along k, steps of `k` values; mi_most: two workgroups per CU, qmm_twin.hip, tiles of mi to mi_most fragments)
+struct Cost { uint32_t wn, mi, kw; int per_cu; double start, step[3][2], sum, sum_per_mi; uint32_t k, mi_most; };
+static const Cost kCosts[2][12] = {
+    {{8, 8, 1, 1, 8.19, {{0.503, 0.118}}, 7.46, 1.10},
+     {8, 4, 1, 1, 3.71, {{0.428, 0.110}}, 4.90, 1.74},
+     {4, 4, 1, 2, 4.64, {{0.270, 0.073}, {0.531, 0.083}}, 3.39, 1.59},
+     {4, 2, 1, 3, 3.50, {{0.300, 0.057}, {0.490, 0.053}, {0.707, 0.074}}, 3.49, 1.88},
+     {4, 4, 2, 1, 5.09, {{0.356, 0.159}}, 3.52, 2.07},
+     {4, 2, 2, 1, 3.90, {{0.398, 0.146}}, 3.46, 2.43},
+     {2, 1, 8, 2, 4.14, {{0.256, 0.271}, {1.023, 0.000}}, 3.00, 0.10, 256},
+     {2, 2, 8, 1, 5.20, {{0.089, 0.370}}, 2.80, 0.00, 256},
+     {4, 1, 4, 1, 4.56, {{0.201, 0.751}}, 3.20, 1.04, 256},
+     {4, 2, 4, 1, 5.46, {{0.296, 0.467}}, 2.87, 1.33, 256},
+     {8, 3, 1, 2, 5.86, {{0.365, 0.171}, {0.572, 0.278}}, 0, 0, 0, 5},
+     {4, 3, 1, 2, 4.85, {{0.269, 0.098}, {0.358, 0.153}}, 0, 0, 0, 7}},
+    {{8, 8, 1, 1, 7.26, {{0.608, 0.104}}, 8.71, 1.34},
+     {8, 4, 1, 1, 3.33, {{0.516, 0.102}}, 5.39, 1.89},
+     {4, 4, 1, 2, 4.87, {{0.352, 0.047}, {0.628, 0.091}}, 3.44, 1.65},
+     {4, 2, 1, 3, 3.36, {{0.349, 0.055}, {0.702, 0.000}, {1.128, 0.000}}, 3.53, 2.00},
+     {4, 4, 2, 1, 4.87, {{0.517, 0.141}}, 3.57, 2.17},
+     {4, 2, 2, 1, 3.44, {{0.519, 0.139}}, 4.01, 2.62},
+     {2, 1, 8, 1, 4.61, {{0.000, 0.671}}, 2.59, 0.00, 256},
+     {2, 2, 8, 1, 5.17, {{0.061, 0.452}}, 2.30, 0.00, 256},
+     {4, 1, 4, 1, 4.56, {{0.032, 1.080}}, 3.39, 0.00, 256},
+     {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128},
+     {8, 3, 1, 2, 3.81, {{0.571, 0.154}, {0.722, 0.256}}, 0, 0, 0, 4},
+     {4, 3, 1, 2, 3.84, {{0.330, 0.105}, {0.395, 0.173}}, 0, 0, 0, 7}}};
+// A launch of `tiles` workgroups, `steps` steps of 64 k each, `frags` fragments high on average
+static double rounds_us(const Cost& c, double tiles, double frags, double steps) {
+  const double cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+  const double load = tiles / cus, full = std::floor(load / c.per_cu), rest = load - full * c.per_cu;
+  double t = steps * full * (c.step[c.per_cu - 1][0] + c.step[c.per_cu - 1][1] * frags);
+  if (rest > 1e-9) {
+    const double* s = c.step[(int)std::ceil(rest - 1e-9) - 1];
+    t += steps * (s[0] + s[1] * frags * (full > 0 || load >= 1 ? 1.0 : 0.5 + 0.5 * load));
+  }
+  return t;
+}
+
 // What the estimate of two workgroups per CU, in `wn` * 32 columns, may be of the best other plan's for them to be ahead: the table's errors differ from
 // tile to tile (it has the 256 x 256 tile too long against the others and the tiles of 128 rows by 256 columns too short, over short rows above all).  Of 615
 // shapes of 65 to 4096 rows timed in both forms these lines take 205, 12 % faster on average, four of them 2 to 5 % slower (the best choice: 311, 10 %).
@@ -506,33 +545,6 @@ static double twin_limit(const TilePlan& other, uint32_t wn, uint32_t M, uint32_
 enum { PLAN_ROUNDED = 0, PLAN_EXACT = 1, PLAN_TWIN = 2 };  // any kernel, those with exact weights, two workgroups per CU only
 static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, int kind, double* us) {
   const bool exact = kind == PLAN_EXACT;
-  // (kw >= 4: waves along k, steps of `k` values; mi_most: two workgroups per CU, qmm_twin.hip, tiles of mi to mi_most fragments)
-  struct Cost { uint32_t wn, mi, kw; int per_cu; double start, step[3][2], sum, sum_per_mi; uint32_t k, mi_most; };
-  static const Cost costs[2][12] = {
-      {{8, 8, 1, 1, 8.19, {{0.503, 0.118}}, 7.46, 1.10},
-       {8, 4, 1, 1, 3.71, {{0.428, 0.110}}, 4.90, 1.74},
-       {4, 4, 1, 2, 4.64, {{0.270, 0.073}, {0.531, 0.083}}, 3.39, 1.59},
-       {4, 2, 1, 3, 3.50, {{0.300, 0.057}, {0.490, 0.053}, {0.707, 0.074}}, 3.49, 1.88},
-       {4, 4, 2, 1, 5.09, {{0.356, 0.159}}, 3.52, 2.07},
-       {4, 2, 2, 1, 3.90, {{0.398, 0.146}}, 3.46, 2.43},
-       {2, 1, 8, 2, 4.14, {{0.256, 0.271}, {1.023, 0.000}}, 3.00, 0.10, 256},
-       {2, 2, 8, 1, 5.20, {{0.089, 0.370}}, 2.80, 0.00, 256},
-       {4, 1, 4, 1, 4.56, {{0.201, 0.751}}, 3.20, 1.04, 256},
-       {4, 2, 4, 1, 5.46, {{0.296, 0.467}}, 2.87, 1.33, 256},
-       {8, 3, 1, 2, 5.86, {{0.365, 0.171}, {0.572, 0.278}}, 0, 0, 0, 5},
-       {4, 3, 1, 2, 4.85, {{0.269, 0.098}, {0.358, 0.153}}, 0, 0, 0, 7}},
-      {{8, 8, 1, 1, 7.26, {{0.608, 0.104}}, 8.71, 1.34},
-       {8, 4, 1, 1, 3.33, {{0.516, 0.102}}, 5.39, 1.89},
-       {4, 4, 1, 2, 4.87, {{0.352, 0.047}, {0.628, 0.091}}, 3.44, 1.65},
-       {4, 2, 1, 3, 3.36, {{0.349, 0.055}, {0.702, 0.000}, {1.128, 0.000}}, 3.53, 2.00},
-       {4, 4, 2, 1, 4.87, {{0.517, 0.141}}, 3.57, 2.17},
-       {4, 2, 2, 1, 3.44, {{0.519, 0.139}}, 4.01, 2.62},
-       {2, 1, 8, 1, 4.61, {{0.000, 0.671}}, 2.59, 0.00, 256},
-       {2, 2, 8, 1, 5.17, {{0.061, 0.452}}, 2.30, 0.00, 256},
-       {4, 1, 4, 1, 4.56, {{0.032, 1.080}}, 3.39, 0.00, 256},
-       {4, 2, 4, 1, 5.28, {{0.156, 0.302}}, 3.22, 0.64, 128},
-       {8, 3, 1, 2, 3.81, {{0.571, 0.154}, {0.722, 0.256}}, 0, 0, 0, 4},
-       {4, 3, 1, 2, 3.84, {{0.330, 0.105}, {0.395, 0.173}}, 0, 0, 0, 7}}};
   constexpr double kExactStep = 1.5;  // two products: 8 to 64 rows 1.35 to 1.45 x, 300 to 2000 rows 1.55 to 1.65
   const double cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
   const uint32_t rounds = (K + 127) / 128;
@@ -544,19 +556,14 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
     for (uint32_t splits : {1u, 2u, 3u, 4u, 6u, 8u}) {
       const uint32_t stages = c.k != 0 ? (K + c.k - 1) / c.k : 0;
       if (splits > 1 && (c.mi_most != 0 || rounds < 2 * splits * c.kw || (double)(tiles * splits) > 1.6 * c.per_cu * cus || (uint64_t)splits * M * N > (1u << 27))) break;
-      const double load = (double)(tiles * splits) / cus, full = std::floor(load / c.per_cu), rest = load - full * c.per_cu;
       const double steps = c.k != 0 ? (stages + splits - 1) / splits : 2.0 * ((((rounds + splits - 1) / splits) + c.kw - 1) / c.kw);
-      double t = steps * full * (c.step[c.per_cu - 1][0] + c.step[c.per_cu - 1][1] * frags);
-      if (rest > 1e-9) {
-        const double* s = c.step[(int)std::ceil(rest - 1e-9) - 1];
-        t += steps * (s[0] + s[1] * frags * (full > 0 || load >= 1 ? 1.0 : 0.5 + 0.5 * load));
-      }
+      double t = rounds_us(c, (double)(tiles * splits), frags, steps);
       t = c.start + (exact ? kExactStep : 1.0) * t;
       if (splits > 1) t += c.sum + c.sum_per_mi * splits * ((double)M * N / (1 << 20));
       if (t < best_us) { best_us = t; best = TilePlan{c.wn, mi, c.kw, splits, c.mi_most != 0}; }
     }
   };
-  for (const Cost& c : costs[bits == 8])
+  for (const Cost& c : kCosts[bits == 8])
     if (kind != PLAN_TWIN && c.mi_most == 0 && !(c.k != 0 && c.mi == 2 && M <= 32)) price(c, c.mi);
   *us = best_us;  // (the dispatch's lines were drawn for these: a shorter estimate must not send a call to a kernel that is longer still)
   if (exact) return best;
@@ -566,7 +573,7 @@ static TilePlan estimate_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits,
   const TilePlan other = best;
   const double other_us = best_us;
   best_us = 1e30;
-  for (const Cost& c : costs[bits == 8])
+  for (const Cost& c : kCosts[bits == 8])
     for (uint32_t mi = c.mi; mi <= c.mi_most; ++mi)
       if (M > 64 || c.wn == 8 || kind == PLAN_TWIN) price(c, mi);
   if (kind == PLAN_TWIN) return best;
@@ -592,6 +599,14 @@ TilePlan qmm_tile_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits, bool e
 TilePlan qmm_twin_plan(uint32_t M, uint32_t N, uint32_t K, uint32_t bits) {
   double us;
   return estimate_plan(M, N, K, bits, PLAN_TWIN, &us);
+}
+
+double qmm_tile_grouped_us(uint32_t bits, bool twin, uint32_t tile_rows, double row_tiles, double frags, uint32_t N, uint32_t K) {
+  const uint32_t wn = twin || tile_rows == 256 ? 8 : 4, mi = twin ? 3 : tile_rows / 32;
+  for (const Cost& c : kCosts[bits == 8])
+    if (c.wn == wn && c.mi == mi && c.kw == 1 && (c.mi_most != 0) == twin)
+      return c.start + rounds_us(c, row_tiles * ((N + wn * 32 - 1) / (wn * 32)), frags, 2.0 * ((K + 127) / 128));
+  return 1e30;
 }
 
 size_t qmm_tile_workspace_bytes(const TilePlan& plan, uint32_t M, uint32_t N) {
@@ -635,6 +650,8 @@ int32_t launch_qmm_tile(const QmmArgs& a, const TilePlan& plan, hipStream_t s) {
 int32_t launch_qmm_tile_grouped(const GroupedQmmArgs& a, uint32_t x_rows, hipStream_t s) {
   if (!qmm_tile_supported(a.N, a.K, a.group_size, a.bits) || (a.row_map != nullptr && !qmm_tile_maps_rows(x_rows, a.K)))
     return fail(RMLX_INVALID_SHAPE, "grouped qmm: unsupported shape N=%u K=%u bits=%u group_size=%u, %u rows", a.N, a.K, a.bits, a.group_size, x_rows);
+  if (a.twin && (a.exact || a.tile_rows > (a.bits == 4 ? 160u : 128u)))
+    return fail(RMLX_RUNTIME_ERROR, "grouped qmm: two workgroups per CU take rounded weights and row tiles of up to 160 rows (8-bit: 128), got %u", a.tile_rows);
   if (a.max_tiles == 0) return RMLX_OK;
   if (a.tile_rows == 32) return launch_qmm_slice_grouped(a, x_rows, s);
   TileParams p{};

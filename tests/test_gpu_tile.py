@@ -215,6 +215,15 @@ def test_routed_block_on_two_workgroups_per_cu(hip, tokens, experts, hidden, int
     assert_close(out, model.moe_forward(x, idx, w, gate, up, down, gs, 1, bits=bits), f"E={experts} D={hidden} I={inter} T={tokens} bits={bits} gs={gs}")
 
 
+# By the prices on 256 CUs: on two workgroups per CU, 4-bit at 130 rows an expert (group sizes 32 and 64) and 300 (128), 8-bit at 300 (32) and 90 (64), dimensions in
+# multiples of 64, which round their weights; on the other tiles, 70 rows, 170 rows, 8-bit 110 rows.
+@pytest.mark.parametrize("tokens,experts,hidden,inter,bits,gs,fused", [(4160, 32, 1088, 576, 4, 32, False), (4160, 32, 1088, 576, 4, 64, True), (7200, 24, 1152, 640, 4, 128, True),
+                                                                      (7200, 24, 1088, 1152, 8, 32, False), (3600, 40, 1088, 576, 8, 64, False),
+                                                                      (2240, 32, 1088, 1152, 4, 64, True), (5440, 32, 1088, 576, 4, 64, False), (4400, 40, 1088, 576, 8, 64, True)])
+def test_routed_block_by_its_prices(hip, tokens, experts, hidden, inter, bits, gs, fused):
+    test_routed_block_on_two_workgroups_per_cu(hip, tokens, experts, hidden, inter, bits, gs, fused)
+
+
 @pytest.mark.parametrize("tokens,experts,top_k,hidden,inter", [(262200, 8, 8, 512, 512), (131100, 2, 1, 8192, 512)])
 def test_routed_block_over_more_than_two_gib(hip, tokens, experts, top_k, hidden, inter):
     """Hidden activations, and activations reached through the token map, of more than 2 GiB; the last tokens, which lie beyond it."""
