@@ -319,7 +319,7 @@ int32_t rmlx_hip_moe_forward_grouped(const rmlx_qweight* gate, const rmlx_qweigh
 
 /* Kernel choice of the expert projections (ExpertGroup and the MoeLayer entry points): batches with at least
  * `min_rows` rows per expert on average (rows / num_experts; for ExpertGroup rows / n_items) multiply with a
- * grouped MFMA GEMM -- the tile GEMM (32, 64, 128 or 256 rows of one expert, every 4- / 8-bit shape) where it is ahead
+ * grouped MFMA GEMM -- the tile GEMM (32, 64, 128, 160 or 256 rows of one expert, every 4- / 8-bit shape) where it is ahead
  * (with the default threshold also below it, then with exact weights: kernel 13 of rmlx_hip_qmm_select), else row tiles of 16 or 32 rows of one expert, weights dequantised in registers; 4- / 8-bit,
  * group sizes 32 / 64 / 128 (one for the three projections), hidden and intermediate dimensions in multiples of
  * 512 -- smaller ones with the streaming GEMV, which reads an expert's weights once per 8 rows (8-bit experts

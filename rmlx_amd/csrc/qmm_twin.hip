@@ -10,10 +10,11 @@
 // in chunks of an activation fragment: its NI products, its next read, its share of the unpacking and, behind the barrier, one load.
 // Rows past the tile are loaded as zeros (products with zeros cost less power than with repeats; no traffic), k past the row as well.
 //
-// What bounds it: power and vector issue, as qmm_tile.hip (matrix unit 0.66 busy at 1.56 GHz over 128 experts of 128 rows), but not the ends
-// of a tile: those take 7 to 9 us of every tile of a lone workgroup per CU (2560 rows, 16384 x 1536: eight-wave tiles 140 us, here 121; x 4096 322 / 302;
-// 4096 rows, 16384 x 1536 203 / 193).  With a workgroup of eight waves that splits k in two instead (same LDS reads): 130 us, its sums meet
-// in LDS behind the loop.  Routed block, 2048 tokens, top-8 of 128 experts of 1536 x 4096: 873 -> 786 us (gate / up 521 -> 472, down 317 -> 285 under the profiler).
+// What bounds it: power and vector issue, as qmm_tile.hip (128 experts of 128 rows: matrix unit 0.65 of the cycles busy in gate / up, 0.51 in down, five vector
+// instructions a product, at 1.45 to 1.6 GHz), but not the ends of a tile: those take 7 to 9 us of every tile of a lone workgroup per CU (2560 rows, 16384 x 1536:
+// eight-wave tiles 145 us, here 119; 1551 rows, 11328 x 4544 185 / 155).  With a workgroup of eight waves that splits k in two instead (same LDS reads): 130 us, its sums meet
+// in LDS behind the loop.  Routed block, 2048 tokens, top-8 of 128 experts of 1536 x 4096: 872 -> 777 us, in turn on one card
+// (the card's power moves both by 5 % from one to another).
 // NI = 1 (up to seven fragments) fills the chip with half the columns: 300 rows, 16384 x 4096 58.7 (256 columns) / 56.5 (128 columns, three stages) / 49.2.
 #include <type_traits>
 
